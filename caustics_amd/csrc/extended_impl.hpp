@@ -356,24 +356,6 @@ __device__ void chain_images(cd* zb, uint32_t* fb, uint64_t* perm, int M) {
     __syncthreads();
 }
 
-// block-wide exclusive prefix sum of per-thread counts (NT threads)
-template <int NT>
-__device__ inline int block_exclusive_scan(int v, int* sh, int& total) {
-    const int tid = threadIdx.x;
-    sh[tid] = v;
-    __syncthreads();
-    for (int off = 1; off < NT; off <<= 1) {
-        const int t = (tid >= off) ? sh[tid - off] : 0;
-        __syncthreads();
-        sh[tid] += t;
-        __syncthreads();
-    }
-    total = sh[NT - 1];
-    const int r = sh[tid] - v;
-    __syncthreads();
-    return r;
-}
-
 __device__ inline double block_sum(double v, double* sh) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     v = wave_sum(v);
@@ -1373,90 +1355,168 @@ __global__ __launch_bounds__(kExtWaveBlock) void k_ext_chain(ExtArgs A, int cur,
 }
 
 // ---- one refinement round, part 1 (extended_source.py:108-135): the n_add largest
-// image gaps (bitonic sort of the gap keys in LDS, descending by (gap, position)),
-// insertion shifts, the next limb order and the carried-over gap keys, one task per new
-// point.  Points stay where they are (append order); only the order and keys move.
-// NT threads per source: one wave for short contours, four when the sort is long.
-template <int NL, int NT>
+// image gaps (descending by (gap, position)), insertion shifts, the next limb order and the
+// carried-over gap keys, one task per new point.  Points stay where they are (append
+// order); only the order and keys move.
+//
+// Only the set of the n_add largest keys matters (the append order of the new points is
+// never seen again: everything later goes through the limb order), so the keys are not
+// sorted.  Each thread holds its PER keys (limb position tid + i NT) in registers and the
+// threshold is found by bisection on the key's bit pattern, one ballot and popcount per
+// register and step; some 15-20 steps isolate the n_add-th key, and equal keys are taken
+// from the last position on, as a descending sort by (key, position) takes them.  The
+// shifts come from the same ballots.
+// NT threads per source: one wave for short contours, four above kExtSelWave points.
+// Bound: latency of the bisection's dependent steps.  A bitonic sort of all keys in LDS
+// took 15.5 us at 150 limb points (one source) and 361 us for 4,096 binary sources of
+// 256-4096 points.
+constexpr int kExtSelWave = 512;
+template <int NL, int NT, int PER>
 __global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round) {
     constexpr int DEG = ext_degree<NL>();
-    extern __shared__ uint64_t s_dyn[];
-    __shared__ int s_int[NT];
-    const int tid = threadIdx.x;
+    constexpr int NW = NT / 64;
+    __shared__ int s_cnt[2][NW];       // bisection counts, double buffered (one barrier a step)
+    __shared__ uint64_t s_max[NW];
+    __shared__ int s_sel[PER * NW];    // selected / tied keys per (register, wave)
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t src = blockIdx.x;
     const ExtBatch B = ext_batch(A);
     const int n = B.npts[src];
     if (n == 0) return;   // skipped source
-    const int M = ext_points(n, round), nadd = ext_n_add(n);
+    const int M = ext_points(n, round), nadd = ext_n_add(n);   // M <= PER * NT
     ExtWS W = ext_ws(ext_source_base<DEG>(A, src), DEG, A.mmax);
     const int nxt = cur ^ 1;
     const int32_t* ord = W.ord[cur];
     const uint64_t* gk = W.gk[cur];
-    int P2 = 1;
-    while (P2 < M - 1) P2 <<= 1;
-    uint64_t* s_key = s_dyn;
-    int* s_idx = reinterpret_cast<int*>(s_dyn + P2);
-    for (int k = tid; k < P2; k += NT) {
-        s_key[k] = (k < M - 1) ? gk[k] : 0ull;
-        s_idx[k] = (k < M - 1) ? k : -1;
+    uint64_t key[PER];
+    uint64_t mx = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int k = tid + i * NT;
+        key[i] = k < M - 1 ? gk[k] : 0ull;
+        mx = key[i] > mx ? key[i] : mx;
     }
-    __syncthreads();
-    for (int size = 2; size <= P2; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = tid; i < P2; i += NT) {
-                const int j = i ^ stride;
-                if (j > i) {
-                    const bool desc = (i & size) == 0;
-                    const uint64_t ki = s_key[i], kj = s_key[j];
-                    const int ii = s_idx[i], ij = s_idx[j];
-                    const bool i_less = (ki < kj) || (ki == kj && ii < ij);
-                    if (desc == i_less) {
-                        s_key[i] = kj;
-                        s_key[j] = ki;
-                        s_idx[i] = ij;
-                        s_idx[j] = ii;
-                    }
-                }
-            }
+    int par = 0;
+    // number of keys >= t (t >= 1, so the padding's zero keys never count)
+    auto count = [&](uint64_t t) -> int {
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) c += __popcll(__ballot(key[i] >= t));
+        if constexpr (NW > 1) {
+            if (lane == 0) s_cnt[par][wv] = c;
             __syncthreads();
+            c = 0;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) c += s_cnt[par][q];
+            par ^= 1;
+        }
+        return c;
+    };
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const uint64_t o = __shfl_xor(mx, off, 64);
+        mx = o > mx ? o : mx;
+    }
+    if constexpr (NW > 1) {
+        if (lane == 0) s_max[wv] = mx;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NW; ++q) mx = s_max[q] > mx ? s_max[q] : mx;
+    }
+    // count(>= lo) >= nadd > count(>= hi) = chi; keys are non-negative doubles' bits
+    uint64_t lo = 0, hi = mx + 1;
+    int chi = 0;
+    bool exact = false;
+    if (nadd == 0) {
+        lo = hi;       // nothing is selected
+        exact = true;
+    }
+    const uint64_t low = 24ull << 52;   // a first step 24 binades below the largest gap
+    bool probe = mx > low;
+    while (!exact && hi - lo > 1) {
+        const uint64_t mid = probe ? mx - low : lo + ((hi - lo) >> 1);
+        probe = false;
+        const int c = count(mid);
+        if (c == nadd) exact = true;
+        if (c >= nadd) {
+            lo = mid;
+        } else {
+            hi = mid;
+            chi = c;
         }
     }
-    // selected gaps -> exclusive prefix count = shift of every point
-    int* shift = reinterpret_cast<int*>(W.perm);
-    const int per = (M + NT - 1) / NT;
-    const int k0 = tid * per, k1 = min(M, k0 + per);
-    for (int k = k0; k < k1; ++k) shift[k] = 0;
-    __syncthreads();
-    for (int c = tid; c < nadd; c += NT) shift[s_idx[c]] = 1;
-    __syncthreads();
-    int cnt = 0;
-    for (int k = k0; k < k1; ++k) cnt += shift[k];
-    int total;
-    int run = block_exclusive_scan<NT>(cnt, s_int, total);
-    for (int k = k0; k < k1; ++k) {
-        const int ins = shift[k];
-        shift[k] = run | (ins << 30);   // bit 30: the gap after point k is refined
-        run += ins;
+    // keys >= lo are selected when that is exactly nadd of them; otherwise the chi keys
+    // above lo and the last nadd - chi of the keys equal to lo
+    unsigned sel = 0;   // bit i: the gap after point tid + i NT is refined
+    if (exact) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (key[i] >= lo && tid + i * NT < M - 1) sel |= 1u << i;
+    } else {
+        int tot = 0;    // all keys equal to lo
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const uint64_t m = __ballot(key[i] == lo && tid + i * NT < M - 1);
+            if (lane == 0) s_sel[i * NW + wv] = __popcll(m);
+        }
+        __syncthreads();
+        for (int q = 0; q < PER * NW; ++q) tot += s_sel[q];
+        int before = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const bool tie = key[i] == lo && tid + i * NT < M - 1;
+            const uint64_t m = __ballot(tie);
+            int b = before;
+            for (int q = 0; q < NW; ++q) {
+                if (q < wv) b += s_sel[i * NW + q];
+                before += s_sel[i * NW + q];
+            }
+            const int rank = b + __popcll(m & ((1ull << lane) - 1ull));   // ties before this one
+            if (key[i] > lo || (tie && tot - rank <= nadd - chi)) sel |= 1u << i;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (int k = tid; k < M; k += NT) {
-        const int sh = shift[k];
-        const int d = k + (sh & 0x3FFFFFFF);
-        W.ord[nxt][d] = ord[k];
-        if (k + 1 < M && !(sh >> 30)) W.gk[nxt][d] = gk[k];
+    // insertion shift of every point = selected gaps before it
+    uint64_t bal[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        bal[i] = __ballot((sel >> i) & 1u);
+        if (NW > 1 && lane == 0) s_sel[i * NW + wv] = __popcll(bal[i]);
     }
+    if constexpr (NW > 1) __syncthreads();
     const int64_t t0 = B.off_add[src];
-    for (int c = tid; c < nadd; c += NT) {
-        const int k = s_idx[c];
-        const int d = k + (shift[k] & 0x3FFFFFFF) + 1;
-        const int a = ord[k], b = ord[k + 1];
-        B.t_src[t0 + c] = (int32_t)src;
-        B.t_left[t0 + c] = a;
-        B.t_right[t0 + c] = b;
-        B.t_dst[t0 + c] = d;
-        B.t_app[t0 + c] = M + c;
-        B.t_th[t0 + c] = 0.5 * (W.theta[0][a] + W.theta[0][b]);
-        W.ord[nxt][d] = M + c;
+    int run = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (i * NT >= M) break;
+        int b = run;
+        if constexpr (NW > 1) {
+            for (int q = 0; q < NW; ++q) {
+                if (q < wv) b += s_sel[i * NW + q];
+                run += s_sel[i * NW + q];
+            }
+        } else {
+            run += __popcll(bal[i]);
+        }
+        const int k = tid + i * NT;
+        if (k >= M) continue;
+        const int c = b + __popcll(bal[i] & ((1ull << lane) - 1ull));
+        const int d = k + c;
+        const int a = ord[k];
+        W.ord[nxt][d] = a;
+        if ((sel >> i) & 1u) {
+            const int e = ord[k + 1];
+            const int64_t t = t0 + c;
+            B.t_src[t] = (int32_t)src;
+            B.t_left[t] = a;
+            B.t_right[t] = e;
+            B.t_dst[t] = d + 1;
+            B.t_app[t] = M + c;
+            B.t_th[t] = 0.5 * (W.theta[0][a] + W.theta[0][e]);
+            W.ord[nxt][d + 1] = M + c;
+        } else if (k + 1 < M) {
+            W.gk[nxt][d] = key[i];
+        }
     }
 }
 
@@ -1954,19 +2014,18 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
     hipLaunchKernelGGL((k_ext_limb_init<NL, MODE>), dim3(ext_flat_grid(lanes_init)),
                        dim3(kExtFlatBlock), 0, s, a);
     hipLaunchKernelGGL((k_ext_chain<NL>), dim3(nb), dim3(kExtWaveBlock), 0, s, a, 0, 0);  // initial
-    int P2 = 1;
-    while (P2 < a.mmax) P2 <<= 1;
-    const size_t lds = (size_t)P2 * (sizeof(uint64_t) + sizeof(int));
     const int add_grid = ext_flat_grid(S * (int64_t)(a.nadd_max > 0 ? a.nadd_max : 1));
     int cur = 0;
-    const bool wide = P2 > 512;   // long contours: four waves share each sort
+    static_assert(kExtSelWave % 64 == 0 && kExtSortMax % kExtBlock == 0, "select register tiles");
     for (int round = 0; round < 10; ++round) {
-        if (wide)
-            hipLaunchKernelGGL((k_ext_select<NL, kExtBlock>), dim3(nb), dim3(kExtBlock), lds, s, a,
-                               cur, round);
+        // one wave while its 8 registers of keys hold the contour (no barrier in the
+        // bisection); four waves of 16 above
+        if (a.mmax <= kExtSelWave)
+            hipLaunchKernelGGL((k_ext_select<NL, kExtWaveBlock, kExtSelWave / 64>), dim3(nb),
+                               dim3(kExtWaveBlock), 0, s, a, cur, round);
         else
-            hipLaunchKernelGGL((k_ext_select<NL, kExtWaveBlock>), dim3(nb), dim3(kExtWaveBlock),
-                               lds, s, a, cur, round);
+            hipLaunchKernelGGL((k_ext_select<NL, kExtBlock, kExtSortMax / kExtBlock>), dim3(nb),
+                               dim3(kExtBlock), 0, s, a, cur, round);
         hipLaunchKernelGGL((k_ext_solve_add<NL, MODE>), dim3(add_grid), dim3(kExtFlatBlock), 0, s,
                            a, cur);
         cur ^= 1;

@@ -74,6 +74,18 @@ def test_binary_uniform_near_caustics(gpu, rho):
     compare(m, mo, f"binary uniform rho={rho}")
 
 
+@pytest.mark.parametrize("npts", [19, 20, 519, 520, 4096])
+def test_gap_selection_edges(gpu, npts):
+    """No refined gap (19), one per round (20), the longest contour of the one-wave gap
+    selection and the shortest of the four-wave one (519, 520), the largest contour; the
+    source on the lens axis has gaps equal up to rounding."""
+    w = np.concatenate([caustic_points(1e-2, npts=1, s=0.9, q=0.2), [0.3 + 0.0j]])
+    kw = dict(nlenses=2, npts_limb=npts, s=0.9, q=0.2)
+    m = mag_extended_source(w, 1e-2, **kw).cpu().numpy()
+    mo = np.array([E.mag_extended_source(x, 1e-2, **kw) for x in w])
+    compare(m, mo, f"binary uniform npts_limb={npts}")
+
+
 def test_binary_ld_near_caustics(gpu):
     rho = 1e-2
     w = caustic_points(rho, npts=6, s=0.9, q=0.2)
