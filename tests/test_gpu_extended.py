@@ -422,3 +422,24 @@ def test_workspace_contents_do_not_change_results(gpu, nlenses):
     for a, b in zip(*out):
         assert torch.equal(a, b)
     assert out[0][0][1].item() == 0 and bool(torch.isfinite(out[0][0]).all())
+
+
+@pytest.mark.parametrize("nlenses", [1, 2, 3])
+@pytest.mark.parametrize("npts_ld,u1", [(2, 0.5), (3, 1.0), (101, 0.0), (256, 0.7)])
+def test_line_integral_rule_sizes(gpu, nlenses, npts_ld, u1):
+    """Smallest, odd and largest Gauss-Legendre rules of the P and Q lines, profiles from
+    uniform (u1 = 0) to fully darkened: the oracle's value, the forward and the forward+VJP
+    kernel's bits alike, finite gradients."""
+    from caustics_amd.extended_source import extended_fwd_vjp
+
+    prm = {1: {}, 2: dict(s=0.9, q=0.2), 3: dict(s=0.9, q=0.2, q3=0.01, r3=0.7, psi=0.4)}[nlenses]
+    rho = 2e-2
+    w = (np.array([0.1 + 0.05j, rho + 1e-12, 0.3j]) if nlenses == 1 else
+         caustic_points(rho, npts=3, s=0.9, q=0.2)[:3])
+    kw = dict(nlenses=nlenses, npts_limb=100, limb_darkening=True, npts_ld=npts_ld)
+    m = mag_extended_source(w, rho, u1=u1, **kw, **prm).cpu().numpy()
+    mv, g, _ = extended_fwd_vjp(w, rho, np.ones(len(w)), u1=u1, **kw, **prm)
+    assert np.array_equal(m, mv.cpu().numpy())
+    assert torch.isfinite(g).all()
+    mo = np.array([E.mag_extended_source(x, rho, u1=u1, **kw, **prm) for x in w])
+    compare(m, mo, f"rule n={npts_ld} u1={u1} nlenses={nlenses}")
