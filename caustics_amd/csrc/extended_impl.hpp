@@ -266,24 +266,13 @@ __device__ inline cd contour_point(ZRows zb, const Piece* pc, int np, int k) {
 
 namespace caus {
 
-// Gauss-Legendre nodes/weights on [-1,1] by Newton iteration on P_n (ascending x)
-__device__ inline void gauss_legendre(int n, double2* xw) {
-    for (int i = threadIdx.x; i < n; i += kExtBlock) {
-        // root i counted from x = +1 downwards, stored ascending
-        double z = cos(3.14159265358979323846 * (i + 0.75) / (n + 0.5));
-        double pp = 1.0;
-        for (int it = 0; it < 100; ++it) {
-            double p1 = 1.0, p2 = 0.0;
-            for (int j = 1; j <= n; ++j) {
-                const double p3 = p2;
-                p2 = p1;
-                p1 = ((2.0 * j - 1.0) * z * p2 - (j - 1.0) * p3) / j;
-            }
-            pp = n * (z * p1 - p2) / (z * z - 1.0);
-            const double dz = p1 / pp;
-            z -= dz;
-            if (fabs(dz) < 1e-16) break;
-        }
+// Node i of the n-point Gauss-Legendre rule on [-1,1] by Newton iteration on P_n; xw holds
+// (node, weight) in ascending order
+__device__ inline void gauss_legendre(int n, int i, double2* xw) {
+    // root i counted from x = +1 downwards, stored ascending
+    double z = cos(3.14159265358979323846 * (i + 0.75) / (n + 0.5));
+    double pp = 1.0;
+    for (int it = 0; it < 100; ++it) {
         double p1 = 1.0, p2 = 0.0;
         for (int j = 1; j <= n; ++j) {
             const double p3 = p2;
@@ -291,8 +280,18 @@ __device__ inline void gauss_legendre(int n, double2* xw) {
             p1 = ((2.0 * j - 1.0) * z * p2 - (j - 1.0) * p3) / j;
         }
         pp = n * (z * p1 - p2) / (z * z - 1.0);
-        xw[n - 1 - i] = make_double2(z, 2.0 / ((1.0 - z * z) * pp * pp));
+        const double dz = p1 / pp;
+        z -= dz;
+        if (fabs(dz) < 1e-16) break;
     }
+    double p1 = 1.0, p2 = 0.0;
+    for (int j = 1; j <= n; ++j) {
+        const double p3 = p2;
+        p2 = p1;
+        p1 = ((2.0 * j - 1.0) * z * p2 - (j - 1.0) * p3) / j;
+    }
+    pp = n * (z * p1 - p2) / (z * z - 1.0);
+    xw[n - 1 - i] = make_double2(z, 2.0 / ((1.0 - z * z) * pp * pp));
 }
 
 // s = sqrt(x) and h ~ 1/(2 sqrt x) for x > 0 in the normal range (x >= 2^-767): the
@@ -323,7 +322,7 @@ struct LDSource {
     double e[NL];
     cd r[NL];
     cd w0;
-    double rho, irho, rho2, irho2, u1, c3;
+    double rho, rho2x, irho, irho2, u1, c3;   // rho2x = 2 rho
 };
 template <int NL>
 __device__ __forceinline__ LDSource<NL> ld_source(const LensFrame<NL>& lf, cd w0, double rho,
@@ -337,7 +336,7 @@ __device__ __forceinline__ LDSource<NL> ld_source(const LensFrame<NL>& lf, cd w0
     q.w0 = cd{uniform(w0.re), uniform(w0.im)};
     q.rho = uniform(rho);
     q.irho = uniform(rcp(rho));
-    q.rho2 = uniform(rho * rho);
+    q.rho2x = uniform(2.0 * rho);
     q.irho2 = uniform(q.irho * q.irho);
     q.u1 = uniform(u1);
     q.c3 = uniform(3.0 / (3.0 - u1));
@@ -347,11 +346,12 @@ __device__ __forceinline__ LDSource<NL> ld_source(const LensFrame<NL>& lf, cd w0
 // One node of a line integral at z (integrate.py:29-44): r = |lens_eq(z) - w0| / rho,
 // B = c3 (u1 B_r + 1 - 2 u1), c3 = 3/(3-u1), B_r = 1 + t with t = sqrt(1 - r^2) inside the
 // disk (r <= 1) and t = -sqrt(1 - 1/r^2) outside.  Returned: v_j = 1/(conj z - conj r_j),
-// D = lens_eq(z) - w0, n2 = |D|^2, t and p, with dB_r/dD = -2 rho^2 p D.
-// No square root of |D|^2 is needed: with m = min(1/rho^2, 1/|D|^2) both sides have
-//   |t|^2 = |rho^2 - |D|^2| m,   -(dB_r/d|D|) / |D| = rho^2 m^2 / |t|   (rho^2 m = 1 inside),
-// and rho^2 - |D|^2 is exact near the limb, where |t| is sensitive.  Contraction is off so
-// that the forward-only and the forward+VJP kernels round alike.
+// D = lens_eq(z) - w0, n2 = |D|^2, t and p, with dB_r/dD = -(2/rho^2) p D.
+// q = min(r, 1/r) serves both sides, |t| = sqrt(1 - q^2), and the derivative
+//   -(dB_r/d|D|) / |D| = min(1, 1/r^2)^2 / (rho^2 |t|)
+// needs no division by |D|.  Near the limb t keeps only the rounding of r and 1/r, so these
+// are one multiplication each.  Contraction is off so that the forward-only and the
+// forward+VJP kernels round alike.
 template <int NL>
 __device__ __forceinline__ void ld_node(cd z, const LDSource<NL>& q, cd (&v)[NL], cd& D,
                                         double& n2, double& t, double& p) {
@@ -386,14 +386,17 @@ __device__ __forceinline__ void ld_node(cd z, const LDSource<NL>& q, cd (&v)[NL]
     for (int j = 1; j < NL; ++j) G = cd{fma(q.e[j], v[j].re, G.re), fma(q.e[j], v[j].im, G.im)};
     D = z - G - q.w0;
     n2 = norm2(D);
-    const double diff = q.rho2 - n2;
-    const double m = fmin(q.irho2, rcp(n2));   // n2 = 0: the reciprocal is NaN, m = 1/rho^2
-    const double x = fabs(diff) * m;
+    double aD, hD;
+    sqrt_half_rsq(fmax(n2, 0x1p-700), aD, hD);
+    const double r = aD * q.irho, ir = q.rho2x * hD;
+    const double k = fmin(r, ir);
+    const double x = 1.0 - k * k;
     double s, h;
     sqrt_half_rsq(fmax(x, 0x1p-200), s, h);
     h = x > 0.0 ? h : 0.0;
-    t = copysign(s, diff);
-    p = (h * m) * m;
+    t = copysign(s, 1.0 - r);
+    const double m = fmin(ir, 1.0), m2 = m * m;
+    p = (h * m2) * m2;
 }
 
 // one trapezoid term of the limb-darkened contour integral (integrate.py:118-121),
@@ -478,12 +481,6 @@ __device__ inline cd seg_point(ZRows zb, const Seg& s, int k) {
     if (s.empty || k < 0 || k >= s.len) return cd{0.0, 0.0};
     return pt<DEG>(zb, s.start + k, s.row);
 }
-template <int DEG>
-__device__ inline cd act_point(ZRows zb, const ActSeg& a, int k) {
-    if (a.empty || k < 0 || k > a.t) return cd{0.0, 0.0};
-    return contour_point<DEG>(zb, a.pc, a.np, k);
-}
-
 // line ending at the head / tail (second element is the connection point).
 // Dense-array semantics: points beyond the segment are zero, dynamic_slice clamps.
 template <class F>
@@ -642,10 +639,10 @@ struct LDAdj {
 // the derivatives along and across the line at weight w_i are Im / Re (u + conj(u) K)
 // = components of sum u + sum_j e_j conj(sum conj(u) v_j^2).  The node loop therefore holds
 // only these sums; the profile's constants and the line's scale are applied once a part.
-// Bound: FP64 issue.  Per node of two lenses 77 FP64 operations and 3 quarter-rate seeds;
-// with the profile, its radius and every derivative formed node by node it was 124 and 3.
-// Integration of 4,096 binary sources of 256-4096 limb points (3.2e9 nodes): 17.0 -> 10.9 ms,
-// of 12,000 triple-lens sources (2.0e9 nodes): 17.8 -> 11.7 ms.
+// Bound: FP64 issue.  Per node of two lenses 87 FP64 operations and 3 quarter-rate seeds;
+// with every derivative formed node by node it was 124 and 3.  Integration of 4,096 binary
+// sources of 256-4096 limb points (3.2e9 nodes): 17.0 -> 11.8 ms, of 12,000 triple-lens
+// sources (2.0e9 nodes): 17.8 -> 10.8 ms (of which 0.5 ms the Gauss-Legendre nodes).
 template <int NL, bool ISP>
 __device__ __forceinline__ double ld_line_adj(double fixed, double a, double b,
                                               const LDSource<NL>& q, const GLNodes& g, double wA,
@@ -665,7 +662,7 @@ __device__ __forceinline__ double ld_line_adj(double fixed, double a, double b,
         dsp_db = 1.0;
         dsp_drho = (b > a) ? -2.0 : 2.0;
     }
-    const double kap = -2.0 * q.c3 * q.u1 * q.rho2;   // dB/dD = kap p D
+    const double kap = -2.0 * q.c3 * q.u1 * q.irho2;   // dB/dD = kap p D
     // B = c3 (u1 (1 + t) + 1 - 2 u1), c3' = c3^2/3: dB/du1 = bu0 + bu1 t
     const double dc3 = q.c3 * q.c3 / 3.0;
     const double bu0 = dc3 * (1.0 - q.u1) - q.c3, bu1 = dc3 * q.u1 + q.c3;
@@ -950,8 +947,10 @@ __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* 
 // Batch pipeline.  The contours of a batch of sources are computed by a fixed
 // sequence of launches over the whole batch, so that the root solves (nearly all of
 // the arithmetic) run one limb point per lane at the solver's occupancy:
-//   k_ext_plan        1 block      effective npts, prefix offsets of the flat work lists
-//   k_ext_limb_init   flat         initial limb angles, kExtPer consecutive angles per lane
+//   k_ext_limb_init   1-2 + flat   effective npts, prefix offsets of the flat work lists;
+//                                  Gauss-Legendre nodes; limb point 0 of every source
+//   k_ext_limb_init   flat         the other initial limb angles, kExtPer consecutive ones
+//                                  per lane
 //   k_ext_chain       per source   image continuation (extended_source.py:34-53), limb
 //                                  order and gap keys of the initial points
 //   10 x k_ext_select per source   gap-key sort, insertion shifts, next limb order, tasks
@@ -973,7 +972,6 @@ namespace caus {
 
 constexpr int kExtPer = 4;          // initial limb angles per lane of k_ext_limb_init
 constexpr int kExtFlatBlock = 256;  // block of the flat kernels
-constexpr int kExtPlanBlock = 1024;
 
 struct ExtArgs {
     const cd* w0;
@@ -1019,7 +1017,9 @@ struct ExtBatch {
     int32_t* t_dst;     // its limb angle
     int32_t* t_app;
     double* t_th;
+    double2* gl;        // 2 x 128 Gauss-Legendre nodes and weights (limb darkening)
 };
+constexpr int kExtGL = 128;   // most nodes of one part of a line (npts_ld <= 256)
 
 __host__ __device__ inline size_t ext_task_cap(int64_t S, int nadd_max) {
     return (size_t)S * (size_t)(nadd_max > 0 ? nadd_max : 1);
@@ -1029,7 +1029,7 @@ __host__ __device__ inline size_t ext_header_bytes(int64_t S, int nadd_max) {
     const size_t cap = ext_task_cap(S, nadd_max);
     return ext_align(2 * (size_t)(S + 1) * sizeof(int64_t)) + ext_align((size_t)S * 4) +
            ext_align((size_t)S) + ext_align(5 * cap * sizeof(int32_t)) +
-           ext_align(cap * sizeof(double));
+           ext_align(cap * sizeof(double)) + 2 * kExtGL * sizeof(double2);
 }
 
 __host__ __device__ inline size_t ext_source_bytes(int deg, int mmax) {
@@ -1059,6 +1059,8 @@ __device__ inline ExtBatch ext_batch(const ExtArgs& A) {
     b.t_app = b.t_dst + cap;
     p += ext_align(5 * cap * sizeof(int32_t));
     b.t_th = (double*)p;
+    p += ext_align(cap * sizeof(double));
+    b.gl = (double2*)p;
     return b;
 }
 
@@ -1100,99 +1102,150 @@ __device__ inline int ext_points(int npts, int round) {
 
 constexpr double kExtPi = 3.14159265358979323846;
 
-// ---- plan: effective npts (out-of-range values clamped and flagged) and the prefix
-// offsets of the flat work lists, one block scanning the batch in chunks
-static __global__ __launch_bounds__(kExtPlanBlock) void k_ext_plan(ExtArgs A) {
-    __shared__ int64_t s_a[kExtPlanBlock], s_b[kExtPlanBlock];
-    const ExtBatch B = ext_batch(A);
-    const int tid = threadIdx.x;
-    int64_t carry_a = 0, carry_b = 0;
-    for (int64_t base = 0; base < A.S; base += kExtPlanBlock) {
-        const int64_t s = base + tid;
-        int64_t ca = 0, cb = 0;
-        if (s < A.S) {
-            int n = A.npts ? A.npts[s] : A.npts_def;
-            bool bad = false;
-            if (n != 0 && (n < 4 || n > A.npts_def)) {
-                bad = true;
-                n = n < 4 ? 4 : A.npts_def;
-            }
-            B.npts[s] = n;   // 0: the source is skipped (no limb points, no work)
-            B.fail[s] = bad ? 1 : 0;
-            ca = (ext_npts_init(n) + kExtPer - 1) / kExtPer;
-            cb = ext_n_add(n);
-        }
-        s_a[tid] = ca;
-        s_b[tid] = cb;
-        __syncthreads();
-        for (int off = 1; off < kExtPlanBlock; off <<= 1) {
-            const int64_t ta = tid >= off ? s_a[tid - off] : 0;
-            const int64_t tb = tid >= off ? s_b[tid - off] : 0;
-            __syncthreads();
-            s_a[tid] += ta;
-            s_b[tid] += tb;
-            __syncthreads();
-        }
-        if (s < A.S) {
-            B.off_init[s] = carry_a + s_a[tid] - ca;
-            B.off_add[s] = carry_b + s_b[tid] - cb;
-        }
-        carry_a += s_a[kExtPlanBlock - 1];
-        carry_b += s_b[kExtPlanBlock - 1];
-        __syncthreads();
+// effective limb resolution of source s: 0 (skipped) or 4..npts_def, out-of-range values
+// clamped and flagged
+__device__ __forceinline__ int ext_npts(const ExtArgs& A, int64_t s, bool& bad) {
+    const int n = A.npts ? A.npts[s] : A.npts_def;
+    bad = n != 0 && (n < 4 || n > A.npts_def);
+    return bad ? (n < 4 ? 4 : A.npts_def) : n;
+}
+
+// effective npts and the prefix offsets of the flat work lists: one workgroup, each thread
+// a run of consecutive sources
+__device__ inline void ext_plan(const ExtArgs& A, const ExtBatch& B) {
+    constexpr int NT = kExtFlatBlock;
+    __shared__ int64_t s_a[NT / 64], s_b[NT / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int64_t run = (A.S + NT - 1) / NT;
+    const int64_t s0 = min(A.S, tid * run), s1 = min(A.S, s0 + run);
+    int64_t ca = 0, cb = 0;
+    for (int64_t s = s0; s < s1; ++s) {
+        bool bad;
+        const int n = ext_npts(A, s, bad);
+        B.npts[s] = n;   // 0: the source is skipped (no limb points, no work)
+        ca += (ext_npts_init(n) + kExtPer - 1) / kExtPer;
+        cb += ext_n_add(n);
     }
-    if (tid == 0) {
-        B.off_init[A.S] = carry_a;
-        B.off_add[A.S] = carry_b;
+    int64_t ia = ca, ib = cb;   // inclusive sums over the threads
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int64_t ta = __shfl_up(ia, off, 64), tb = __shfl_up(ib, off, 64);
+        if (lane >= off) {
+            ia += ta;
+            ib += tb;
+        }
+    }
+    if (lane == 63) {
+        s_a[wv] = ia;
+        s_b[wv] = ib;
+    }
+    __syncthreads();
+    for (int q = 0; q < wv; ++q) {
+        ia += s_a[q];
+        ib += s_b[q];
+    }
+    int64_t oa = ia - ca, ob = ib - cb;
+    for (int64_t s = s0; s < s1; ++s) {
+        const int n = B.npts[s];
+        B.off_init[s] = oa;
+        B.off_add[s] = ob;
+        oa += (ext_npts_init(n) + kExtPer - 1) / kExtPer;
+        ob += ext_n_add(n);
+    }
+    if (tid == NT - 1) {
+        B.off_init[A.S] = oa;
+        B.off_add[A.S] = ob;
     }
 }
 
-// ---- initial limb points (extended_source.py:100-106): one run of kExtPer consecutive
-// angles per lane.  The lane's first angle starts from the standard initial estimates,
-// each later one from the previous angle's roots.  A warm start can leave two estimates
-// inside one cluster of nearly double images (near a caustic), where the FP64 stopping
-// test accepts both before they separate; the compensated polish that ends every solve
-// continues the Aberth iteration there and takes them to the cluster's distinct roots.
-// Limb point 0 is solved in the reference's root order (ext_solve_point, first).
+// ---- initial limb points (extended_source.py:100-106), two launches.
+// START: the first workgroup plans the batch, with limb darkening (ngl = npts_ld) the next
+// one computes the Gauss-Legendre nodes, and the others solve limb point 0 of every source,
+// flanes sources per workgroup while one wave of each suffices, and set the failure flags.
+// Otherwise: the points after it, one run of kExtPer consecutive angles per lane.  The
+// lane's first angle starts from the standard initial estimates (after point 0: from its
+// roots), each later one from the previous angle's roots.  A warm start can leave two
+// estimates inside one cluster of nearly double images (near a caustic), where the FP64
+// stopping test accepts both before they separate; the compensated polish that ends every
+// solve continues the Aberth iteration there and takes them to the cluster's distinct roots.
+// Point 0 is solved in the reference's root order (ext_solve_point, first).  That solve costs
+// as much as the rest of a run, and one lane of it holds its whole wave: with the points 0
+// inside the runs 12,000 triple-lens sources took 5.6 ms, apart 4.5 ms for both launches (4,096
+// binary ones 0.71 and 0.67 ms).  The nodes were found by a wave of every source before its
+// integration (some 30 us each).  Both launches run one kernel, so that the ill-conditioned
+// solves of all points are compiled, and round, alike.
 template <int NL, int MODE>
 __global__ __launch_bounds__(kExtFlatBlock)
 __attribute__((amdgpu_waves_per_eu(2)))  // 2 waves/SIMD measured faster than 1
-void k_ext_limb_init(ExtArgs A) {
+void k_ext_limb_init(ExtArgs A, int start, int ngl, int flanes) {
     constexpr int DEG = ext_degree<NL>();
     const ExtBatch B = ext_batch(A);
-    const int64_t total = B.off_init[A.S];
-    const int64_t stride = (int64_t)gridDim.x * kExtFlatBlock;
-    for (int64_t t = (int64_t)blockIdx.x * kExtFlatBlock + threadIdx.x; t < total; t += stride) {
-        int64_t lo = 0, hi = A.S;  // off_init[lo] <= t < off_init[hi]
-        while (hi - lo > 1) {
-            const int64_t mid = (lo + hi) >> 1;
-            if (B.off_init[mid] <= t) lo = mid;
-            else hi = mid;
+    int64_t blk = blockIdx.x, per_block = kExtFlatBlock, total, stride;
+    if (start) {
+        if (blk == 0) {
+            ext_plan(A, B);
+            return;
+        }
+        if (ngl && blk == 1) {
+            static_assert(kExtFlatBlock == 2 * kExtGL, "one thread per node");
+            const int part = threadIdx.x / kExtGL, i = threadIdx.x % kExtGL;
+            const int n = part == 0 ? ngl / 2 : ngl - ngl / 2;
+            if (i < n) gauss_legendre(n, i, B.gl + part * kExtGL);
+            return;
+        }
+        blk -= ngl ? 2 : 1;
+        if ((int)threadIdx.x >= flanes) return;
+        per_block = flanes;
+        total = A.S;
+        stride = total;
+    } else {
+        total = B.off_init[A.S];
+        stride = (int64_t)gridDim.x * kExtFlatBlock;
+    }
+    for (int64_t t = blk * per_block + threadIdx.x; t < total; t += stride) {
+        int64_t lo = t;
+        int n, k0 = 0, kb = 0;
+        bool bad = false;
+        if (start) {
+            n = ext_npts(A, t, bad);
+        } else {
+            lo = 0;
+            int64_t hi = A.S;  // off_init[lo] <= t < off_init[hi]
+            while (hi - lo > 1) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (B.off_init[mid] <= t) lo = mid;
+                else hi = mid;
+            }
+            n = B.npts[lo];
+            k0 = (int)(t - B.off_init[lo]) * kExtPer;
+            kb = max(k0, 1);
         }
         const int64_t s = lo;
-        const int M0 = ext_npts_init(B.npts[s]);
-        const int k0 = (int)(t - B.off_init[s]) * kExtPer, k1 = min(M0, k0 + kExtPer);
+        const int M0 = ext_npts_init(n);
+        const int k1 = start ? (n == 0 ? 0 : 1) : min(M0, k0 + kExtPer);
         LensFrame<NL> lf;
         cd w0;
         double rho;
         ext_source<NL>(A, s, lf, w0, rho);
         ExtWS W = ext_ws(ext_source_base<DEG>(A, s), DEG, A.mmax);
         cd z[DEG];
+        if (kb > k0) load_pt<DEG>(W.z[0], 0, z);
         SolveStats st{0, 0, 0, 0};
-        for (int k = k0; k < k1; ++k) {
+        bool fail = bad;
+        for (int k = kb; k < k1; ++k) {
             const double th = ext_limb_angle(k, M0 - 1);
             double sn, cs;
             sincos(th, &sn, &cs);
             uint32_t f;
-            // the lane's later angles start from the previous angle's roots
             if (!ext_solve_point<NL, MODE>(ext_limb_point(w0, rho, cs, sn), lf, z, f, A.itmax,
                                            A.work ? &st : nullptr, k > k0, k == 0))
-                B.fail[s] = 1;
+                fail = true;
             W.theta[0][k] = th;
             store_pt<DEG>(W.z[0], k, z);
             W.flg[0][k] = f;
         }
-        if (A.work) ext_count(A.work, st, k1 - k0);
+        if (start || fail) B.fail[s] = fail ? 1 : 0;
+        if (A.work) ext_count(A.work, st, k1 - kb);
     }
 }
 
@@ -1487,20 +1540,39 @@ void k_ext_solve_add(ExtArgs A, int cur) {
 }
 
 // ---- closed rows, segments and stitching (extended_source.py:156-727) for the final
-// points in buffer `buf`; writes the source's ExtContours
+// points in buffer `buf`; writes the source's ExtContours.  One workgroup per source: its
+// four waves take a quarter of the boundaries each, wave by wave the segments' lengths, and
+// the first one stitches with one remaining segment per lane: the sort is a rank count, each
+// lane tests its segment's four connections, and the nearest admissible one among the four
+// nearest is one wave reduction and a count.
+// Bound: latency of the merge steps.  With every lane of one wave repeating the serial sort
+// and search over records in LDS: one source 45 us, 4,096 binary sources 0.86 ms, 12,000
+// triple-lens sources 3.0 ms; this form 13 us, 0.18 ms, 2.2 ms.
+// LDS written by some lanes of a wave, read by others of the same wave
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+struct ExtCand {          // a candidate segment
+    Seg s;
+    cd h0, h1, t0, t1;    // its lines at the head and at the tail (head_line, tail_line)
+};
 template <int NL>
-__global__ __launch_bounds__(kExtWaveBlock) void k_ext_contours(ExtArgs A, int buf) {
+__global__ __launch_bounds__(kExtBlock) void k_ext_contours(ExtArgs A, int buf) {
     constexpr int DEG = ext_degree<NL>();
     constexpr int NIMG = NL * NL + 1;
     constexpr int NSEG = 3 * NIMG;  // nr_of_segments
     constexpr int NRUN = 10;        // starts / ends kept per row (the reference's split)
+    constexpr int NW = kExtBlock / 64;
+    static_assert(NSEG <= kExtMaxSeg && NSEG < 64, "one segment per lane");
     __shared__ ActSeg s_con[3];
-    __shared__ ActSeg s_act;
-    __shared__ Seg s_cand[kExtMaxSeg];
-    __shared__ int s_st[DEG][NRUN], s_en[DEG][NRUN], s_nst[DEG], s_nen[DEG];
+    __shared__ ExtCand s_cand[NSEG];
+    __shared__ int s_st[NW][DEG][NRUN], s_en[NW][DEG][NRUN], s_nst[NW][DEG], s_nen[NW][DEG];
+    __shared__ int s_ord[64];
     __shared__ unsigned s_allmask;
+    __shared__ int s_nc;
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const int lane = tid & 63, wv = tid >> 6;
     const int64_t src = blockIdx.x;
     const ExtBatch B = ext_batch(A);
     if (B.npts[src] == 0) return;   // skipped source
@@ -1511,10 +1583,10 @@ __global__ __launch_bounds__(kExtWaveBlock) void k_ext_contours(ExtArgs A, int b
     const uint32_t* fb = W.flg[buf];
     // closure test (extended_source.py:289-291)
     if (tid == 0) s_allmask = 0xFFFFu;
-    if (tid < DEG) s_nst[tid] = s_nen[tid] = 0;
+    if (tid < NW * DEG) (&s_nst[0][0])[tid] = (&s_nen[0][0])[tid] = 0;
     __syncthreads();
     unsigned am = 0xFFFFu;
-    for (int k = tid; k < M; k += kExtWaveBlock) am &= fb[k];
+    for (int k = tid; k < M; k += kExtBlock) am &= fb[k];
     atomicAnd(&s_allmask, am);
     __syncthreads();
     unsigned closed = 0;
@@ -1526,75 +1598,85 @@ __global__ __launch_bounds__(kExtWaveBlock) void k_ext_contours(ExtArgs A, int b
     }
     const bool all_closed = closed == (1u << DEG) - 1u;
     if (!all_closed) {
-        // changepoints per boundary c in [0, M] (extended_source.py:163-188); rows that
-        // are closed contribute nothing (their segments were zeroed)
+        // changepoints per boundary c in [0, M] (extended_source.py:163-188), a quarter of the
+        // boundaries per wave; rows that are closed contribute nothing (their segments were
+        // zeroed).  Each wave keeps the first NRUN starts and ends of every row.
         const unsigned open = ((1u << DEG) - 1u) & ~closed;
-        uint64_t* cpw = W.perm;
-        for (int c = tid; c <= M; c += kExtWaveBlock) {
-            uint64_t word = 0;
+        const int share = ((M + 1 + NW - 1) / NW + 63) & ~63;
+        const int c0 = wv * share, c1 = min(M + 1, c0 + share);
+        for (int base = c0; base < c1; base += 64) {
+            const int c = base + lane;
+            unsigned word = 0;
+            if (c < c1) {
+                const unsigned fp = (c > 0) ? fb[c - 1] : 0u, fc = (c < M) ? fb[c] : 0u;
 #pragma unroll
-            for (int r = 0; r < DEG; ++r) {
-                if (!((open >> r) & 1u)) continue;
-                const int mp = (c > 0) ? (int)((fb[c - 1] >> r) & 1u) : 0;
-                const int mc = (c < M) ? (int)((fb[c] >> r) & 1u) : 0;
-                bool cp;
-                int dm;
-                if (c == 0) {
-                    cp = mc != 0;
-                    dm = mc ? 1 : 0;
-                } else if (c == M) {
-                    cp = mp != 0;
-                    dm = mp ? -1 : 0;
-                } else {
-                    const cd za = mp ? pt<DEG>(zb, c - 1, r) : cd{0.0, 0.0};
-                    const cd zc = mc ? pt<DEG>(zb, c, r) : cd{0.0, 0.0};
-                    const int pa = mp ? ((((fb[c - 1] >> (16 + r)) & 1u) ? -1 : 1)) : 0;
-                    const int pc_ = mc ? ((((fb[c] >> (16 + r)) & 1u) ? -1 : 1)) : 0;
-                    dm = mc - mp;
-                    cp = (norm2(zc - za) > 0.01) || (pc_ != pa) || (dm != 0);
+                for (int r = 0; r < DEG; ++r) {
+                    if (!((open >> r) & 1u)) continue;
+                    const int mp = (int)((fp >> r) & 1u), mc = (int)((fc >> r) & 1u);
+                    bool cp;
+                    int dm;
+                    if (c == 0) {
+                        cp = mc != 0;
+                        dm = mc ? 1 : 0;
+                    } else if (c == M) {
+                        cp = mp != 0;
+                        dm = mp ? -1 : 0;
+                    } else {
+                        const cd za = mp ? pt<DEG>(zb, c - 1, r) : cd{0.0, 0.0};
+                        const cd zc = mc ? pt<DEG>(zb, c, r) : cd{0.0, 0.0};
+                        const int pa = mp ? (((fp >> (16 + r)) & 1u) ? -1 : 1) : 0;
+                        const int pc_ = mc ? (((fc >> (16 + r)) & 1u) ? -1 : 1) : 0;
+                        dm = mc - mp;
+                        cp = (norm2(zc - za) > 0.01) || (pc_ != pa) || (dm != 0);
+                    }
+                    if (cp && dm >= 0) word |= 1u << r;
+                    if (cp && dm <= 0) word |= 1u << (16 + r);
                 }
-                if (cp && dm >= 0) word |= 1ull << r;
-                if (cp && dm <= 0) word |= 1ull << (16 + r);
             }
-            cpw[c] = word;
+            if (__ballot(word != 0) == 0ull) continue;
+            const uint64_t below = (1ull << lane) - 1ull;
+            for (int r = 0; r < DEG; ++r) {
+                const uint64_t ms = __ballot((word >> r) & 1u);
+                const uint64_t me = __ballot((word >> (16 + r)) & 1u);
+                if ((ms | me) == 0ull) continue;
+                const int ns = s_nst[wv][r], ne = s_nen[wv][r];
+                if ((word >> r) & 1u) {
+                    const int rank = ns + __popcll(ms & below);
+                    if (rank < NRUN) s_st[wv][r][rank] = c;
+                }
+                if ((word >> (16 + r)) & 1u) {
+                    const int rank = ne + __popcll(me & below);
+                    if (rank < NRUN) s_en[wv][r][rank] = c;
+                }
+                wave_sync();
+                if (lane == 0) {
+                    s_nst[wv][r] = min(NRUN, ns + __popcll(ms));
+                    s_nen[wv][r] = min(NRUN, ne + __popcll(me));
+                }
+                wave_sync();
+            }
         }
         __syncthreads();
-        if (tid < 64) {
-            // the first NRUN starts and ends of every row, by ballots over 64 boundaries
-            for (int base = 0; base <= M; base += 64) {
-                const int c = base + lane;
-                const uint64_t wd = (c <= M) ? cpw[c] : 0ull;
-                const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-                for (int r = 0; r < DEG; ++r) {
-                    const uint64_t ms = __ballot((wd >> r) & 1ull);
-                    const uint64_t me = __ballot((wd >> (16 + r)) & 1ull);
-                    const int ns = s_nst[r], ne = s_nen[r];
-                    if ((wd >> r) & 1ull) {
-                        const int rank = ns + __popcll(ms & below);
-                        if (rank < NRUN) s_st[r][rank] = c;
-                    }
-                    if ((wd >> (16 + r)) & 1ull) {
-                        const int rank = ne + __popcll(me & below);
-                        if (rank < NRUN) s_en[r][rank] = c;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane == 0) {
-                        s_nst[r] = min(NRUN, ns + __popcll(ms));
-                        s_nen[r] = min(NRUN, ne + __popcll(me));
-                    }
-                    __builtin_amdgcn_wave_barrier();
+        if (wv == 0) {
+            // candidate index row*10+slot; nonempty (>= 2 points) ones in descending index
+            // order (:222-240), one index per lane
+            auto nth = [&](const int (&l)[NW][DEG][NRUN], const int (&n)[NW][DEG], int r,
+                           int q) -> int {   // q-th start / end of row r over the waves
+                for (int w = 0; w < NW; ++w) {
+                    if (q < n[w][r]) return l[w][r][q];
+                    q -= n[w][r];
                 }
-            }
-            // candidate index row*10+slot; nonempty (>= 2 points) ones in descending
-            // index order (:222-240); wave-uniform, every lane writes the same values
+                return 0;
+            };
             int nc = 0;
-            for (int r = DEG - 1; r >= 0 && nc < NSEG; --r) {
-                if (!((open >> r) & 1u)) continue;
-                const int ns = s_nst[r], ne = s_nen[r];
-                for (int q = NRUN - 1; q >= 0 && nc < NSEG; --q) {
-                    const int l = q < ns ? s_st[r][q] : 0, rr = q < ne ? s_en[r][q] : 0;
-                    if (l == 0 && rr == 0) continue;
-                    if (rr - l < 2) continue;
+            for (int base = 0; base < DEG * NRUN; base += 64) {
+                const int idx = DEG * NRUN - 1 - (base + lane);
+                const int r = max(idx, 0) / NRUN, q = max(idx, 0) % NRUN;
+                const int l = nth(s_st, s_nst, r, q), rr = nth(s_en, s_nen, r, q);
+                const bool ok = idx >= 0 && ((open >> r) & 1u) && rr - l >= 2;
+                const uint64_t m = __ballot(ok);
+                const int rank = nc + __popcll(m & ((1ull << lane) - 1ull));
+                if (ok && rank < NSEG) {
                     Seg sg;
                     sg.row = r;
                     sg.start = l;
@@ -1604,176 +1686,186 @@ __global__ __launch_bounds__(kExtWaveBlock) void k_ext_contours(ExtArgs A, int b
                     sg.length = 0.0;
                     sg.head = pt<DEG>(zb, l, r);
                     sg.tail = pt<DEG>(zb, rr - 1, r);
-                    s_cand[nc] = sg;
-                    ++nc;
+                    ExtCand& o = s_cand[rank];
+                    o.s = sg;
+                    auto get = [&](int k) { return seg_point<DEG>(zb, sg, k); };
+                    head_line(get, sg.len - 1, o.h0, o.h1);
+                    tail_line(get, sg.len - 1, 4 * M, o.t0, o.t1);
                 }
+                nc = min(NSEG, nc + __popcll(m));
             }
-            for (int q = nc; q < NSEG; ++q) {
-                Seg sg;
-                sg.empty = 1;
-                sg.len = 0;
-                sg.length = 0.0;
-                sg.par = 0;
-                sg.row = 0;
-                sg.start = 0;
-                sg.head = sg.tail = cd{0.0, 0.0};
-                s_cand[q] = sg;
+            if (lane >= nc && lane < NSEG) {
+                ExtCand& o = s_cand[lane];
+                o.s.empty = 1;
+                o.s.len = 0;
+                o.s.length = 0.0;
+                o.s.par = 0;
+                o.s.row = 0;
+                o.s.start = 0;
+                o.s.head = o.s.tail = o.h0 = o.h1 = o.t0 = o.t1 = cd{0.0, 0.0};
             }
-            __builtin_amdgcn_wave_barrier();
-            // segment lengths, lanes over points
-            for (int q = 0; q < nc; ++q) {
-                const Seg sg = s_cand[q];
-                double L = 0.0;
-                for (int k = lane; k + 1 < sg.len; k += 64)
-                    L += sqrt(norm2(pt<DEG>(zb, sg.start + k + 1, sg.row) -
-                                    pt<DEG>(zb, sg.start + k, sg.row)));
-                L = wave_sum(L);
-                __builtin_amdgcn_wave_barrier();
-                if (lane == 0) s_cand[q].length = L;
-                __builtin_amdgcn_wave_barrier();
-            }
-            // stitching, 3 contours, merge scans of 20, 18, 16 (:495-667, :690)
-            Seg* cand = s_cand;
-            ActSeg& act = s_act;
-            int R = NSEG;
+            if (lane == 0) s_nc = nc;
+        }
+        __syncthreads();
+        // segment lengths, a segment per wave in turn, lanes over points
+        for (int q = wv; q < s_nc; q += NW) {
+            const Seg sg = s_cand[q].s;
+            double L = 0.0;
+            for (int k = lane; k + 1 < sg.len; k += 64)
+                L += sqrt(norm2(pt<DEG>(zb, sg.start + k + 1, sg.row) -
+                                pt<DEG>(zb, sg.start + k, sg.row)));
+            L = wave_sum(L);
+            if (lane == 0) s_cand[q].s.length = L;
+        }
+        __syncthreads();
+        if (wv == 0) {
+            // stitching, 3 contours, merge scans of 20, 18, 16 (:495-667, :690); lane q < R
+            // holds the q-th remaining segment
+            int R = NSEG, id = lane < NSEG ? lane : 0;
             int maxm = 20;
-            for (int ci = 0; ci < 3; ++ci) {
+            for (int ci = 0; ci < 3; ++ci, maxm -= 2) {
                 // stable sort by length, empties (length 0) last
-                for (int a = 1; a < R; ++a) {
-                    const Seg key = cand[a];
-                    int b = a - 1;
-                    auto later = [](const Seg& x, const Seg& y) {  // x after y ?
-                        const bool xe = x.empty || x.length == 0.0;
-                        const bool ye = y.empty || y.length == 0.0;
-                        if (xe != ye) return xe;
-                        if (xe) return false;
-                        return x.length > y.length;
-                    };
-                    while (b >= 0 && later(cand[b], key)) {
-                        const Seg t = cand[b];
-                        __builtin_amdgcn_wave_barrier();
-                        cand[b + 1] = t;
-                        __builtin_amdgcn_wave_barrier();
-                        --b;
+                {
+                    const bool xe = s_cand[id].s.empty || s_cand[id].s.length == 0.0;
+                    const double xl = s_cand[id].s.length;
+                    s_ord[lane] = id;
+                    wave_sync();
+                    int rank = 0;
+                    for (int p = 0; p < R; ++p) {
+                        const Seg& o = s_cand[s_ord[p]].s;
+                        const double yl = o.length;
+                        const bool ye = o.empty || yl == 0.0;
+                        // p sorts before this lane's segment
+                        const bool before = xe != ye ? xe : (!xe && xl > yl);
+                        const bool after = xe != ye ? ye : (!xe && yl > xl);
+                        rank += (before || (!after && p < lane)) ? 1 : 0;
                     }
-                    __builtin_amdgcn_wave_barrier();
-                    cand[b + 1] = key;
-                    __builtin_amdgcn_wave_barrier();
+                    wave_sync();
+                    if (lane < R) s_ord[rank] = id;
+                    wave_sync();
                 }
-                const Seg c0 = cand[0];
-                __builtin_amdgcn_wave_barrier();
-                if (lane == 0) {
-                    act.empty = c0.empty;
-                    act.np = 1;
-                    act.pc[0] = Piece{c0.row, c0.start, c0.len, 0};
-                    act.t = c0.empty ? 0 : c0.len - 1;
-                    act.par = c0.par;
-                }
-                cd ah = c0.head, at = c0.tail;  // act's first and last point
-                for (int q = 1; q < R; ++q) {
-                    const Seg t = cand[q];
-                    __builtin_amdgcn_wave_barrier();
-                    cand[q - 1] = t;
-                    __builtin_amdgcn_wave_barrier();
-                }
+                const int i0 = s_ord[0];
                 R -= 1;
-                __builtin_amdgcn_wave_barrier();
+                id = lane < R ? s_ord[lane + 1] : i0;
+                wave_sync();
+                const Seg c0 = s_cand[i0].s;
+                ActSeg& act = s_con[ci];
+                // the contour so far, the same in every lane; its pieces in LDS
+                const int aempty = c0.empty;
+                int np = 1, at_ = c0.empty ? 0 : c0.len - 1, apar = c0.par;
+                if (lane == 0) act.pc[0] = Piece{c0.row, c0.start, c0.len, 0};
+                wave_sync();
+                cd ah = c0.head, at = c0.tail;  // its first and last point
+                const ExtCand me = s_cand[id];
+                cd head = me.s.head, tail = me.s.tail;
+                bool empty = me.s.empty != 0 || lane >= R;
                 for (int it = 0; it < maxm; ++it) {
-                    bool any = false;
-                    for (int q = 0; q < R; ++q) any = any || !cand[q].empty;
-                    if (!any) break;
-                    auto ag = [&](int k) { return act_point<DEG>(zb, act, k); };
-                    // 4 nearest (ctype-major flat index, stable)
-                    int bi[4];
-                    double bd[4];
-                    int nb = 0;
-                    for (int ct = 0; ct < 4; ++ct) {
-                        for (int q = 0; q < R; ++q) {
-                            const cd sh = cand[q].head, stl = cand[q].tail;
-                            const cd d = ct == 0 ? at - sh : ct == 1 ? ah - stl
-                                                           : ct == 2 ? ah - sh : at - stl;
-                            const double dd = sqrt(norm2(d));
-                            const int f = ct * R + q;
-                            int pos = nb;
-                            while (pos > 0 && bd[pos - 1] > dd) --pos;
-                            if (pos < 4) {
-                                for (int u = min(nb, 3); u > pos; --u) {
-                                    bd[u] = bd[u - 1];
-                                    bi[u] = bi[u - 1];
-                                }
-                                bd[pos] = dd;
-                                bi[pos] = f;
-                                if (nb < 4) ++nb;
+                    if (__ballot(!empty) == 0ull) break;
+                    // lines at the contour's ends (head_line, tail_line) from its points 0, 1, 2
+                    // and t, t-1, t-2 and the last two of the reference's dense array, a
+                    // lane each
+                    cd e = cd{0.0, 0.0};
+                    if (lane < 8 && !aempty) {
+                        const int k = lane < 3 ? lane : lane < 6 ? at_ - (lane - 3) : 4 * M - 8 + lane;
+                        if (k >= 0 && k <= at_) e = contour_point<DEG>(zb, act.pc, np, k);
+                    }
+                    cd hx[3], tx[3];
+#pragma unroll
+                    for (int u = 0; u < 3; ++u) {
+                        hx[u] = cd{__shfl(e.re, u, 64), __shfl(e.im, u, 64)};
+                        tx[u] = cd{__shfl(e.re, 3 + u, 64), __shfl(e.im, 3 + u, 64)};
+                    }
+                    const bool hc = (norm2(hx[1] - hx[0]) > 1e-10) || (at_ <= 1);
+                    cd ah0 = hc ? hx[1] : hx[2], ah1 = hc ? hx[0] : hx[1];
+                    const bool tc = (at_ <= 1) || (norm2(tx[0] - tx[1]) > 1e-10);
+                    // t = 0 clamps the line's start to point 0
+                    cd at0 = tc ? (at_ == 0 ? tx[0] : tx[1]) : tx[2];
+                    cd at1 = tc ? (at_ == 0 ? cd{0.0, 0.0} : tx[0]) : tx[1];
+                    if ((tc ? at_ - 1 : at_ - 2) > 4 * M - 2) {   // the slice is clamped there
+                        at0 = cd{__shfl(e.re, 6, 64), __shfl(e.im, 6, 64)};
+                        at1 = cd{__shfl(e.re, 7, 64), __shfl(e.im, 7, 64)};
+                    }
+                    // the four connections of this lane's segment
+                    double dd[4];
+                    dd[0] = sqrt(norm2(at - head));
+                    dd[1] = sqrt(norm2(ah - tail));
+                    dd[2] = sqrt(norm2(ah - head));
+                    dd[3] = sqrt(norm2(at - tail));
+                    double best = 0.0;
+                    int bf = -1;
+                    if (!empty) {   // zero segments connect only within 1e-5 of 0
+                        const bool same = apar * me.s.par > 0;
+#pragma unroll
+                        for (int ct = 0; ct < 4; ++ct) {
+                            if ((ct < 2) != same) continue;
+                            const bool hd = ct == 1 || ct == 2;   // at the contour's head
+                            const bool sh = ct == 0 || ct == 2;   // at the segment's head
+                            if ((bf < 0 || dd[ct] < best) &&
+                                geom_condition(hd ? ah0 : at0, hd ? ah1 : at1,
+                                               sh ? me.h0 : me.t0, sh ? me.h1 : me.t1)) {
+                                best = dd[ct];
+                                bf = ct * R + lane;
                             }
                         }
                     }
-                    int chosen = -1;
-                    for (int u = 0; u < nb && chosen < 0; ++u) {
-                        const int ct = bi[u] / R, q = bi[u] % R;
-                        const Seg sq = cand[q];
-                        if (sq.empty) continue;  // zero segments connect only within 1e-5 of 0
-                        const bool same = act.par * sq.par > 0;
-                        const bool okp = (ct < 2) ? same : !same;
-                        if (!okp) continue;
-                        auto sg = [&](int k) { return seg_point<DEG>(zb, sq, k); };
-                        const int ts = sq.len - 1;
-                        const int dl = 4 * M;
-                        cd a0, a1, b0, b1;
-                        if (ct == 0) {
-                            tail_line(ag, act.t, dl, a0, a1);
-                            head_line(sg, ts, b0, b1);
-                        } else if (ct == 1) {
-                            head_line(ag, act.t, a0, a1);
-                            tail_line(sg, ts, dl, b0, b1);
-                        } else if (ct == 2) {
-                            head_line(ag, act.t, a0, a1);
-                            head_line(sg, ts, b0, b1);
-                        } else {
-                            tail_line(ag, act.t, dl, a0, a1);
-                            tail_line(sg, ts, dl, b0, b1);
+                    if (__ballot(bf >= 0) == 0ull) break;   // nothing connects, now or later
+                    // nearest admissible connection by (distance, ctype-major index)
+                    uint64_t bk = bf >= 0 ? (uint64_t)__double_as_longlong(best) : ~0ull;
+                    int f = bf >= 0 ? bf : 0x7fffffff;
+#pragma unroll
+                    for (int off = 32; off >= 1; off >>= 1) {
+                        const uint64_t ok = __shfl_xor(bk, off, 64);
+                        const int of = __shfl_xor(f, off, 64);
+                        if (ok < bk || (ok == bk && of < f)) {
+                            bk = ok;
+                            f = of;
                         }
-                        if (act.empty) {
-                            a0 = a1 = cd{0.0, 0.0};
-                        }
-                        if (geom_condition(a0, a1, b0, b1)) chosen = u;
                     }
-                    if (chosen < 0) continue;
-                    const int ct = bi[chosen] / R, q = bi[chosen] % R;
-                    const Seg sq = cand[q];
-                    const Piece fw{sq.row, sq.start, sq.len, 0}, bw{sq.row, sq.start, sq.len, 1};
-                    if (act.np >= kExtMaxPieces) continue;
-                    const int np0 = act.np, t0 = act.t, par0 = act.par;
-                    __builtin_amdgcn_wave_barrier();
-                    if (ct == 0) {          // T-H: act + s
-                        if (lane == 0) act.pc[np0] = fw;
-                        at = sq.tail;
-                    } else if (ct == 3) {   // T-T: act + reversed s
-                        if (lane == 0) act.pc[np0] = bw;
-                        at = sq.head;
-                    } else {                // H-T: s + act;  H-H: reversed s + act
-                        if (lane == 0) {
-                            for (int u = np0; u > 0; --u) act.pc[u] = act.pc[u - 1];
-                            act.pc[0] = (ct == 1) ? fw : bw;
-                        }
+                    // it has to be among the four nearest of all, empty ones included
+                    int nearer = 0;
+#pragma unroll
+                    for (int ct = 0; ct < 4; ++ct) {
+                        const uint64_t k = (uint64_t)__double_as_longlong(dd[ct]);
+                        const bool nr = lane < R && (k < bk || (k == bk && ct * R + lane < f));
+                        nearer += __popcll(__ballot(nr));
+                    }
+                    if (nearer >= 4 || np >= kExtMaxPieces) break;
+                    const int ct = f / R, q = f % R;
+                    const int qi = __shfl(id, q, 64);
+                    const Seg sq = s_cand[qi].s;
+                    if (ct == 0 || ct == 3) {   // T-H: act + s;  T-T: act + reversed s
+                        if (lane == 0) act.pc[np] = Piece{sq.row, sq.start, sq.len, ct == 3};
+                        at = ct == 0 ? sq.tail : sq.head;
+                    } else {                    // H-T: s + act;  H-H: reversed s + act
+                        Piece mv{0, 0, 0, 0};
+                        if (lane < np) mv = act.pc[lane];
+                        wave_sync();
+                        if (lane < np) act.pc[lane + 1] = mv;
+                        if (lane == 0) act.pc[0] = Piece{sq.row, sq.start, sq.len, ct == 2};
                         ah = (ct == 1) ? sq.head : sq.tail;
+                        apar = (ct == 1) ? sq.par : -sq.par;
                     }
-                    if (lane == 0) {
-                        act.np = np0 + 1;
-                        act.t = t0 + (sq.len - 1) + 1;
-                        if (ct == 1 || ct == 2) act.par = (ct == 1) ? sq.par : -sq.par;
+                    np += 1;
+                    at_ += sq.len;
+                    if (lane == q) {
                         // the reference zeroes a merged segment (rest[i] = 0): its ends
                         // then rank by their distance from the origin, not as the
                         // contour's own ends
-                        cand[q].empty = 1;
-                        cand[q].head = cd{0.0, 0.0};
-                        cand[q].tail = cd{0.0, 0.0};
+                        empty = true;
+                        head = tail = cd{0.0, 0.0};
+                        s_cand[qi].s.empty = 1;
+                        s_cand[qi].s.head = cd{0.0, 0.0};
+                        s_cand[qi].s.tail = cd{0.0, 0.0};
                     }
-                    (void)par0;
-                    __builtin_amdgcn_wave_barrier();
+                    wave_sync();
                 }
-                if (lane == 0) s_con[ci] = act;
-                __builtin_amdgcn_wave_barrier();
-                maxm -= 2;
+                if (lane == 0) {
+                    act.np = np;
+                    act.t = at_;
+                    act.par = apar;
+                    act.empty = aempty;
+                }
+                wave_sync();
             }
         }
         __syncthreads();
@@ -1781,8 +1873,17 @@ __global__ __launch_bounds__(kExtWaveBlock) void k_ext_contours(ExtArgs A, int b
     if (tid == 0) {
         C->closed = closed;
         C->open = all_closed ? 0 : 1;
-        if (!all_closed) {
-            for (int ci = 0; ci < 3; ++ci) C->con[ci] = s_con[ci];
+    }
+    if (!all_closed) {
+        // the used pieces and the fields after them
+        for (int ci = 0; ci < 3; ++ci) {
+            if (tid < s_con[ci].np) C->con[ci].pc[tid] = s_con[ci].pc[tid];
+            if (tid == 0) {
+                C->con[ci].np = s_con[ci].np;
+                C->con[ci].t = s_con[ci].t;
+                C->con[ci].par = s_con[ci].par;
+                C->con[ci].empty = s_con[ci].empty;
+            }
         }
     }
 }
@@ -1796,7 +1897,7 @@ void k_ext_integrate(ExtArgs A, int buf) {
     constexpr int DEG = ext_degree<NL>();
     constexpr int ND = ext_nd<NL>();
     __shared__ double s_d[8];
-    __shared__ double2 s_gl[2 * 128];
+    __shared__ double2 s_gl[2 * kExtGL];
     const int tid = threadIdx.x;
     const int64_t src = blockIdx.x;
     const ExtBatch B = ext_batch(A);
@@ -1822,9 +1923,8 @@ void k_ext_integrate(ExtArgs A, int buf) {
         g.n1 = A.npts_ld / 2;
         g.n2 = A.npts_ld - g.n1;
         g.a = s_gl;
-        g.b = s_gl + 128;
-        gauss_legendre(g.n1, s_gl);
-        gauss_legendre(g.n2, s_gl + 128);
+        g.b = s_gl + kExtGL;
+        for (int i = tid; i < 2 * kExtGL; i += kExtBlock) s_gl[i] = B.gl[i];
     }
     __syncthreads();
     const ZRows zb{W.z[buf], A.mmax};
@@ -1921,10 +2021,14 @@ template <int NL, int MODE, bool LD, bool VJP>
 int ext_run(hipStream_t s, const ExtArgs& a) {
     const int64_t S = a.S;
     const unsigned nb = (unsigned)S;
-    hipLaunchKernelGGL(k_ext_plan, dim3(1), dim3(kExtPlanBlock), 0, s, a);
+    // points 0: a wave of 16 sources per workgroup while those are few, then full workgroups
+    const int flanes = S <= 16 * 1024 ? 16 : kExtFlatBlock, ngl = LD ? a.npts_ld : 0;
+    hipLaunchKernelGGL((k_ext_limb_init<NL, MODE>),
+                       dim3((unsigned)((S + flanes - 1) / flanes + (LD ? 2 : 1))),
+                       dim3(kExtFlatBlock), 0, s, a, 1, ngl, flanes);
     const int64_t lanes_init = S * (int64_t)((ext_npts_init(a.npts_def) + kExtPer - 1) / kExtPer);
     hipLaunchKernelGGL((k_ext_limb_init<NL, MODE>), dim3(ext_flat_grid(lanes_init)),
-                       dim3(kExtFlatBlock), 0, s, a);
+                       dim3(kExtFlatBlock), 0, s, a, 0, 0, 0);
     hipLaunchKernelGGL((k_ext_chain<NL, false>), dim3(nb), dim3(kExtBlock), 0, s, a, 0);  // initial
     const int add_grid = ext_flat_grid(S * (int64_t)(a.nadd_max > 0 ? a.nadd_max : 1));
     int cur = 0;
@@ -1944,7 +2048,7 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
     }
     hipLaunchKernelGGL((k_ext_chain<NL, true>), dim3(nb), dim3(kExtBlock), 0, s, a, cur);  // final
     if constexpr (NL > 1)
-        hipLaunchKernelGGL((k_ext_contours<NL>), dim3(nb), dim3(kExtWaveBlock), 0, s, a, 1);
+        hipLaunchKernelGGL((k_ext_contours<NL>), dim3(nb), dim3(kExtBlock), 0, s, a, 1);
     hipLaunchKernelGGL((k_ext_integrate<NL, LD, VJP>), dim3(nb), dim3(kExtBlock), 0, s, a, 1);
     return hipGetLastError() == hipSuccess ? CAUS_OK : CAUS_ERR_LAUNCH;
 }

@@ -29,6 +29,7 @@ __device__ __forceinline__ void frame_from_lens_params(const double* p, LensFram
     } else {
         lf.e[1] = p[2];
         lf.e[2] = 1.0 - p[1] - p[2];
+        lf.e01 = p[1] + p[2];
         lf.r[2] = cd{p[3], p[4]};
     }
 }

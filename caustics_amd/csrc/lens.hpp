@@ -17,6 +17,7 @@ template <int NL>
 struct LensFrame {
     double e[NL];  // masses
     cd r[NL];      // positions
+    double e01;    // three lenses: e[0] + e[1]
 };
 
 // Tangent of the lens frame along one parameter direction.
@@ -45,9 +46,12 @@ __device__ __forceinline__ void lens_frame(const double* prm, LensFrame<NL>& lf,
         lf.e[1] = 1.0 - lf.e[0];
     } else {
         const double q3 = prm[2], R = prm[3], psi = prm[4];
+        // explicit fma: the masses enter ill-conditioned polynomials, and every kernel has to
+        // round them alike
         lf.e[0] = q / (1.0 + q + q3);
         lf.e[1] = q * lf.e[0];
-        lf.e[2] = 1.0 - lf.e[0] - lf.e[1];
+        lf.e[2] = fma(-q, lf.e[0], 1.0 - lf.e[0]);
+        lf.e01 = fma(q, lf.e[0], lf.e[0]);
         double sp, cp;
         sincos(psi, &sp, &cp);
         lf.r[2] = cd{R * cp, R * sp};
@@ -116,6 +120,15 @@ __device__ __forceinline__ Poly<A + B - 1> pmul(const Poly<A>& x, const Poly<B>&
     return o;
 }
 
+// a x + y and a x + b y with real weights and explicit fma, so that no kernel contracts them
+// otherwise: an ulp in a coefficient moves nearly multiple roots by its square root
+__device__ __forceinline__ cd axpy(double a, cd x, cd y) {
+    return cd{fma(a, x.re, y.re), fma(a, x.im, y.im)};
+}
+__device__ __forceinline__ cd wsum2(double a, cd x, double b, cd y) {
+    return axpy(a, x, cd{b * y.re, b * y.im});
+}
+
 // Lens polynomial in the lens frame, ascending, degree NL^2+1:
 //   P(z) = (z - w) prod_j M_j - D sum_j e_j prod_{k!=j} M_k,
 //   D = prod_j (z - r_j),  N = sum_j e_j prod_{k!=j} (z - r_k),  M_j = (conj(w) - conj(r_j)) D + N.
@@ -162,8 +175,9 @@ __device__ __forceinline__ void lens_poly(cd w, const LensFrame<NL>& lf, cd (&p)
         Poly<3> D12 = pmul(lin[1], lin[2]);
         Poly<3> Nn;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-            Nn.c[i] = lf.e[0] * D12.c[i] + lf.e[1] * D02.c[i] + lf.e[2] * D01.c[i];
+        for (int i = 0; i < 2; ++i)
+            Nn.c[i] = axpy(lf.e[2], D01.c[i], wsum2(lf.e[0], D12.c[i], lf.e[1], D02.c[i]));
+        Nn.c[2] = cd{lf.e01 + lf.e[2], 0.0};
         Poly<4> M[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -183,7 +197,7 @@ __device__ __forceinline__ void lens_poly(cd w, const LensFrame<NL>& lf, cd (&p)
         Poly<7> S;
 #pragma unroll
         for (int i = 0; i < 7; ++i)
-            S.c[i] = lf.e[0] * M12.c[i] + lf.e[1] * M02.c[i] + lf.e[2] * M01.c[i];
+            S.c[i] = axpy(lf.e[2], M01.c[i], wsum2(lf.e[0], M12.c[i], lf.e[1], M02.c[i]));
         Poly<10> DS = pmul(D, S);
 #pragma unroll
         for (int i = 0; i < 10; ++i) P.c[i] = P.c[i] - DS.c[i];
