@@ -48,6 +48,16 @@ SIGNATURES = {
                                              _i32]),
     "caus_mag_point_source_vjp": (ctypes.c_int, [_vp, _i32, _vp, _i64, _vp, _i64, _vp, _vp, _vp,
                                                  _vp, _vp, _i32, _i32]),
+    "caus_mag_point_source_jac": (ctypes.c_int, [_vp, _i32, _vp, _i64, ctypes.POINTER(_vp),
+                                                 ctypes.POINTER(_i64), _i64, _vp, _vp, _i32,
+                                                 _i32]),
+    "caus_jacobian_workspace_bytes": (ctypes.c_int64, [_i32, _i64, _i64]),
+    "caus_jacobian_vjp": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _i64, _vp, _vp, _vp, _vp,
+                                         _i64]),
+    "caus_lightcurve_point_source_jac": (ctypes.c_int, [_vp, _i32, _vp, _i64,
+                                                        ctypes.POINTER(_vp),
+                                                        ctypes.POINTER(_i64), _i64, _vp, _vp,
+                                                        _i32, _i32]),
     "caus_lightcurve_workspace_bytes": (ctypes.c_int64, [_i32, _i64, _i64]),
     "caus_lightcurve_point_source": (ctypes.c_int, [_vp, _i32, _vp, _i64, _vp, _i64, _vp, _vp,
                                                     _vp, _vp, _i64, _vp, _i32, _i32]),
@@ -124,6 +134,16 @@ def stream_ptr(device=None):
 
 def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def columns(cols):
+    """Device pointers and strides of 1-D float64 columns (stride 0: one value for every
+    row), as two C arrays."""
+    n = len(cols)
+    if any(c.dtype != torch.float64 or not c.is_cuda for c in cols):
+        raise ValueError("parameter columns must be float64 tensors on the GPU")
+    return ((_vp * n)(*[c.data_ptr() for c in cols]),
+            (_i64 * n)(*[c.stride(0) if c.dim() and c.shape[0] > 1 else 0 for c in cols]))
 
 
 def check(rc, what):

@@ -120,20 +120,47 @@ __device__ __forceinline__ double mag_with_tangents(cd wl, const LensFrame<NL>& 
     }
 }
 
+// Parameter columns where they lie: parameter k of row r at p[k][r * st[k]] (stride 0: one
+// value for all rows), so that a caller's tensors need no gathering into rows first.
+constexpr int kPsMaxCols = 9;   // 4 trajectory + 5 lens parameters
+struct PsCols {
+    const double* p[kPsMaxCols];
+    int64_t st[kPsMaxCols];
+    template <int N>
+    __device__ __forceinline__ void load(int64_t row, double (&v)[N]) const {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = p[k][row * st[k]];
+    }
+};
+// columns of row-major rows, row i at rows + i * stride
+inline PsCols ps_rows(const double* rows, int64_t stride) {
+    PsCols c;
+    for (int k = 0; k < kPsMaxCols; ++k) {
+        c.p[k] = rows + k;
+        c.st[k] = stride;
+    }
+    return c;
+}
+
 // ---------------------------------------------------------------------------
 // point-source magnification at arbitrary source positions
-//   VJP=false: mag only.  VJP=true: also g_w = g*(dm/dRe w + i dm/dIm w) and
+//   VJP=false: mag only.  VJP=true: also the derivatives along Re w, Im w and every lens
+//   parameter: with jac they go there plane by plane (jac[d * N + i], the form a later
+//   backward pass scales), else g_w = g*(dm/dRe w + i dm/dIm w) and
 //   g_params[i][k] = g * dm/dparam_k (per evaluation).
+// Item i uses parameter row i / per.
 template <int NL, int MODE, bool VJP>
 __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
-    const cd* __restrict__ w, int64_t N, const double* __restrict__ params, int64_t pstride,
-    const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ g_w,
-    double* __restrict__ g_params, uint8_t* __restrict__ status, int itmax) {
+    const cd* __restrict__ w, int64_t N, PsCols params, int64_t per,
+    const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ jac,
+    double* __restrict__ g_w, double* __restrict__ g_params, uint8_t* __restrict__ status,
+    int itmax) {
     constexpr int NP = NL == 1 ? 0 : n_user_params<NL>();
     constexpr int ND = VJP ? 2 + NP : 0;
     const int64_t i = (int64_t)blockIdx.x * kPsBlock + threadIdx.x;
     if (i >= N) return;
-    const double* prm = params + i * pstride;
+    double prm[NP > 0 ? NP : 1];
+    if constexpr (NP > 0) params.load<NP>(per == 1 ? i : i / per, prm);
     LensFrame<NL> lf;
     double x_cm = 0.0;
     if constexpr (NL == 1) {
@@ -172,6 +199,11 @@ __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
     mag[i] = m;
     if (status) status[i] = ok ? 1 : 0;
     if constexpr (VJP) {
+        if (jac) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) jac[d * N + i] = dm[d];
+            return;
+        }
         const double g = g_mag[i];
         if (g_w) {
             g_w[2 * i] = g * dm[0];
@@ -189,7 +221,8 @@ __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
 // then the lens parameters.  w(t) = e^{-i alpha}(u0 + i tau), tau = (t - t0)/tE
 // (trajectory.py:152-155 without parallax, psi -> alpha).  Grid (ceil(T/256), L):
 // each block is one light curve's chunk of epochs; with VJP the block reduces
-// g_mag * dm/dparam over its epochs in a fixed order into ws[l][chunk][param].
+// g_mag * dm/dparam over its epochs in a fixed order into ws[l][chunk][param]; with jac the
+// derivatives themselves go there plane by plane (jac[param * L T + l * T + epoch]).
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -205,16 +238,17 @@ __host__ __device__ inline int lc_epochs_per_lane(int64_t T, int64_t L) {
 
 template <int NL, int MODE, bool VJP>
 __global__ __launch_bounds__(kPsBlock) void k_lightcurve_point_source(
-    const double* __restrict__ t, int64_t T, const double* __restrict__ lcp,
-    const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ ws,
-    uint8_t* __restrict__ status, int itmax, int epl) {
+    const double* __restrict__ t, int64_t T, PsCols lcp,
+    const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ jac,
+    double* __restrict__ ws, uint8_t* __restrict__ status, int itmax, int epl) {
     constexpr int NP = NL == 1 ? 0 : n_user_params<NL>();
     constexpr int NQ = 4 + NP;
     constexpr int ND = VJP ? NQ : 0;
     constexpr int DEG = NL == 1 ? 2 : ps_degree<NL>();
     __shared__ double red[kPsBlock / 64][NQ];
     const int64_t l = blockIdx.y;
-    const double* prm = lcp + l * NQ;
+    double prm[NQ];
+    lcp.load<NQ>(l, prm);
     double gsum[NQ];
 #pragma unroll
     for (int k = 0; k < NQ; ++k) gsum[k] = 0.0;
@@ -275,13 +309,20 @@ __global__ __launch_bounds__(kPsBlock) void k_lightcurve_point_source(
         mag[l * T + ti] = m;
         if (status) status[l * T + ti] = ok ? 1 : 0;
         if constexpr (VJP) {
-            const double g = g_mag[l * T + ti];
+            if (jac) {
+                const int64_t LT = (int64_t)gridDim.y * T;
 #pragma unroll
-            for (int k = 0; k < NQ; ++k) gsum[k] += g * dm[k];
+                for (int k = 0; k < NQ; ++k) jac[k * LT + l * T + ti] = dm[k];
+            } else {
+                const double g = g_mag[l * T + ti];
+#pragma unroll
+                for (int k = 0; k < NQ; ++k) gsum[k] += g * dm[k];
+            }
         }
     }
     }
     if constexpr (VJP) {
+        if (jac) return;
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
@@ -310,51 +351,52 @@ static __global__ void k_lightcurve_finalize(const double* __restrict__ ws, doub
 }
 
 template <int NL>
-int mag_point_source_nl(hipStream_t s, const cd* w, int64_t N, const double* params,
-                        int64_t pstride, const double* g_mag, double* mag, double* g_w,
-                        double* g_params, uint8_t* status, int itmax, int mode, bool vjp);
+int mag_point_source_nl(hipStream_t s, const cd* w, int64_t N, const PsCols& params,
+                        int64_t per, const double* g_mag, double* mag,
+                        double* jac, double* g_w, double* g_params, uint8_t* status, int itmax,
+                        int mode, bool vjp);
 template <int NL>
-int lightcurve_point_source_nl(hipStream_t s, const double* t, int64_t T, const double* lcp,
-                               int64_t L, const double* g_mag, double* mag, double* ws,
-                               uint8_t* status, int itmax, int mode, bool vjp);
+int lightcurve_point_source_nl(hipStream_t s, const double* t, int64_t T, const PsCols& lcp,
+                               int64_t L, const double* g_mag, double* mag, double* jac,
+                               double* ws, uint8_t* status, int itmax, int mode, bool vjp);
 
 #define CAUS_DEFINE_PS(NL)                                                                       \
     template <>                                                                                  \
-    int mag_point_source_nl<NL>(hipStream_t s, const cd* w, int64_t N, const double* params,    \
-                                int64_t pstride, const double* g_mag, double* mag, double* g_w, \
-                                double* g_params, uint8_t* status, int itmax, int mode,          \
-                                bool vjp) {                                                      \
+    int mag_point_source_nl<NL>(hipStream_t s, const cd* w, int64_t N, const PsCols& params,     \
+                                int64_t per, const double* g_mag, double* mag,                   \
+                                double* jac, double* g_w, double* g_params, uint8_t* status,     \
+                                int itmax, int mode, bool vjp) {                                 \
         const dim3 grid((unsigned)((N + kPsBlock - 1) / kPsBlock)), block(kPsBlock);             \
         switch (mode * 2 + (vjp ? 1 : 0)) {                                                      \
             case 0:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, false>), grid, block, 0, s, \
-                                   w, N, params, pstride, g_mag, mag, g_w, g_params, status,     \
-                                   itmax);                                                       \
+                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, false>), grid, block, 0, s,\
+                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
+                                   status, itmax);                                               \
                 break;                                                                           \
             case 1:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, true>), grid, block, 0, s,  \
-                                   w, N, params, pstride, g_mag, mag, g_w, g_params, status,     \
-                                   itmax);                                                       \
+                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, true>), grid, block, 0, s, \
+                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
+                                   status, itmax);                                               \
                 break;                                                                           \
             case 2:                                                                              \
                 hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64_COMP, false>), grid, block, \
-                                   0, s, w, N, params, pstride, g_mag, mag, g_w, g_params,       \
-                                   status, itmax);                                               \
+                                   0, s, w, N, params, per, g_mag, mag, jac, g_w,                \
+                                   g_params, status, itmax);                                     \
                 break;                                                                           \
             case 3:                                                                              \
                 hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64_COMP, true>), grid, block,  \
-                                   0, s, w, N, params, pstride, g_mag, mag, g_w, g_params,       \
-                                   status, itmax);                                               \
+                                   0, s, w, N, params, per, g_mag, mag, jac, g_w,                \
+                                   g_params, status, itmax);                                     \
                 break;                                                                           \
             case 4:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, false>), grid, block, 0, s, \
-                                   w, N, params, pstride, g_mag, mag, g_w, g_params, status,     \
-                                   itmax);                                                       \
+                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, false>), grid, block, 0, s,\
+                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
+                                   status, itmax);                                               \
                 break;                                                                           \
             case 5:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, true>), grid, block, 0, s,  \
-                                   w, N, params, pstride, g_mag, mag, g_w, g_params, status,     \
-                                   itmax);                                                       \
+                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, true>), grid, block, 0, s, \
+                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
+                                   status, itmax);                                               \
                 break;                                                                           \
             default:                                                                             \
                 return CAUS_ERR_ARG;                                                             \
@@ -362,37 +404,43 @@ int lightcurve_point_source_nl(hipStream_t s, const double* t, int64_t T, const 
         return hipGetLastError() == hipSuccess ? CAUS_OK : CAUS_ERR_LAUNCH;                      \
     }                                                                                            \
     template <>                                                                                  \
-    int lightcurve_point_source_nl<NL>(hipStream_t s, const double* t, int64_t T,               \
-                                       const double* lcp, int64_t L, const double* g_mag,        \
-                                       double* mag, double* ws, uint8_t* status, int itmax,      \
+    int lightcurve_point_source_nl<NL>(hipStream_t s, const double* t, int64_t T,                \
+                                       const PsCols& lcp, int64_t L, const double* g_mag,        \
+                                       double* mag, double* jac, double* ws, uint8_t* status, int itmax,\
                                        int mode, bool vjp) {                                     \
         const int epl = lc_epochs_per_lane(T, L);                                                \
         const int64_t per_block = (int64_t)kPsBlock * epl;                                       \
-        const dim3 grid((unsigned)((T + per_block - 1) / per_block), (unsigned)L), block(kPsBlock); \
+        const dim3 grid((unsigned)((T + per_block - 1) / per_block), (unsigned)L), block(kPsBlock);\
         switch (mode * 2 + (vjp ? 1 : 0)) {                                                      \
             case 0:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64, false>), grid,      \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             case 1:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64, true>), grid,       \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             case 2:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64_COMP, false>), grid, \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             case 3:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64_COMP, true>), grid,  \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             case 4:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_CF32, false>), grid,      \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             case 5:                                                                              \
                 hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_CF32, true>), grid,       \
-                                   block, 0, s, t, T, lcp, g_mag, mag, ws, status, itmax, epl);       \
+                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
+                                   epl);                                                         \
                 break;                                                                           \
             default:                                                                             \
                 return CAUS_ERR_ARG;                                                             \

@@ -4,9 +4,9 @@
 epochs along rectilinear trajectories w(t) = e^{-i alpha}(u0 + i (t - t0)/tE)
 (src/caustics/trajectory.py:152-155 with no parallax and psi -> alpha), one fused
 HIP kernel per (light curve, epoch).  Its gradient with respect to every parameter
-(t0, u0, tE, alpha and the lens parameters) comes from the fused forward+VJP kernel,
-which re-solves the roots, forms per-epoch implicit-derivative tangents and reduces
-them per light curve in a fixed order (deterministic).
+(t0, u0, tE, alpha and the lens parameters) comes from the per-epoch implicit-derivative
+tangents that the same kernel keeps where one is needed; the backward pass scales them
+and sums them per light curve in a fixed order (deterministic).
 
 ``lightcurve_fwd_vjp`` exposes that fused kernel directly: one root solve gives the
 magnifications and the vector-Jacobian product for a cotangent ``g_mag``.
@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .point_source import PARAM_NAMES, _mode_id
+from .point_source import JACOBIAN_MAX_BYTES, PARAM_NAMES, _mode_id, jacobian_vjp
 
 __all__ = ["mag_point_source_lightcurve", "lightcurve_fwd_vjp", "hexadecapole_gate",
            "hexadecapole_vjp", "mag", "mag_fwd_vjp", "TRAJ_NAMES"]
@@ -56,19 +56,49 @@ def lightcurve_fwd_vjp(t, lc_params, g_mag, nlenses=2, roots_itmax=2500, mode="f
 
 
 class _LightCurve(torch.autograd.Function):
+    """Columns of the L parameter rows (each one value or L) to (L, T) magnifications; where
+    a gradient is needed the forward keeps the Jacobian, which the backward scales and sums
+    over each light curve."""
+
     @staticmethod
-    def forward(ctx, nlenses, itmax, mode, t, lcp):
-        mag, _, _ = _call(t, lcp, None, nlenses, itmax, mode)
-        ctx.save_for_backward(t, lcp)
-        ctx.meta = (nlenses, itmax, mode)
+    def forward(ctx, nlenses, itmax, mode, need, t, *cols):
+        L = max([c.numel() for c in cols])
+        T = t.numel()
+        flat = [c.reshape(-1) if c.numel() == L else c.reshape(-1).expand(L) for c in cols]
+        mag = torch.empty((L, T), dtype=torch.float64, device=t.device)
+        jac = None
+        if need and len(cols) * 8 * L * T <= JACOBIAN_MAX_BYTES:
+            jac = torch.empty((len(cols), L * T), dtype=torch.float64, device=t.device)
+        rc = _lib.lib().caus_lightcurve_point_source_jac(
+            _lib.stream_ptr(), nlenses, _lib.ptr(t), T, *_lib.columns(flat), L, _lib.ptr(mag),
+            _lib.ptr(jac), itmax, mode)
+        _lib.check(rc, "caus_lightcurve_point_source_jac")
+        if need:
+            ctx.save_for_backward(t, jac, *([] if jac is not None else
+                                            [torch.stack(flat, -1).contiguous()]))
+        ctx.meta = (nlenses, itmax, mode, L, [c.shape for c in cols])
         return mag
 
     @staticmethod
     def backward(ctx, g):
-        t, lcp = ctx.saved_tensors
-        nlenses, itmax, mode = ctx.meta
-        _, gp, _ = _call(t, lcp, g.contiguous().to(torch.float64), nlenses, itmax, mode)
-        return None, None, None, None, gp
+        t, jac, *lcp = ctx.saved_tensors
+        nlenses, itmax, mode, L, shapes = ctx.meta
+        g = g.contiguous().to(torch.float64)
+        if jac is not None:
+            _, gp = jacobian_vjp(jac, 0, max(t.numel(), 1), g, False, True)
+        else:
+            _, gp, _ = _call(t, lcp[0], g, nlenses, itmax, mode)
+            gp = gp.t()
+        if t.numel() == 0:
+            gp = torch.zeros((len(shapes), L), dtype=torch.float64, device=t.device)
+        gps = []
+        gp = gp.unbind(0)
+        for k, shape in enumerate(shapes):
+            if not ctx.needs_input_grad[5 + k]:
+                gps.append(None)
+            else:
+                gps.append((gp[k] if shape.numel() == L else gp[k].sum()).reshape(shape))
+        return (None, None, None, None, None, *gps)
 
 
 def mag_point_source_lightcurve(t, t0, u0, tE, alpha, nlenses=2, roots_itmax=2500,
@@ -80,11 +110,10 @@ def mag_point_source_lightcurve(t, t0, u0, tE, alpha, nlenses=2, roots_itmax=250
     vals = dict(t0=t0, u0=u0, tE=tE, alpha=alpha, **params)
     cols = [torch.as_tensor(np.asarray(vals[n]) if not isinstance(vals[n], torch.Tensor)
                             else vals[n], device="cuda").to(torch.float64) for n in names]
-    L = max([c.numel() for c in cols])
-    lcp = torch.stack([c.reshape(-1).expand(L) for c in cols], -1).contiguous()
     t = torch.as_tensor(t, device="cuda", dtype=torch.float64).contiguous().reshape(-1)
-    return _LightCurve.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode), t,
-                             lcp)
+    need = torch.is_grad_enabled() and any(c.requires_grad for c in cols)
+    return _LightCurve.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode), need,
+                             t, *cols)
 
 
 def hexadecapole_gate(w_points, rho, nlenses=2, u1=0.0, roots_itmax=2500, **params):

@@ -3,9 +3,9 @@
 ``mag_point_source(w, nlenses=2, roots_itmax=2500, roots_compensated=False, **params)``
 (:1762-1830) runs in one fused HIP kernel per evaluation: parameter map and x_cm
 shift, FP64 coefficients, all-roots solve, lens-equation filter (1e-6), sum of
-1/|det J|.  Its gradient (torch.autograd) comes from the fused VJP kernel, which
-re-solves the roots and pushes implicit-derivative tangents of w and of every lens
-parameter through det J.
+1/|det J|.  Where a gradient is needed (torch.autograd) the same kernel pushes
+implicit-derivative tangents of w and of every lens parameter through det J and keeps
+that Jacobian; the backward pass scales it and sums it over broadcast parameters.
 
 ``lens_eq`` and ``lens_eq_det_jac`` (:1536-1580) take lens-frame parameters
 (a, e1[, e2, r3]) exactly as in the reference and are elementwise tensor expressions.
@@ -60,56 +60,114 @@ def _prepare(w, nlenses, params):
     return w, ps
 
 
+# A backward pass scales and reduces the Jacobian that the forward pass kept, (2 + P) * 8
+# bytes a position (a light curve's epoch (4 + P) * 8).  Solving the roots again instead
+# costs 8 times as much (512,000 binary epochs: 93 against 11 us on one MI355X) and no
+# memory, so calls whose Jacobian would exceed this many bytes do that.
+JACOBIAN_MAX_BYTES = 4 << 30
+
+
+def jacobian_vjp(jac, nw, rows, g, want_w, want_p):
+    """Backward pass of the kept Jacobian jac (nw + np, N) for cotangents g (N,): (g_w (N,)
+    complex or None, g_p (np, N / rows) sums over rows of consecutive items or None)."""
+    npl, N = jac.shape
+    n_p = npl - nw
+    g_w = torch.empty(N, dtype=torch.complex128, device=jac.device) if want_w else None
+    g_p = None
+    if want_p and n_p:
+        shape = (n_p, N // rows)
+        g_p = (torch.empty if N else torch.zeros)(shape, dtype=torch.float64, device=jac.device)
+    L = _lib.lib()
+    wsb = L.caus_jacobian_workspace_bytes(n_p, N, rows)
+    ws = torch.empty(wsb // 8, dtype=torch.float64, device=jac.device) if wsb > 0 else None
+    rc = L.caus_jacobian_vjp(_lib.stream_ptr(), _lib.ptr(jac), N, nw, n_p, rows, _lib.ptr(g),
+                             _lib.ptr(g_w), _lib.ptr(g_p), _lib.ptr(ws), wsb)
+    _lib.check(rc, "caus_jacobian_vjp")
+    return g_w, g_p
+
+
+def _param_rows(shape, ps):
+    """Items per parameter row when every parameter is broadcast over the same trailing
+    dimensions of shape (the shape of the items), else 1 (a row for each item)."""
+    N = 1
+    for n in shape:
+        N *= n
+    if all(p.numel() == 1 for p in ps):
+        return max(N, 1)
+    first = (1,) * (len(shape) - ps[0].dim()) + tuple(ps[0].shape)
+    if any((1,) * (len(shape) - p.dim()) + tuple(p.shape) != first for p in ps[1:]):
+        return 1
+    per, d = 1, len(shape)
+    while d > 0 and first[d - 1] == 1:
+        d -= 1
+        per *= shape[d]
+    return per if first[:d] == tuple(shape[:d]) and N else 1
+
+
 class _MagPointSource(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, nlenses, itmax, mode, w, *ps):
-        shape = torch.broadcast_shapes(w.shape, *[p.shape for p in ps]) if ps else w.shape
+    def forward(ctx, nlenses, itmax, mode, need, w, *ps):
+        shape = torch.broadcast_tensors(w, *ps)[0].shape
         wf = w.expand(shape).contiguous().reshape(-1)
         N = wf.numel()
         P = len(ps)
-        if P and all(p.numel() == 1 for p in ps):
-            prm = torch.stack([p.reshape(()) for p in ps]).contiguous()
-            pstride = 0
-        elif P:
-            prm = torch.stack([p.expand(shape).reshape(-1) for p in ps], -1).contiguous()
-            pstride = P
+        per = _param_rows(shape, ps) if P else 1
+        if per > 1 or N == 1:
+            cols = [p.reshape(-1) for p in ps]
         else:
-            prm = None
-            pstride = 0
+            cols = [p.expand(shape).reshape(-1) for p in ps]
         mag = torch.empty(N, dtype=torch.float64, device=w.device)
-        status = torch.empty(N, dtype=torch.uint8, device=w.device)
-        rc = _lib.lib().caus_mag_point_source(_lib.stream_ptr(), nlenses, _lib.ptr(wf), N,
-                                              _lib.ptr(prm), pstride, _lib.ptr(mag),
-                                              _lib.ptr(status), itmax, mode)
-        _lib.check(rc, "caus_mag_point_source")
-        ctx.save_for_backward(wf, *( [prm] if prm is not None else []))
-        ctx.meta = (nlenses, itmax, mode, shape, pstride, w.shape, [p.shape for p in ps])
+        jac = None
+        if need and (2 + P) * 8 * N <= JACOBIAN_MAX_BYTES:
+            jac = torch.empty((2 + P, N), dtype=torch.float64, device=w.device)
+        rc = _lib.lib().caus_mag_point_source_jac(_lib.stream_ptr(), nlenses, _lib.ptr(wf), N,
+                                                  *_lib.columns(cols), per, _lib.ptr(mag),
+                                                  _lib.ptr(jac), itmax, mode)
+        _lib.check(rc, "caus_mag_point_source_jac")
+        if jac is not None:
+            ctx.save_for_backward(wf, jac)
+        elif need:
+            prm = torch.stack([c.expand(N // per) for c in cols], -1).contiguous() if P else None
+            ctx.save_for_backward(wf, None, prm)
+        ctx.meta = (nlenses, itmax, mode, shape, per, w.shape, [p.shape for p in ps])
         return mag.reshape(shape)
 
     @staticmethod
     def backward(ctx, g):
-        nlenses, itmax, mode, shape, pstride, wshape, pshapes = ctx.meta
-        saved = ctx.saved_tensors
-        wf = saved[0]
-        prm = saved[1] if len(saved) > 1 else None
-        N = wf.numel()
+        nlenses, itmax, mode, shape, per, wshape, pshapes = ctx.meta
+        wf, jac, *prm = ctx.saved_tensors
         P = len(pshapes)
+        N = wf.numel()
+        want_w, want_p = ctx.needs_input_grad[4], any(ctx.needs_input_grad[5:])
         gf = g.expand(shape).contiguous().reshape(-1).to(torch.float64)
-        mag = torch.empty(N, dtype=torch.float64, device=wf.device)
-        g_w = torch.empty(N, dtype=torch.complex128, device=wf.device)
-        g_p = torch.empty((N, max(P, 1)), dtype=torch.float64, device=wf.device)
-        rc = _lib.lib().caus_mag_point_source_vjp(
-            _lib.stream_ptr(), nlenses, _lib.ptr(wf), N, _lib.ptr(prm), pstride, _lib.ptr(gf),
-            _lib.ptr(mag), _lib.ptr(g_w), _lib.ptr(g_p), None, itmax, mode)
-        _lib.check(rc, "caus_mag_point_source_vjp")
-        gw = g_w.reshape(shape).sum_to_size(wshape) if ctx.needs_input_grad[3] else None
+        if jac is not None:
+            g_w, g_p = jacobian_vjp(jac, 2, per, gf, want_w, want_p)
+            pshape = shape if per == 1 else None   # summed over the rows already
+        else:
+            prm = prm[0] if P else None
+            pstride = P if P and prm.shape[0] > 1 else 0
+            if pstride and per > 1:
+                prm = prm.repeat_interleave(per, 0)
+            mag = torch.empty(N, dtype=torch.float64, device=wf.device)
+            g_w = torch.empty(N, dtype=torch.complex128, device=wf.device)
+            g_p = torch.empty((N, max(P, 1)), dtype=torch.float64, device=wf.device)
+            rc = _lib.lib().caus_mag_point_source_vjp(
+                _lib.stream_ptr(), nlenses, _lib.ptr(wf), N, _lib.ptr(prm), pstride, _lib.ptr(gf),
+                _lib.ptr(mag), _lib.ptr(g_w), _lib.ptr(g_p), None, itmax, mode)
+            _lib.check(rc, "caus_mag_point_source_vjp")
+            g_p = g_p.t()
+            pshape = shape
+        gw = g_w.reshape(shape).sum_to_size(wshape) if want_w else None
         gps = []
+        g_p = g_p.unbind(0) if g_p is not None else None
         for k, ps_shape in enumerate(pshapes):
-            if ctx.needs_input_grad[4 + k]:
-                gps.append(g_p[:, k].reshape(shape).sum_to_size(ps_shape))
-            else:
+            if not ctx.needs_input_grad[5 + k]:
                 gps.append(None)
-        return (None, None, None, gw, *gps)
+            elif pshape is None:
+                gps.append(g_p[k].reshape(ps_shape))
+            else:
+                gps.append(g_p[k].reshape(shape).sum_to_size(ps_shape))
+        return (None, None, None, None, gw, *gps)
 
 
 def mag_point_source(w, nlenses=2, roots_itmax=2500, roots_compensated=False, mode=None,
@@ -123,8 +181,9 @@ def mag_point_source(w, nlenses=2, roots_itmax=2500, roots_compensated=False, mo
     if nlenses not in (1, 2, 3):
         raise ValueError("`nlenses` has to be set to be <= 3.")
     w, ps = _prepare(w, nlenses, params)
+    need = torch.is_grad_enabled() and (w.requires_grad or any(p.requires_grad for p in ps))
     return _MagPointSource.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode),
-                                 w, *ps)
+                                 need, w, *ps)
 
 
 _DEGREE = {1: 2, 2: 5, 3: 10}

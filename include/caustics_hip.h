@@ -120,6 +120,29 @@ int caus_mag_point_source_vjp(void* stream, int32_t nlenses, const double* w, in
                               double* mag, double* g_w, double* g_params, uint8_t* status,
                               int32_t itmax, int32_t mode);
 
+/* Magnification with its Jacobian kept for a later backward pass: one root solve, no
+ * cotangents yet.
+ *   params   P columns (device pointers in a host array) and their strides: parameter k of
+ *            row r at params[k][r * strides[k]], stride 0 for one value
+ *   per      items per parameter row: item i uses row i / per
+ *   jac      (2+P, N) output or NULL (magnification only): dmag/dRe w, dmag/dIm w,
+ *            dmag/dparam_k, each a plane of N */
+int caus_mag_point_source_jac(void* stream, int32_t nlenses, const double* w, int64_t N,
+                              const double* const* params, const int64_t* strides,
+                              int64_t per, double* mag, double* jac, int32_t itmax, int32_t mode);
+
+/* The backward pass of a kept Jacobian of nw + np planes of N, nw (0 or 2) of them along
+ * Re w and Im w, for cotangents g (N,):
+ *   g_w      (N,) complex or NULL:  g * (plane 0 + i plane 1)
+ *   g_params (np, N / R) or NULL:   sum of g * plane over each row of R consecutive items
+ *            (R = 1: per item), in a fixed order
+ *   workspace of caus_jacobian_workspace_bytes(np, N, R) bytes (-1: invalid arguments;
+ *   R must divide N, np <= 9) */
+int64_t caus_jacobian_workspace_bytes(int32_t np, int64_t N, int64_t R);
+int caus_jacobian_vjp(void* stream, const double* jac, int64_t N, int32_t nw, int32_t np,
+                      int64_t R, const double* g, double* g_w, double* g_params,
+                      double* workspace, int64_t workspace_bytes);
+
 /* Point-source light curves along rectilinear trajectories w(t) = e^{-i alpha}(u0 + i (t-t0)/tE)
  * (src/caustics/trajectory.py:152-155 without parallax), L light curves x T epochs.
  *   t          (T,) epochs;  lc_params (L, 4+P) rows (t0, u0, tE, alpha, lens params...)
@@ -134,6 +157,14 @@ int caus_lightcurve_point_source(void* stream, int32_t nlenses, const double* t,
                                  double* mag, double* g_params, double* workspace,
                                  int64_t workspace_bytes, uint8_t* status, int32_t itmax,
                                  int32_t mode);
+
+/* Light curves with their Jacobian kept for a later backward pass (caus_jacobian_vjp with
+ * nw = 0, np = 4+P, R = T): 4+P parameter columns of L rows as above, jac (4+P, L, T)
+ * planes dmag/dparam or NULL.  L <= 65535. */
+int caus_lightcurve_point_source_jac(void* stream, int32_t nlenses, const double* t, int64_t T,
+                                     const double* const* params, const int64_t* strides,
+                                     int64_t L, double* mag, double* jac, int32_t itmax,
+                                     int32_t mode);
 
 /* caus_lightcurve_point_source without a workspace argument: it allocates nothing and
  * takes no caller memory beyond inputs and outputs.  No counterpart in the reference; it

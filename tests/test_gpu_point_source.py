@@ -226,3 +226,81 @@ def test_critical_and_caustic_curves(gpu, nlenses):
     lp, x_cm = lens.lens_params(nlenses, **prm)
     det = lens.lens_eq_det_jac(zc + x_cm, nlenses, **lp)
     assert np.max(np.abs(det)) < 1e-9
+
+
+# rows of one item, of a wave (up to 512), one item past it, one workgroup, several chunks with
+# a ragged last one; the scalar case is one row over everything
+@pytest.mark.parametrize("rows,per", [(7, 1), (9, 2), (5, 512), (3, 513), (300, 700), (2, 2049),
+                                      (1, 6200)])
+@pytest.mark.parametrize("nlenses", [2, 3])
+def test_kept_jacobian_sums(gpu, nlenses, rows, per, monkeypatch):
+    """Gradients summed over broadcast parameters equal the sums of per-position gradients
+    (to the rounding of a sum of `per` terms), and equal those of the backward pass that
+    solves again."""
+    from caustics_amd import _lib, lightcurve, point_source
+    g = np.random.default_rng(rows * per + nlenses)
+    p = dict(s=g.uniform(0.6, 1.6, (rows, 1)), q=10 ** g.uniform(-3, 0, (rows, 1)))
+    if nlenses == 3:
+        p.update(q3=10 ** g.uniform(-3, -1, (rows, 1)), r3=g.uniform(0.3, 1.5, (rows, 1)),
+                 psi=g.uniform(0, 6, (rows, 1)))
+    w = torch.as_tensor(g.normal(size=(rows, per)) + 1j * g.normal(size=(rows, per)),
+                        device="cuda")
+    gm = torch.as_tensor(g.normal(size=(rows, per)), device="cuda")
+
+    def grads(full):
+        wl = w.clone().requires_grad_()
+        ps = {k: torch.as_tensor(np.broadcast_to(v, (rows, per)) if full else v,
+                                 device="cuda").clone().requires_grad_() for k, v in p.items()}
+        m = ca.mag_point_source(wl, nlenses=nlenses, **ps)
+        return [x.cpu().numpy() for x in (m.detach(), *torch.autograd.grad(
+            m, [wl, *ps.values()], gm))]
+
+    item, row = grads(True), grads(False)
+    np.testing.assert_array_equal(item[0], row[0])
+    np.testing.assert_array_equal(item[1], row[1])
+    eps = np.finfo(float).eps
+
+    def close(a, terms):
+        bound = 2 * per * eps * np.abs(terms).sum(1, keepdims=True)
+        assert (np.abs(a - terms.sum(1, keepdims=True)) <= bound).all()
+
+    for a, terms in zip(row[2:], item[2:]):
+        close(a, terms)
+    monkeypatch.setattr(point_source, "JACOBIAN_MAX_BYTES", 0)
+    again = grads(False)
+    np.testing.assert_array_equal(again[0], row[0])
+    np.testing.assert_array_equal(again[1], row[1])
+    for a, terms in zip(again[2:], item[2:]):
+        close(a, terms)
+    monkeypatch.undo()
+
+    # light curves: rows of `per` epochs, one parameter shared by all of them
+    t = torch.as_tensor(np.sort(g.uniform(-2, 2, per)), device="cuda")
+    cols = dict(t0=g.uniform(-0.2, 0.2, rows), u0=np.array(0.31), tE=g.uniform(1, 2, rows),
+                alpha=g.uniform(0, 6, rows), **{k: v[:, 0] for k, v in p.items()})
+
+    def lc():
+        ps = {k: torch.as_tensor(v, device="cuda").requires_grad_() for k, v in cols.items()}
+        m = ca.mag_point_source_lightcurve(t, nlenses=nlenses, **ps)
+        return [x.cpu().numpy() for x in (m.detach(), *torch.autograd.grad(
+            m, list(ps.values()), gm))]
+
+    kept = lc()
+    monkeypatch.setattr(lightcurve, "JACOBIAN_MAX_BYTES", 0)
+    again = lc()
+    flat = [torch.as_tensor(v, device="cuda").reshape(-1).expand(rows) for v in cols.values()]
+    jac = torch.empty((len(cols), rows, per), dtype=torch.float64, device="cuda")
+    mag = torch.empty((rows, per), dtype=torch.float64, device="cuda")
+    assert _lib.lib().caus_lightcurve_point_source_jac(
+        _lib.stream_ptr(), nlenses, _lib.ptr(t), per, *_lib.columns(flat), rows, _lib.ptr(mag),
+        _lib.ptr(jac), 2500, _lib.MODES["fp64"]) == _lib.CAUS_OK
+    np.testing.assert_array_equal(kept[0], mag.cpu().numpy())
+    np.testing.assert_array_equal(again[0], kept[0])
+    for k, name in enumerate(cols):
+        terms = (gm * jac[k]).cpu().numpy()
+        if name == "u0":   # shared by all the light curves
+            terms = terms.reshape(1, -1)
+        n = terms.shape[1]
+        for got in (kept[1 + k], again[1 + k]):
+            bound = 2 * n * eps * np.abs(terms).sum(1)
+            assert (np.abs(got.reshape(-1) - terms.sum(1)) <= bound).all(), name
