@@ -953,9 +953,10 @@ __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* 
 //                                  per lane
 //   k_ext_chain       per source   image continuation (extended_source.py:34-53), limb
 //                                  order and gap keys of the initial points
-//   10 x k_ext_select per source   gap-key sort, insertion shifts, next limb order, tasks
+//   10 x k_ext_select per source   largest gaps, insertion shifts, next limb order, tasks
 //        k_ext_solve_add flat      new points appended, matched to their left neighbour,
 //                                  keys of their two gaps
+//   (small batches: k_ext_init_grouped for the second launch, k_ext_refine for all rounds)
 //   k_ext_chain       per source   points gathered in limb order, image continuation
 //   k_ext_contours    per source   closure test, segments, stitching -> piece lists
 //   k_ext_integrate   per source   contour integrals, magnification, reverse mode
@@ -1335,18 +1336,32 @@ __global__ __launch_bounds__(kExtBlock) void k_ext_chain(ExtArgs A, int cur) {
 // took 15.5 us at 150 limb points (one source) and 361 us for 4,096 binary sources of
 // 256-4096 points.
 constexpr int kExtSelWave = 512;
+// LDS written by some lanes of a wave, read by others of the same wave
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int NT, int PER>
+struct ExtSelLds {
+    int cnt[2][NT / 64];           // bisection counts, double buffered (one barrier a step)
+    uint64_t max[NT / 64];
+    int sel[PER * (NT / 64)];      // selected / tied keys per (register, wave)
+};
+// the NT threads tid = 0 .. NT-1 of a workgroup run it together (one wave of a larger
+// workgroup where NT is 64)
 template <int NL, int NT, int PER>
-__global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round) {
+__device__ __forceinline__ void ext_select(const ExtArgs& A, const ExtBatch& B, int64_t src, int n,
+                                           int cur, int round, int tid, ExtSelLds<NT, PER>& sh) {
     constexpr int DEG = ext_degree<NL>();
     constexpr int NW = NT / 64;
-    __shared__ int s_cnt[2][NW];       // bisection counts, double buffered (one barrier a step)
-    __shared__ uint64_t s_max[NW];
-    __shared__ int s_sel[PER * NW];    // selected / tied keys per (register, wave)
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int64_t src = blockIdx.x;
-    const ExtBatch B = ext_batch(A);
-    const int n = B.npts[src];
-    if (n == 0) return;   // skipped source
+    auto sync = [] {
+        if constexpr (NW > 1) __syncthreads();
+        else wave_sync();
+    };
+    int (&s_cnt)[2][NW] = sh.cnt;
+    uint64_t (&s_max)[NW] = sh.max;
+    int (&s_sel)[PER * NW] = sh.sel;
+    const int lane = tid & 63, wv = tid >> 6;
     const int M = ext_points(n, round), nadd = ext_n_add(n);   // M <= PER * NT
     ExtWS W = ext_ws(ext_source_base<DEG>(A, src), DEG, A.mmax);
     const int nxt = cur ^ 1;
@@ -1423,7 +1438,7 @@ __global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round
             const uint64_t m = __ballot(key[i] == lo && tid + i * NT < M - 1);
             if (lane == 0) s_sel[i * NW + wv] = __popcll(m);
         }
-        __syncthreads();
+        sync();
         for (int q = 0; q < PER * NW; ++q) tot += s_sel[q];
         int before = 0;
 #pragma unroll
@@ -1438,7 +1453,7 @@ __global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round
             const int rank = b + __popcll(m & ((1ull << lane) - 1ull));   // ties before this one
             if (key[i] > lo || (tie && tot - rank <= nadd - chi)) sel |= 1u << i;
         }
-        __syncthreads();
+        sync();
     }
     // insertion shift of every point = selected gaps before it
     uint64_t bal[PER];
@@ -1482,6 +1497,15 @@ __global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round
             W.gk[nxt][d] = key[i];
         }
     }
+}
+template <int NL, int NT, int PER>
+__global__ __launch_bounds__(NT) void k_ext_select(ExtArgs A, int cur, int round) {
+    __shared__ ExtSelLds<NT, PER> sh;
+    const int64_t src = blockIdx.x;
+    const ExtBatch B = ext_batch(A);
+    const int n = B.npts[src];
+    if (n == 0) return;   // skipped source
+    ext_select<NL, NT, PER>(A, B, src, n, cur, round, threadIdx.x, sh);
 }
 
 // ---- one refinement round, part 2: every new point of the batch, one per lane,
@@ -1539,6 +1563,322 @@ void k_ext_solve_add(ExtArgs A, int cur) {
     }
 }
 
+// ---- one polynomial per group of lanes, one root per lane -------------------------------
+// A small batch has too few limb points to fill the device with one polynomial per lane, and
+// a launch then lasts as long as one lane needs for all DEG roots after each other.  Here lane
+// j of a group of 8 (two lenses) or 16 (three) holds root j: an Ehrlich-Aberth sweep and a
+// sweep of the compensated polish take one root's instructions.  Roots are exchanged through
+// LDS within a wave.  All roots move together (Jacobi form), where the one-lane solver moves
+// them one after the other; both end in the compensated polish, which takes every root to the
+// double nearest the exact one whatever led there, so the results are the same.
+template <int NL>
+constexpr int ext_group() {
+    return NL == 3 ? 16 : 8;
+}
+
+// sweeps of the group's polish: only clusters need more than two, and there all roots moving
+// together take more of them than one after the other (kPolishSweeps)
+constexpr int kGroupPolishSweeps = 40;
+template <int NL>
+struct GroupSolve {
+    static constexpr int DEG = ext_degree<NL>();
+    static constexpr int GL = ext_group<NL>();
+    static_assert(DEG < GL, "a lane per coefficient");
+    double2* zs;   // this group's GL slots
+    int j;         // root of this lane (valid below DEG)
+
+    __device__ __forceinline__ void put(cd z) const {
+        wave_sync();
+        zs[j] = make_double2(z.re, z.im);
+        wave_sync();
+    }
+    __device__ __forceinline__ cd get(int i) const {
+        const double2 v = zs[i];
+        return cd{v.x, v.y};
+    }
+    // sum over the other roots of 1/(x - z_i); they are read from the group's slots
+    template <int RCP_STEPS>
+    __device__ __forceinline__ cd aberth(cd x) const {
+        cd S = cd{0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < DEG; ++i) {
+            cd d = x - get(i);
+            const bool own = i == j;
+            d.re = own ? 1.0 : d.re;   // keeps the reciprocal finite
+            const cd r = crcp<RCP_STEPS>(d);
+            S = S + cd{own ? 0.0 : r.re, own ? 0.0 : r.im};
+        }
+        return S;
+    }
+    // plain FP64 sweeps until every root of every group of the wave has met the stopping test
+    // (fast_step); returns whether this lane's root has
+    __device__ __forceinline__ bool iterate(const cd (&p)[DEG + 1], cd& z, int itmax,
+                                            SolveStats& st) const {
+        double al[DEG + 1];
+#pragma unroll
+        for (int i = 0; i <= DEG; ++i) al[i] = cabs(p[i]);
+#pragma unroll
+        for (int i = 0; i <= DEG; ++i) al[i] = al[i] * fma(ALPHA_W, (double)i, 1.0);
+        bool done = j >= DEG;
+        for (int it = 0; it < itmax && __ballot(!done) != 0ull; ++it) {
+            put(z);
+            if (done) continue;
+            ++st.it64;
+            const cd x = z;
+            const double ax = __builtin_amdgcn_sqrt(norm2(x));
+            double b = al[DEG];
+#pragma unroll
+            for (int k = DEG - 1; k >= 0; --k) b = fma(b, ax, al[k]);
+            cd h = p[DEG], hd = cd{0.0, 0.0};
+#pragma unroll
+            for (int k = DEG - 1; k >= 0; --k) {
+                hd = cfma(hd, x, h);
+                h = cfma(h, x, p[k]);
+            }
+            const double tb = EA_EPS * b;
+            if (norm2(h) > tb * tb)
+                z = x - cdiv<2>(h, hd - h * aberth<0>(x));
+            else
+                done = true;
+        }
+        return done;
+    }
+    // polish_roots, every root of a sweep at once
+    __device__ __forceinline__ void polish(const cd (&p)[DEG + 1], cd& z) const {
+        bool act = j < DEG;
+        for (int sweep = 0; sweep < kGroupPolishSweeps && __ballot(act) != 0ull; ++sweep) {
+            put(z);
+            if (!act) continue;
+            cd h, hd;
+            if (sweep == 0)
+                horner_comp_value<DEG>(p, z, h, hd);
+            else
+                horner_comp_vd<DEG>(p, z, h, hd);
+            const cd den = hd - h * aberth<2>(z);
+            act = false;
+            if (norm2(den) > 0.0) {
+                const cd corr = cdiv<2>(h, den);
+                const cd zn = z - corr;
+                if (isfinite(zn.re) && isfinite(zn.im)) {
+                    act = norm2(corr) > 0x1p-80 * norm2(z);
+                    z = zn;
+                }
+            }
+        }
+    }
+};
+
+// this lane's group within its wave: the lanes' bits of a ballot
+template <int GL>
+__device__ __forceinline__ uint32_t group_bits(uint64_t ballot) {
+    const int base = (threadIdx.x & 63) & ~(GL - 1);
+    return (uint32_t)(ballot >> base) & ((1u << GL) - 1u);
+}
+
+// limb point at angle th of one source by one group: the roots (one a lane, left in the
+// group's slots) and the flag word; false if one did not converge
+template <int NL>
+__device__ __forceinline__ bool ext_group_point(const GroupSolve<NL>& G, cd w,
+                                                const LensFrame<NL>& lf, cd& z, int itmax,
+                                                uint32_t& flags, SolveStats& st) {
+    constexpr int DEG = ext_degree<NL>();
+    constexpr int GL = ext_group<NL>();
+    bool ok = true, real = true, neg = false;
+    if constexpr (NL == 1) {
+        const double sq = sqrt(1.0 + 4.0 * rcp(norm2(w)));
+        z = (G.j == 0 ? 0.5 * (1.0 + sq) : 0.5 * (1.0 - sq)) * w;
+        neg = norm2(z) < 1.0;
+    } else {
+        cd p[DEG + 1];
+        lens_poly<NL>(w, lf, p);
+        ok = G.iterate(p, z, itmax, st);
+        ok = ok && (G.j >= DEG || (isfinite(z.re) && isfinite(z.im)));
+        G.polish(p, z);
+        const ImageTerms<NL> it = image_terms<NL>(z, lf);
+        real = norm2(z - it.G - w) < 1e-12;
+        neg = 1.0 - norm2(it.K) < 0.0;
+    }
+    const uint32_t in = (1u << DEG) - 1u;
+    const uint32_t fr = group_bits<GL>(__ballot(real)) & in;
+    const uint32_t fn = group_bits<GL>(__ballot(neg)) & in;
+    flags = fr | (fn << 16);
+    G.put(z);
+    return (group_bits<GL>(__ballot(ok)) & in) == in;
+}
+
+// The third lens' position from its polar form again, where the solve's coefficients are
+// formed: there the compiler contracts the products into the sums that take them, as it does
+// in k_ext_solve_add, and the ill-conditioned roots near a lens of small mass follow an ulp of
+// a coefficient by up to its square root.
+__device__ __forceinline__ void lens3_refresh(const double* prm, double sp, double cp,
+                                              LensFrame<3>& lf) {
+    double R = prm[3];
+    asm volatile("" : "+v"(R));   // not hoisted out of the caller's loop
+    lf.r[2] = cd{R * cp, R * sp};
+}
+
+// ---- the initial limb points after point 0, one a group of lanes, each from point 0's roots;
+// per_source workgroups for every source.  Used where the batch is small (ext_grouped).
+template <int NL>
+__global__ __launch_bounds__(kExtBlock) void k_ext_init_grouped(ExtArgs A, int per_source) {
+    constexpr int DEG = ext_degree<NL>();
+    constexpr int GL = ext_group<NL>();
+    __shared__ double2 s_z[kExtBlock];
+    const int tid = threadIdx.x;
+    const int64_t src = blockIdx.x / per_source;
+    const ExtBatch B = ext_batch(A);
+    const int M0 = ext_npts_init(B.npts[src]);
+    const int k0 = 1 + (int)(blockIdx.x % per_source) * (kExtBlock / GL);
+    if (k0 >= M0) return;
+    const int kq = k0 + tid / GL;
+    const bool mine = kq < M0;
+    const int k = mine ? kq : M0 - 1;   // groups past the last point repeat it, write nothing
+    LensFrame<NL> lf;
+    cd w0;
+    double rho;
+    ext_source<NL>(A, src, lf, w0, rho);
+    ExtWS W = ext_ws(ext_source_base<DEG>(A, src), DEG, A.mmax);
+    const int j = tid & (GL - 1);
+    const GroupSolve<NL> G{s_z + (tid & ~(GL - 1)), j};
+    const double th = ext_limb_angle(k, M0 - 1);
+    double sn, cs;
+    sincos(th, &sn, &cs);
+    cd z = j < DEG ? W.z[0][j] : cd{0.0, 0.0};
+    uint32_t f;
+    SolveStats st{0, 0, 0, 0};
+    const bool ok = ext_group_point<NL>(G, ext_limb_point(w0, rho, cs, sn), lf, z, A.itmax,
+                                        f, st);
+    if (!mine) return;
+    if (j < DEG) W.z[0][(size_t)k * DEG + j] = z;
+    if (j == 0) {
+        W.theta[0][k] = th;
+        W.flg[0][k] = f;
+        if (!ok) B.fail[src] = 1;
+    }
+    if (A.work) ext_count(A.work, st, j == 0 ? 1 : 0);
+}
+
+// ---- all ten refinement rounds of one source by one workgroup: ext_select, then the new
+// points one a group of lanes.  Used where the batch is small (ext_grouped).
+// Bound: latency of the rounds' serial steps (figures: ext_grouped).
+template <int NL, int SELT, int PER>
+__global__ __launch_bounds__(kExtBlock) void k_ext_refine(ExtArgs A) {
+    constexpr int DEG = ext_degree<NL>();
+    constexpr int GL = ext_group<NL>();
+    __shared__ ExtSelLds<SELT, PER> sh;
+    __shared__ double2 s_z[kExtBlock], s_left[kExtBlock];
+    const int tid = threadIdx.x;
+    const int64_t src = blockIdx.x;
+    const ExtBatch B = ext_batch(A);
+    const int n = B.npts[src];
+    if (n == 0) return;   // skipped source
+    const int nadd = ext_n_add(n);
+    const int64_t t0 = B.off_add[src];
+    LensFrame<NL> lf;
+    cd w0;
+    double rho;
+    ext_source<NL>(A, src, lf, w0, rho);
+    ExtWS W = ext_ws(ext_source_base<DEG>(A, src), DEG, A.mmax);
+    double sp3 = 0.0, cp3 = 0.0;
+    if constexpr (NL == 3) sincos(A.params[src * A.pstride + 4], &sp3, &cp3);
+    const int j = tid & (GL - 1), base = tid & ~(GL - 1);
+    const GroupSolve<NL> G{s_z + base, j};
+    double2* const lefts = s_left + base;
+    SolveStats st{0, 0, 0, 0};
+    bool fail = false;
+    int cur = 0;
+    for (int round = 0; round < 10; ++round, cur ^= 1) {
+        if (tid < SELT) ext_select<NL, SELT, PER>(A, B, src, n, cur, round, tid, sh);
+        __syncthreads();
+        const int nxt = cur ^ 1;
+        for (int q0 = 0; q0 < nadd; q0 += kExtBlock / GL) {
+            // groups past the last point repeat it and write nothing
+            const int q = q0 + tid / GL;
+            const bool mine = q < nadd;
+            const int64_t t = t0 + (mine ? q : nadd - 1);
+            const int a = B.t_left[t], b = B.t_right[t], d = B.t_dst[t], e = B.t_app[t];
+            const double th = B.t_th[t];
+            const cd left = j < DEG ? W.z[0][(size_t)a * DEG + j] : cd{0.0, 0.0};
+            const cd right = j < DEG ? W.z[0][(size_t)b * DEG + j] : cd{0.0, 0.0};
+            const uint32_t fa = W.flg[0][a], fb = W.flg[0][b];
+            lefts[j] = make_double2(left.re, left.im);
+            double sn, cs;
+            sincos(th, &sn, &cs);
+            if constexpr (NL == 3) lens3_refresh(A.params + src * A.pstride, sp3, cp3, lf);
+            cd z = left;   // start from the left neighbour
+            uint32_t f;
+            SolveStats s1{0, 0, 0, 0};
+            const bool ok = ext_group_point<NL>(G, ext_limb_point(w0, rho, cs, sn), lf, z, A.itmax,
+                                                f, s1);
+            if (mine) {
+                st.it64 += s1.it64;
+                fail |= !ok;
+            }
+            // nearest new image of left row j; rows that take distinct ones follow them
+            // whatever the row order, otherwise row by row (greedy_match)
+            int bj = 0;
+            double best = 0.0;
+            bool nan = false;
+#pragma unroll
+            for (int i = 0; i < DEG; ++i) {
+                const double dd = norm2(G.get(i) - left);
+                nan |= dd != dd;
+                if (i == 0 || dd < best) {
+                    best = dd;
+                    bj = i;
+                }
+            }
+            const bool odd = group_bits<GL>(__ballot(nan && j < DEG)) != 0;
+            uint32_t hit = j < DEG ? 1u << bj : 0u;
+#pragma unroll
+            for (int off = 1; off < GL; off <<= 1) hit |= __shfl_xor(hit, off, 64);
+            if (odd || hit != (1u << DEG) - 1u) {
+                unsigned used = 0;
+#pragma unroll 1
+                for (int i = 0; i < DEG; ++i) {
+                    const double2 lv = lefts[i];
+                    double bd = 0.0;
+                    int bi = -1;
+#pragma unroll 1
+                    for (int c = 0; c < DEG; ++c) {
+                        const double dd = norm2(G.get(c) - cd{lv.x, lv.y});
+                        if (!((used >> c) & 1u) && (bi < 0 || dd < bd)) {
+                            bd = dd;
+                            bi = c;
+                        }
+                    }
+                    used |= 1u << bi;
+                    if (i == j) bj = bi;
+                }
+            }
+            // output row j = raw row bj
+            const cd zn = G.get(bj);
+            const uint32_t in = (1u << DEG) - 1u;
+            const uint32_t fo =
+                (group_bits<GL>(__ballot((f >> bj) & 1u)) & in) |
+                ((group_bits<GL>(__ballot((f >> (16 + bj)) & 1u)) & in) << 16);
+            // keys of the gaps (left, new) at d-1 and (new, right) at d (gap_key)
+            double d1 = j < DEG && (((fa | fo) >> j) & 1u) ? norm2(zn - left) : 0.0;
+            double d2 = j < DEG && (((fo | fb) >> j) & 1u) ? norm2(right - zn) : 0.0;
+#pragma unroll
+            for (int off = 1; off < GL; off <<= 1) {
+                d1 = fmax(d1, __shfl_xor(d1, off, 64));
+                d2 = fmax(d2, __shfl_xor(d2, off, 64));
+            }
+            if (mine && j < DEG) W.z[0][(size_t)e * DEG + j] = zn;
+            if (mine && j == 0) {
+                W.flg[0][e] = fo;
+                W.theta[0][e] = th;
+                W.gk[nxt][d - 1] = (uint64_t)__double_as_longlong(sqrt(fmax(0.0, d1)));
+                W.gk[nxt][d] = (uint64_t)__double_as_longlong(sqrt(fmax(0.0, d2)));
+            }
+        }
+        __syncthreads();
+    }
+    if (fail) B.fail[src] = 1;
+    if (A.work) ext_count(A.work, st, tid == 0 ? 10 * nadd : 0);
+}
+
 // ---- closed rows, segments and stitching (extended_source.py:156-727) for the final
 // points in buffer `buf`; writes the source's ExtContours.  One workgroup per source: its
 // four waves take a quarter of the boundaries each, wave by wave the segments' lengths, and
@@ -1548,11 +1888,6 @@ void k_ext_solve_add(ExtArgs A, int cur) {
 // Bound: latency of the merge steps.  With every lane of one wave repeating the serial sort
 // and search over records in LDS: one source 45 us, 4,096 binary sources 0.86 ms, 12,000
 // triple-lens sources 3.0 ms; this form 13 us, 0.18 ms, 2.2 ms.
-// LDS written by some lanes of a wave, read by others of the same wave
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 struct ExtCand {          // a candidate segment
     Seg s;
     cd h0, h1, t0, t1;    // its lines at the head and at the tail (head_line, tail_line)
@@ -2016,6 +2351,22 @@ void k_ext_integrate(ExtArgs A, int buf) {
 
 int ext_flat_grid(int64_t max_lanes);
 
+// Whether a batch is small enough for one limb point per group of lanes (k_ext_init_grouped,
+// k_ext_refine).  A group's eight or sixteen lanes issue about twice (two lenses) and three
+// times (three) the instructions of one lane per point, so it pays while the flat kernels
+// leave the device mostly idle.  Whole calls on one MI355X, flat -> grouped, uniform disks: two
+// lenses 337 -> 164 us (one source of 150 limb points), 462 -> 289 (400 of 200), 738 -> 628
+// (1,200 of 256), 961 -> 1436 (4,000 of 200); three lenses 1181 -> 780, 2026 -> 1353,
+// 2477 -> 2058, 3586 -> 5706.  Sources with sizes of their own count for less, since most are
+// far below the largest: 1,000 of 256-1024 points 624 -> 484 (two) and 1617 -> 1597 us (three),
+// 1,200 of 256-4096 1016 -> 1373 and 3666 -> 4860.
+template <int NL>
+bool ext_grouped(const ExtArgs& a) {
+    constexpr int64_t tasks = 16000, sources = 1200;
+    const int64_t share = a.npts ? (NL == 3 ? 2 : 4) : 1;
+    return a.S <= sources && a.S * a.nadd_max <= tasks * share;
+}
+
 // the launch sequence for one batch of nlenses = NL
 template <int NL, int MODE, bool LD, bool VJP>
 int ext_run(hipStream_t s, const ExtArgs& a) {
@@ -2027,11 +2378,33 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
                        dim3((unsigned)((S + flanes - 1) / flanes + (LD ? 2 : 1))),
                        dim3(kExtFlatBlock), 0, s, a, 1, ngl, flanes);
     const int64_t lanes_init = S * (int64_t)((ext_npts_init(a.npts_def) + kExtPer - 1) / kExtPer);
-    hipLaunchKernelGGL((k_ext_limb_init<NL, MODE>), dim3(ext_flat_grid(lanes_init)),
-                       dim3(kExtFlatBlock), 0, s, a, 0, 0, 0);
+    const bool grouped = MODE == MODE_FP64 && ext_grouped<NL>(a);
+    // three lenses keep k_ext_limb_init: its coefficients' rounding decides the ill-conditioned
+    // roots near a lens of small mass
+    bool init_grouped = false;
+    if constexpr (NL < 3) init_grouped = grouped;
+    if (init_grouped) {
+        constexpr int per_block = kExtBlock / ext_group<NL>();
+        const int n0 = ext_npts_init(a.npts_def) - 1;
+        const int per_source = n0 > per_block ? (n0 + per_block - 1) / per_block : 1;
+        if constexpr (NL < 3)
+            hipLaunchKernelGGL((k_ext_init_grouped<NL>), dim3(nb * per_source), dim3(kExtBlock), 0,
+                               s, a, per_source);
+    } else {
+        hipLaunchKernelGGL((k_ext_limb_init<NL, MODE>), dim3(ext_flat_grid(lanes_init)),
+                           dim3(kExtFlatBlock), 0, s, a, 0, 0, 0);
+    }
     hipLaunchKernelGGL((k_ext_chain<NL, false>), dim3(nb), dim3(kExtBlock), 0, s, a, 0);  // initial
     const int add_grid = ext_flat_grid(S * (int64_t)(a.nadd_max > 0 ? a.nadd_max : 1));
     int cur = 0;
+    if (grouped) {
+        if (a.mmax <= kExtSelWave)
+            hipLaunchKernelGGL((k_ext_refine<NL, kExtWaveBlock, kExtSelWave / 64>), dim3(nb),
+                               dim3(kExtBlock), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_ext_refine<NL, kExtBlock, kExtSortMax / kExtBlock>), dim3(nb),
+                               dim3(kExtBlock), 0, s, a);
+    } else {
     static_assert(kExtSelWave % 64 == 0 && kExtSortMax % kExtBlock == 0, "select register tiles");
     for (int round = 0; round < 10; ++round) {
         // one wave while its 8 registers of keys hold the contour (no barrier in the
@@ -2045,6 +2418,7 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
         hipLaunchKernelGGL((k_ext_solve_add<NL, MODE>), dim3(add_grid), dim3(kExtFlatBlock), 0, s,
                            a, cur);
         cur ^= 1;
+    }
     }
     hipLaunchKernelGGL((k_ext_chain<NL, true>), dim3(nb), dim3(kExtBlock), 0, s, a, cur);  // final
     if constexpr (NL > 1)

@@ -443,3 +443,32 @@ def test_line_integral_rule_sizes(gpu, nlenses, npts_ld, u1):
     assert torch.isfinite(g).all()
     mo = np.array([E.mag_extended_source(x, rho, u1=u1, **kw, **prm) for x in w])
     compare(m, mo, f"rule n={npts_ld} u1={u1} nlenses={nlenses}")
+
+
+# limb sizes without new points (below 20), of one and two registers a wave in the selection,
+# above one wave's, the largest; a last pass of groups that is only partly filled
+@pytest.mark.parametrize("npts", [4, 19, 20, 150, 520, 1500, 4096])
+@pytest.mark.parametrize("nlenses", [1, 2, 3])
+def test_small_batches_match_large_ones(gpu, nlenses, npts):
+    """A few sources (solved by groups of lanes, all refinement rounds in one launch) give what
+    the same sources give inside a batch too large for that (one limb point per lane): every
+    root ends at the double nearest the exact one on both ways."""
+    from caustics_amd.extended_source import extended_fwd_vjp
+    g = np.random.default_rng(npts + nlenses)
+    n = 5
+    w = 0.3 * (g.normal(size=n) + 1j * g.normal(size=n))
+    rho = 10 ** g.uniform(-2.5, -0.8, n)
+    p = {}
+    if nlenses > 1:
+        p.update(s=g.uniform(0.7, 1.4, n), q=10 ** g.uniform(-3, 0, n))
+    if nlenses == 3:
+        p.update(q3=10 ** g.uniform(-3, -1, n), r3=g.uniform(0.3, 1.5, n),
+                 psi=g.uniform(0, 2 * np.pi, n))
+    copies = 1250 // n if npts < 150 else 16000 // (n * (npts // 20)) + 2
+    rep = lambda x: np.tile(x, copies)  # noqa: E731
+    kw = dict(nlenses=nlenses, npts_limb=npts, limb_darkening=npts != 150, u1=0.4, npts_ld=10)
+    few = extended_fwd_vjp(w, rho, np.ones(n), **kw, **p)
+    many = extended_fwd_vjp(rep(w), rep(rho), np.ones(n * copies), **kw,
+                            **{k: rep(v) for k, v in p.items()})
+    for a, b in zip(few, many):
+        np.testing.assert_allclose(a.cpu().numpy(), b.cpu().numpy()[:n], rtol=1e-12, atol=1e-12)
