@@ -74,6 +74,10 @@ SIGNATURES = {
                                                      _i32, _i32, _vp, _i64, _i32, _vp, _vp, _vp,
                                                      _vp, _vp, _i64, _i32, _i32, _vp]),
     "caus_match_chain": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i32, _i64]),
+    "caus_critical_curves_workspace_bytes": (ctypes.c_int64, [_i32, _i64, _i64]),
+    "caus_critical_curves": (ctypes.c_int, [_vp, _i32, ctypes.POINTER(_vp), ctypes.POINTER(_i64),
+                                            ctypes.POINTER(ctypes.c_double), _i64, _vp, _i64,
+                                            _vp, _vp, _vp, _i64, _i32]),
     "caus_images_point_source": (ctypes.c_int, [_vp, _i32, _vp, _i64, _i64, _vp, _i64, _vp, _vp,
                                                 _vp, _vp, _i32, _i32, _i32]),
     "caus_marginalized_log_likelihood": (ctypes.c_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp,

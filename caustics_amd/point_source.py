@@ -17,6 +17,8 @@ lens-frame parameters; the sequential form warm-starts each position from the pr
 one's roots, so that row j follows one image along the sequence.  They return no
 gradients (``mag_point_source`` and ``ehrlich_aberth`` do).
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -345,17 +347,52 @@ def _critical_coeffs(phi, nlenses, a, e1, e2=None, r3=None):
 def critical_and_caustic_curves(npts=200, nlenses=2, **params):
     """Critical curves and caustics, each (n_curves, npts) complex, in the frame of the
     reference API (point_source.py:1582-1649): roots of the critical-curve polynomial
-    on a grid of phi (GPU solver), continued along phi with match_points (HIP kernel),
-    mapped through the lens equation and shifted by x_cm.  Parameters may also be
+    on a grid of phi (GPU solver), continued along phi with match_points, mapped through
+    the lens equation and shifted by x_cm (HIP kernels).  Parameters may also be
     arrays of length B, giving (B, n_curves, npts)."""
-    from .ehrlich_aberth_primitive import poly_roots
-
     phi = torch.linspace(-np.pi, np.pi, npts, dtype=torch.float64, device="cuda")
     if nlenses == 1:
         return torch.exp(-1j * phi), torch.zeros(npts, dtype=torch.complex128, device="cuda")
     names = PARAM_NAMES[nlenses]
-    vals = [torch.as_tensor(np.asarray(params[k]) if not isinstance(params[k], torch.Tensor)
-                            else params[k], device="cuda").to(torch.float64) for k in names]
+    if torch.is_grad_enabled() and any(isinstance(params[k], torch.Tensor)
+                                       and params[k].requires_grad for k in names):
+        return _curves_tensor(phi, nlenses, [params[k] for k in names])
+    # numbers go to the kernels by value
+    vals = [v if isinstance(v, torch.Tensor) else np.asarray(v) for v in
+            (params[k] for k in names)]
+    batch = vals[0].ndim > 0
+    cols = [None if isinstance(v, np.ndarray) and v.ndim == 0 else
+            torch.as_tensor(v, device="cuda").to(torch.float64).reshape(-1) for v in vals]
+    B = torch.broadcast_shapes(*[(1,) if c is None else c.shape for c in cols])[0]
+    P = len(cols)
+    n = _DEGREE_CRITICAL[nlenses]
+    crit = torch.empty((B, n, npts), dtype=torch.complex128, device="cuda")
+    caus = torch.empty_like(crit)
+    L = _lib.lib()
+    wsb = L.caus_critical_curves_workspace_bytes(nlenses, B, npts)
+    ws = torch.empty((wsb + 7) // 8, dtype=torch.float64, device="cuda")
+    rc = L.caus_critical_curves(
+        _lib.stream_ptr(), nlenses,
+        (ctypes.c_void_p * P)(*[None if c is None else c.data_ptr() for c in cols]),
+        (ctypes.c_int64 * P)(*[0 if c is None or c.numel() == 1 else c.stride(0) for c in cols]),
+        (ctypes.c_double * P)(*[float(v) if c is None else 0.0 for v, c in zip(vals, cols)]),
+        B, _lib.ptr(phi), npts, _lib.ptr(crit), _lib.ptr(caus), _lib.ptr(ws), wsb, 2000)
+    _lib.check(rc, "caus_critical_curves")
+    return (crit, caus) if batch else (crit[0], caus[0])
+
+
+_DEGREE_CRITICAL = {2: 4, 3: 6}
+
+
+def _curves_tensor(phi, nlenses, params):
+    """critical_and_caustic_curves as tensor expressions around the root solver and the
+    continuation, for parameters that require a gradient (it flows through the explicit
+    dependence of the map and the shift on them)."""
+    from .ehrlich_aberth_primitive import poly_roots
+
+    npts = phi.numel()
+    vals = [torch.as_tensor(np.asarray(v) if not isinstance(v, torch.Tensor) else v,
+                            device="cuda").to(torch.float64) for v in params]
     batch = vals[0].dim() > 0
     vals = [v.reshape(-1, 1) for v in vals]
     s, q = vals[0], vals[1]

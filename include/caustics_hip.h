@@ -280,6 +280,20 @@ int caus_mag_extended_source_work(void* stream, int32_t nlenses, const double* w
 int caus_match_chain(void* stream, const double* pts, double* out, int64_t npts, int32_t n,
                      int64_t nchains);
 
+/* Critical curves and caustics of B lenses at npts phases (reference:
+ * critical_and_caustic_curves, src/caustics/point_source.py:1582-1649), nlenses 2 or 3.
+ *   params, strides, values   host arrays, one entry per parameter (s, q[, q3, r3, psi]):
+ *            a device column with its stride (0: one value for every lens), or NULL and the
+ *            value itself
+ *   phi      (npts,) phases on the device
+ *   critical, caustic  (B, n, npts) complex outputs, n = 4 or 6, in the frame of the API
+ *   workspace of caus_critical_curves_workspace_bytes(nlenses, B, npts) bytes */
+int64_t caus_critical_curves_workspace_bytes(int32_t nlenses, int64_t B, int64_t npts);
+int caus_critical_curves(void* stream, int32_t nlenses, const double* const* params,
+                         const int64_t* strides, const double* values, int64_t B,
+                         const double* phi, int64_t npts, double* critical, double* caustic,
+                         void* workspace, int64_t workspace_bytes, int32_t itmax);
+
 /* Images of point sources in the lens frame (reference: _images_point_source,
  * src/caustics/point_source.py:1652-1709) and their sequential, warm-started form
  * (_images_point_source_sequential, :1711-1759).

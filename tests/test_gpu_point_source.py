@@ -304,3 +304,29 @@ def test_kept_jacobian_sums(gpu, nlenses, rows, per, monkeypatch):
         for got in (kept[1 + k], again[1 + k]):
             bound = 2 * n * eps * np.abs(terms).sum(1)
             assert (np.abs(got.reshape(-1) - terms.sum(1)) <= bound).all(), name
+
+
+# one phase, one wave's phases and one more, the default; parameters as numbers, arrays and
+# tensors, one of them shared by the batch
+@pytest.mark.parametrize("npts", [1, 2, 64, 65, 200])
+@pytest.mark.parametrize("nlenses", [2, 3])
+def test_curves_match_tensor_form(gpu, nlenses, npts):
+    """The fused curves equal the tensor expressions of the same polynomial, roots and map (row
+    for row: the coefficients are rounded alike)."""
+    from caustics_amd.point_source import critical_and_caustic_curves
+    g = np.random.default_rng(npts)
+    B = 3
+    p = dict(s=g.uniform(0.6, 1.6, B), q=10 ** g.uniform(-2, 0, B))
+    if nlenses == 3:
+        p.update(q3=0.02, r3=g.uniform(0.5, 1.2, B), psi=g.uniform(0, 6, B))
+    one = {k: float(np.asarray(v).reshape(-1)[0]) for k, v in p.items()}
+    forms = [(one, ()), (p, (B,)),
+             ({**p, "q": torch.as_tensor(p["q"], device="cuda")}, (B,))]
+    for prm, shape in forms:
+        got = critical_and_caustic_curves(npts=npts, nlenses=nlenses, **prm)
+        ref = critical_and_caustic_curves(npts=npts, nlenses=nlenses, **{
+            k: torch.as_tensor(v, dtype=torch.float64, device="cuda").requires_grad_()
+            for k, v in prm.items()})
+        for a, b in zip(got, ref):
+            assert a.shape == b.shape == (*shape, 4 if nlenses == 2 else 6, npts)
+            np.testing.assert_allclose(a.cpu().numpy(), b.detach().cpu().numpy(), atol=1e-9)
