@@ -824,12 +824,18 @@ constexpr int kExtMaxContours = 16;  // >= nlenses^2 + 1 closed rows + 3 stitche
 // ld_line_adj), so they return the same integral.
 // pq, xy, xq, yz hold 2 T doubles each: P and Q, the points' cotangents from the P and from
 // the Q lines, and the parts of the centroid's cotangent (Pbar dP/dy0, Qbar dQ/dx0).
-template <int NL, int DEG, bool VJP>
+// A workgroup takes every parts-th run of 256 neighbouring lines, from run `part` on, and with
+// parts = 1 the sums after them; SUMS: only those sums, the lines being done.  Without the
+// reverse mode P and Q do not depend on who forms them; its sums over a source's lines would, so
+// there parts is 1.
+template <int NL, int DEG, bool VJP, bool SUMS>
 __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* ct, int nc,
                                       int T, double* pq, double* xy, double* xq, double* yz,
                                       const LensFrame<NL>& lf, const LDSource<NL>& q,
-                                      const GLNodes& gl, LDAdj<NL>& adj, double* shd) {
+                                      const GLNodes& gl, LDAdj<NL>& adj, double* shd, int part,
+                                      int parts) {
     const int tid = threadIdx.x;
+    if constexpr (!SUMS) {
     // centroids (integrate.py:112); the closing point repeats c_0 in the sum
     for (int c = 0; c < nc; ++c) {
         const ExtCEntry& e = ct[c];
@@ -849,7 +855,7 @@ __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* 
     }
     __syncthreads();
     // the P lines of every point, then the Q lines, flat over the contours
-    for (int u = tid; u < 2 * T; u += kExtBlock) {
+    for (int u = tid + part * kExtBlock; u < 2 * T; u += parts * kExtBlock) {
         const bool isP = u < T;
         const int gi = isP ? u : u - T;
         int c = 0;
@@ -890,7 +896,9 @@ __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* 
             }
         }
     }
+    if (!VJP && parts > 1) return 0.0;
     __syncthreads();
+    }
     double total = 0.0;
     for (int c = 0; c < nc; ++c) {
         const ExtCEntry& e = ct[c];
@@ -971,6 +979,7 @@ namespace caus {
 #define CAUS_EXT_VJP_WAVES 3
 #endif
 
+constexpr int kExtMaxParts = 16;    // most workgroups of one source's line integrals
 constexpr int kExtPer = 4;          // initial limb angles per lane of k_ext_limb_init
 constexpr int kExtFlatBlock = 256;  // block of the flat kernels
 
@@ -2225,17 +2234,22 @@ __global__ __launch_bounds__(kExtBlock) void k_ext_contours(ExtArgs A, int buf) 
 
 // ---- contour integrals, magnification and its reverse mode (extended_source.py:
 // 860-901; integrate.py:18-121)
-template <int NL, bool LD, bool VJP>
+template <int NL, bool LD, bool VJP, bool SUMS = false>
 __global__ __launch_bounds__(kExtBlock)
 __attribute__((amdgpu_waves_per_eu(VJP ? CAUS_EXT_VJP_WAVES : 3)))
-void k_ext_integrate(ExtArgs A, int buf) {
+void k_ext_integrate(ExtArgs A, int buf, int maxparts, int per_part) {
     constexpr int DEG = ext_degree<NL>();
     constexpr int ND = ext_nd<NL>();
     __shared__ double s_d[8];
     __shared__ double2 s_gl[2 * kExtGL];
     const int tid = threadIdx.x;
-    const int64_t src = blockIdx.x;
+    // parts of one source are S workgroups apart, so that the first parts of the largest
+    // sources start first
+    const int64_t src = VJP ? blockIdx.x : blockIdx.x % A.S;
+    const int part = VJP ? 0 : (int)(blockIdx.x / A.S);
     const ExtBatch B = ext_batch(A);
+    const int parts = LD && !VJP ? min(maxparts, max(1, B.npts[src] / per_part)) : 1;
+    if (SUMS ? parts == 1 : part >= parts) return;
     if (B.npts[src] == 0) {   // skipped source: zero magnification and gradient
         if (tid == 0) {
             A.mag[src] = 0.0;
@@ -2254,7 +2268,7 @@ void k_ext_integrate(ExtArgs A, int buf) {
     const double u1 = LD ? A.u1[src * A.u1stride] : 0.0;
     ExtWS W = ext_ws(ext_source_base<DEG>(A, src), DEG, A.mmax);
     GLNodes g{};
-    if constexpr (LD) {
+    if constexpr (LD && !SUMS) {
         g.n1 = A.npts_ld / 2;
         g.n2 = A.npts_ld - g.n1;
         g.a = s_gl;
@@ -2314,9 +2328,9 @@ void k_ext_integrate(ExtArgs A, int buf) {
     if constexpr (LD) {
         // the append-order points (buffer 0) are not read any more: the Q lines' cotangents
         const LDSource<NL> q = ld_source<NL>(lf, w0, rho, u1);
-        total = integrate_source_ld<NL, DEG, VJP>(zb, thb, s_ct, nc, T, W.pq, W.xy,
-                                                  reinterpret_cast<double*>(W.z[buf ^ 1]), W.yz,
-                                                  lf, q, g, adj, s_d);
+        total = integrate_source_ld<NL, DEG, VJP, SUMS>(
+            zb, thb, s_ct, nc, T, W.pq, W.xy, reinterpret_cast<double*>(W.z[buf ^ 1]), W.yz, lf, q,
+            g, adj, s_d, part, parts);
     } else {
         for (int c = 0; c < nc; ++c) {
             const ExtCEntry& e = s_ct[c];
@@ -2325,6 +2339,7 @@ void k_ext_integrate(ExtArgs A, int buf) {
                 contour_adjoint<NL, DEG>(zb, thb, e.pc, e.np, e.L, e.nterms, lf, e.par, adj);
         }
     }
+    if (LD && !VJP && !SUMS && parts > 1) return;
     const unsigned long long npoints = (unsigned long long)T;
     const double m = fabs(total) / (kExtPi * rho * rho);
     if constexpr (VJP) {
@@ -2365,6 +2380,23 @@ bool ext_grouped(const ExtArgs& a) {
     constexpr int64_t tasks = 16000, sources = 1200;
     const int64_t share = a.npts ? (NL == 3 ? 2 : 4) : 1;
     return a.S <= sources && a.S * a.nadd_max <= tasks * share;
+}
+
+// Limb points per workgroup of a source's limb-darkened line integrals without the reverse mode
+// (a source of n takes n / that many workgroups; their sums follow in a second launch).  One
+// workgroup of four waves issues less than half of a CU's FP64 rate and needs 1.5 ms for a
+// source of 4096 points, so small batches are cut until they fill the 768 resident workgroups,
+// and batches of up to two fillings into parts of 256 points, so that the largest sources do not
+// outlast the rest.  Sources with sizes of their own or skipped ones count half.  One MI355X,
+// whole calls, one workgroup a source -> this: 20 binary epochs of 200 points 324 -> 276 us,
+// 500-epoch mag() event 485 -> 467 us, 1,300 epochs of 256-4096 points 3.1 -> 1.8 ms, three
+// lenses 5.3 -> 3.3 ms; 2,100 epochs of 256-1024 points 1.87 ms either way.  With the reverse
+// mode, sums that do not depend on the cut cost large batches 2-4%, so it is not cut.
+inline int ext_per_part(const ExtArgs& a) {
+    if (a.S > 2 * 768) return INT32_MAX;
+    const int64_t busy = a.npts ? a.S / 2 : a.S;
+    const int64_t fill = a.npts_def * busy / 768;
+    return (int)(fill < 32 ? 32 : (fill > 256 ? 256 : fill));
 }
 
 // the launch sequence for one batch of nlenses = NL
@@ -2423,7 +2455,15 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
     hipLaunchKernelGGL((k_ext_chain<NL, true>), dim3(nb), dim3(kExtBlock), 0, s, a, cur);  // final
     if constexpr (NL > 1)
         hipLaunchKernelGGL((k_ext_contours<NL>), dim3(nb), dim3(kExtBlock), 0, s, a, 1);
-    hipLaunchKernelGGL((k_ext_integrate<NL, LD, VJP>), dim3(nb), dim3(kExtBlock), 0, s, a, 1);
+    const int per_part = ext_per_part(a);
+    const int parts = LD && !VJP ? min(kExtMaxParts, max(1, a.npts_def / per_part)) : 1;
+    hipLaunchKernelGGL((k_ext_integrate<NL, LD, VJP>), dim3(nb * (unsigned)parts), dim3(kExtBlock),
+                       0, s, a, 1, parts, per_part);
+    if constexpr (LD && !VJP) {
+        if (parts > 1)
+            hipLaunchKernelGGL((k_ext_integrate<NL, LD, VJP, true>), dim3(nb), dim3(kExtBlock), 0,
+                               s, a, 1, parts, per_part);
+    }
     return hipGetLastError() == hipSuccess ? CAUS_OK : CAUS_ERR_LAUNCH;
 }
 
