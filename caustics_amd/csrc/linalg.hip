@@ -38,22 +38,59 @@ __device__ __forceinline__ double wave_sum64(double v) {
     return v;
 }
 
+// Where the segments lie: one matrix of magnifications cut at the offsets off (on the
+// device), or every segment by itself, so that slices of a larger tensor, and observations
+// kept per observatory, are read in place.
+struct LLMatrix {
+    const double* A;
+    int64_t n, lda;
+    const double *f, *c;
+    const int64_t* off;
+    double* gA;
+    int64_t ldg;
+};
+struct LLSegments {
+    const double* A[CAUS_LL_MAX_SEGMENTS];
+    int64_t lda[CAUS_LL_MAX_SEGMENTS], n[CAUS_LL_MAX_SEGMENTS];
+    const double *f[CAUS_LL_MAX_SEGMENTS], *c[CAUS_LL_MAX_SEGMENTS];
+    double* gA;     // (B, sum n), segment after segment
+    int64_t ldg;
+};
+struct LLSeg {
+    const double *a, *f, *c;
+    double* ga;
+    int64_t i0, i1;
+};
+__device__ __forceinline__ LLSeg ll_segment(const LLMatrix& m, int k, int64_t b, int64_t&) {
+    // segment bounds, clamped so that malformed offsets cannot leave [0, n)
+    const int64_t i0 = min(max(m.off[k], (int64_t)0), m.n);
+    const int64_t i1 = min(max(m.off[k + 1], i0), m.n);
+    return LLSeg{m.A + b * m.lda, m.f, m.c, m.gA ? m.gA + b * m.ldg : nullptr, i0, i1};
+}
+__device__ __forceinline__ LLSeg ll_segment(const LLSegments& m, int k, int64_t b, int64_t& at) {
+    LLSeg s{m.A[k] + b * m.lda[k], m.f[k], m.c[k], m.gA ? m.gA + b * m.ldg + at : nullptr, 0,
+            m.n[k]};
+    at += m.n[k];
+    return s;
+}
+
+template <class Where>
 __global__ __launch_bounds__(kLLBlock) void k_marginalized_ll(
-    const double* __restrict__ A, int64_t B, int64_t n, int64_t lda,
-    const double* __restrict__ f, const double* __restrict__ c, const int64_t* __restrict__ off,
-    int nseg, const double* __restrict__ g_ll, double* __restrict__ ll,
-    double* __restrict__ beta, double* __restrict__ gA, int64_t ldg) {
+    Where where, int64_t B, int nseg, const double* __restrict__ g_ll, double* __restrict__ ll,
+    double* __restrict__ beta) {
     const int lane = threadIdx.x & 63;
     const int64_t b = (int64_t)blockIdx.x * kLLCurves + (threadIdx.x >> 6);
     if (b >= B) return;  // whole waves leave; nothing below synchronises the block
-    const double* a = A + b * lda;
-    double* ga = gA ? gA + b * ldg : nullptr;
-    const double gb = gA ? (g_ll ? g_ll[b] : 1.0) : 0.0;
+    const double gb = where.gA ? (g_ll ? g_ll[b] : 1.0) : 0.0;
     double total = 0.0;
+    int64_t at = 0;
     for (int k = 0; k < nseg; ++k) {
-        // segment bounds, clamped so that malformed offsets cannot leave [0, n)
-        const int64_t i0 = min(max(off[k], (int64_t)0), n);
-        const int64_t i1 = min(max(off[k + 1], i0), n);
+        const LLSeg seg = ll_segment(where, k, b, at);
+        const double* __restrict__ a = seg.a;
+        const double* __restrict__ f = seg.f;
+        const double* __restrict__ c = seg.c;
+        double* __restrict__ ga = seg.ga;
+        const int64_t i0 = seg.i0, i1 = seg.i1;
         // the first 64 x kLLCache magnifications of the segment are read from HBM once,
         // every load of a lane issued together, and kept in registers for the three
         // passes; f and c are shared by all curves and come from cache; an epoch
@@ -146,7 +183,34 @@ extern "C" int caus_marginalized_log_likelihood(void* stream, const double* A, i
     if (B > (int64_t(1) << 26) || !A || !fobs || !c_inv || !seg_off || !ll) return CAUS_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
     const unsigned nb = (unsigned)((B + kLLCurves - 1) / kLLCurves);
-    hipLaunchKernelGGL(k_marginalized_ll, dim3(nb), dim3(kLLBlock), 0, s, A, B, n, lda, fobs,
-                       c_inv, seg_off, (int)nseg, g_ll, ll, beta, g_A, ldg);
+    const LLMatrix m{A, n, lda, fobs, c_inv, seg_off, g_A, ldg};
+    hipLaunchKernelGGL(k_marginalized_ll<LLMatrix>, dim3(nb), dim3(kLLBlock), 0, s, m, B,
+                       (int)nseg, g_ll, ll, beta);
+    return hipGetLastError() == hipSuccess ? CAUS_OK : CAUS_ERR_LAUNCH;
+}
+
+extern "C" int caus_marginalized_log_likelihood_segments(
+    void* stream, const double* const* A, const int64_t* lda, const double* const* fobs,
+    const double* const* c_inv, const int64_t* n, int32_t nseg, int64_t B, double* ll,
+    double* beta, const double* g_ll, double* g_A) {
+    if (B < 0 || nseg < 1 || nseg > CAUS_LL_MAX_SEGMENTS || !A || !lda || !fobs || !c_inv || !n)
+        return CAUS_ERR_ARG;
+    LLSegments m{};
+    for (int k = 0; k < nseg; ++k) {
+        if (n[k] < 0 || (B > 1 && lda[k] < 0) || (n[k] > 0 && (!A[k] || !fobs[k] || !c_inv[k])))
+            return CAUS_ERR_ARG;
+        m.A[k] = A[k];
+        m.lda[k] = lda[k];
+        m.n[k] = n[k];
+        m.f[k] = fobs[k];
+        m.c[k] = c_inv[k];
+        m.ldg += n[k];
+    }
+    m.gA = g_A;
+    if (B == 0) return CAUS_OK;
+    if (B > (int64_t(1) << 26) || !ll) return CAUS_ERR_ARG;
+    const unsigned nb = (unsigned)((B + kLLCurves - 1) / kLLCurves);
+    hipLaunchKernelGGL(k_marginalized_ll<LLSegments>, dim3(nb), dim3(kLLBlock), 0,
+                       (hipStream_t)stream, m, B, (int)nseg, g_ll, ll, beta);
     return hipGetLastError() == hipSuccess ? CAUS_OK : CAUS_ERR_LAUNCH;
 }

@@ -9,14 +9,17 @@ set and the summed log-likelihood.  Magnification vectors may also carry a leadi
 batch dimension B (one row per parameter set, e.g. the chains of an HMC run): then every
 beta is (B, 2) and ll is (B,).
 
-One HIP kernel (``caus_marginalized_log_likelihood``) computes ll, beta and, in the
-backward pass, d ll / d A; the gradient then flows into whatever produced A (e.g. the
-fused light-curve VJP of ``mag_point_source_lightcurve``).  Gradients flow to A only:
+One HIP kernel computes ll, beta and, where a gradient is needed, d ll / d A; it reads up to
+``MAX_SEGMENTS`` sets where they lie (``caus_marginalized_log_likelihood_segments``) and more of
+them from one matrix (``caus_marginalized_log_likelihood``).  The gradient then flows into
+whatever produced A (e.g. ``mag_point_source_lightcurve``).  Gradients flow to A only:
 the observations are data.  The reference's dense-covariance branch does not run
 (linalg.py:80 calls ``jnp.linals``, :84 uses an undefined ``M``), so
 ``dense_covariance=True`` raises.  ``Lam_sd`` belongs to that branch and is unused, as
 in the reference.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -54,6 +57,41 @@ class _MargLL(torch.autograd.Function):
         return gA, None, None, None, None
 
 
+MAX_SEGMENTS = 8   # CAUS_LL_MAX_SEGMENTS
+
+
+class _MargLLSegments(torch.autograd.Function):
+    """Segments read in place.  Where a gradient is needed the forward keeps d ll / d A, (B, sum
+    n), and the backward scales it."""
+
+    @staticmethod
+    def forward(ctx, need, fs, cs, *As):
+        n = len(As)
+        As = [a if a.shape[1] < 2 or a.stride(1) == 1 else a.contiguous() for a in As]
+        B, lens = As[0].shape[0], [a.shape[1] for a in As]
+        ll = torch.empty(B, dtype=torch.float64, device=As[0].device)
+        beta = torch.empty((B, n, 2), dtype=torch.float64, device=As[0].device)
+        gA = torch.empty((B, sum(lens)), dtype=torch.float64, device=ll.device) if need else None
+        ptrs = lambda xs: (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs])  # noqa: E731
+        rc = _lib.lib().caus_marginalized_log_likelihood_segments(
+            _lib.stream_ptr(), ptrs(As), (ctypes.c_int64 * n)(*[a.stride(0) for a in As]),
+            ptrs(fs), ptrs(cs), (ctypes.c_int64 * n)(*lens), n, B, _lib.ptr(ll), _lib.ptr(beta),
+            None, _lib.ptr(gA))
+        _lib.check(rc, "caus_marginalized_log_likelihood_segments")
+        if need:
+            ctx.save_for_backward(gA)
+        ctx.lens = lens
+        ctx.mark_non_differentiable(beta)
+        return ll, beta
+
+    @staticmethod
+    def backward(ctx, g_ll, _g_beta):
+        (gA,) = ctx.saved_tensors
+        with torch.no_grad():
+            g = g_ll.to(torch.float64)[:, None] * gA
+        return (None, None, None, *g.split(ctx.lens, 1))
+
+
 def _f64(x, device):
     if torch.is_tensor(x):
         return x.to(device=device, dtype=torch.float64).contiguous()
@@ -83,12 +121,16 @@ def marginalized_log_likelihood(A_list, fobs_list, C_inv_list, dense_covariance=
     lens = [a.shape[1] for a in As]
     if [f.numel() for f in fs] != lens or [c.numel() for c in cs] != lens:
         raise ValueError("each fobs / C_inv must have the length of its magnification array")
-    A = torch.cat(As, 1).contiguous()
-    fobs = torch.cat(fs)
-    c_inv = torch.cat(cs)
-    off = torch.tensor([0] + list(torch.tensor(lens).cumsum(0).tolist()), dtype=torch.int64,
-                       device=dev)
-    ll, beta = _MargLL.apply(A, fobs, c_inv, off, len(As))
+    if len(As) <= MAX_SEGMENTS:
+        need = torch.is_grad_enabled() and any(a.requires_grad for a in As)
+        ll, beta = _MargLLSegments.apply(need, fs, cs, *As)
+    else:
+        A = torch.cat(As, 1).contiguous()
+        fobs = torch.cat(fs)
+        c_inv = torch.cat(cs)
+        off = torch.tensor([0] + list(torch.tensor(lens).cumsum(0).tolist()), dtype=torch.int64,
+                           device=dev)
+        ll, beta = _MargLL.apply(A, fobs, c_inv, off, len(As))
     if batched:
         return [beta[:, k] for k in range(len(As))], ll
     return [beta[0, k] for k in range(len(As))], ll[0]

@@ -331,6 +331,15 @@ int caus_marginalized_log_likelihood(void* stream, const double* A, int64_t B, i
                                      const int64_t* seg_off, int32_t nseg, double* ll,
                                      double* beta, const double* g_ll, double* g_A, int64_t ldg);
 
+/* The same with every segment where it lies (at most CAUS_LL_MAX_SEGMENTS of them; host arrays
+ * of nseg entries): magnifications A[k] (B, n[k]) with row stride lda[k], observations fobs[k]
+ * and c_inv[k] (n[k],).  g_A (B, sum n) or NULL: segment after segment. */
+#define CAUS_LL_MAX_SEGMENTS 8
+int caus_marginalized_log_likelihood_segments(
+    void* stream, const double* const* A, const int64_t* lda, const double* const* fobs,
+    const double* const* c_inv, const int64_t* n, int32_t nseg, int64_t B, double* ll,
+    double* beta, const double* g_ll, double* g_A);
+
 /* Source trajectories with annual parallax, and their reverse mode.
  * Replaces AnnualParallaxTrajectory.compute and _compute_delta_sun_position_and_velocity
  * (src/caustics/trajectory.py:104-157), for L parameter sets at once.

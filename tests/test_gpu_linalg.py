@@ -168,3 +168,31 @@ def test_autograd_api_and_lightcurve_chain():
         fd = (ll_of(dict(p1, **{k: p1[k] + h})) - ll_of(dict(p1, **{k: p1[k] - h}))) / (2 * h)
         print(f"{k}: autograd {gr[k]:.6e} fd {fd:.6e}")
         assert gr[k] == pytest.approx(fd, rel=1e-5, abs=1e-6 * max(abs(v) for v in gr.values()))
+
+
+# one segment, sizes around the 1024 magnifications that a wave keeps in registers, the most
+# segments read in place and one more
+@pytest.mark.parametrize("lens", [[700], [1023, 1025], [1024, 3, 2000], [40] * 8, [40] * 9])
+@pytest.mark.parametrize("B", [1, 5])
+def test_segments_in_place_match_matrix(lens, B):
+    """Slices of a larger tensor (other row strides, a column stride) give the bits of one
+    contiguous matrix, and the kept gradient scaled afterwards that of the cotangent inside the
+    kernel up to the rounding of the two products."""
+    from caustics_amd import marginalized_log_likelihood
+    g = np.random.default_rng(sum(lens) + B)
+    A, f, c, off = _curves(g, B, lens)
+    g_ll = g.uniform(0.5, 2.0, B)
+    ll, beta, gA = _kernel(A, f, c, off, g_ll=g_ll)
+    wide = torch.zeros((B, sum(lens) + 7), dtype=torch.float64, device="cuda")
+    wide[:, 3:-4] = torch.as_tensor(A, device="cuda")
+    wide.requires_grad_()
+    As = [wide[:, 3 + off[k]:3 + off[k + 1]] for k in range(len(lens))]
+    As[-1] = As[-1].t().contiguous().t()   # column after column
+    b1, l1 = marginalized_log_likelihood(As, [f[off[k]:off[k + 1]] for k in range(len(lens))],
+                                         [c[off[k]:off[k + 1]] for k in range(len(lens))])
+    np.testing.assert_array_equal(l1.detach().cpu().numpy(), ll)
+    np.testing.assert_array_equal(torch.stack(b1, 1).cpu().numpy(), beta)
+    (gw,) = torch.autograd.grad(l1, wide, torch.as_tensor(g_ll, device="cuda"))
+    gw = gw.cpu().numpy()
+    np.testing.assert_allclose(gw[:, 3:-4], gA, rtol=4 * np.finfo(float).eps)
+    assert not gw[:, :3].any() and not gw[:, -4:].any()
