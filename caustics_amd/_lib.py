@@ -136,7 +136,19 @@ def side_streams(n=2):
 
 
 def stream_ptr(device=None):
+    # the raw handle without a Stream object: 0.7 against 2.9 us, and each entry point asks once
+    # a call
+    if device is None:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+def on_device(x, dtype):
+    """Tensor x in dtype on the current device (x.to(device="cuda", dtype=dtype), without its
+    1 us where x is that already)."""
+    if x.dtype is dtype and x.is_cuda and x.get_device() == torch.cuda.current_device():
+        return x
+    return x.to(device="cuda", dtype=dtype)
 
 
 def ptr(t):

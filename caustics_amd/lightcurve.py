@@ -108,8 +108,9 @@ def mag_point_source_lightcurve(t, t0, u0, tE, alpha, nlenses=2, roots_itmax=250
     parameter (not in t)."""
     names = TRAJ_NAMES + PARAM_NAMES[nlenses]
     vals = dict(t0=t0, u0=u0, tE=tE, alpha=alpha, **params)
-    cols = [torch.as_tensor(np.asarray(vals[n]) if not isinstance(vals[n], torch.Tensor)
-                            else vals[n], device="cuda").to(torch.float64) for n in names]
+    cols = [_lib.on_device(vals[n], torch.float64) if isinstance(vals[n], torch.Tensor)
+            else torch.as_tensor(np.asarray(vals[n]), device="cuda").to(torch.float64)
+            for n in names]
     t = torch.as_tensor(t, device="cuda", dtype=torch.float64).contiguous().reshape(-1)
     need = torch.is_grad_enabled() and any(c.requires_grad for c in cols)
     return _LightCurve.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode), need,

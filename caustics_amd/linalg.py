@@ -94,7 +94,7 @@ class _MargLLSegments(torch.autograd.Function):
 
 def _f64(x, device):
     if torch.is_tensor(x):
-        return x.to(device=device, dtype=torch.float64).contiguous()
+        return _lib.on_device(x, torch.float64).contiguous()
     return torch.as_tensor(np.asarray(x, np.float64), device=device).contiguous()
 
 
@@ -112,7 +112,7 @@ def marginalized_log_likelihood(A_list, fobs_list, C_inv_list, dense_covariance=
     batched = As[0].dim() == 2
     if any((a.dim() == 2) != batched for a in As):
         raise ValueError("all magnification arrays must be 1-D, or all (B, n_k)")
-    As = [(a if batched else a.reshape(1, -1)).to(dev, torch.float64) for a in As]
+    As = [_lib.on_device(a if batched else a.reshape(1, -1), torch.float64) for a in As]
     B = As[0].shape[0]
     if any(a.shape[0] != B for a in As):
         raise ValueError("batched magnification arrays must share the leading dimension")

@@ -53,12 +53,12 @@ def _prepare(w, nlenses, params):
     w = _tensor(w)
     if not w.is_complex():
         w = w.to(torch.float64)
-    w = w.to(device="cuda", dtype=torch.complex128)
+    w = _lib.on_device(w, torch.complex128)
     names = PARAM_NAMES[nlenses]
     missing = [n for n in names if n not in params]
     if missing:
         raise ValueError(f"nlenses={nlenses} needs parameters {names}; missing {missing}")
-    ps = [_tensor(params[n]).to(device="cuda", dtype=torch.float64) for n in names]
+    ps = [_lib.on_device(_tensor(params[n]), torch.float64) for n in names]
     return w, ps
 
 

@@ -127,7 +127,7 @@ class AnnualParallaxTrajectory:
             raise ValueError(f"missing parameters {missing}")
         vals = [v if torch.is_tensor(v) else torch.as_tensor(np.asarray(v, np.float64))
                 for v in (params[k] for k in names)]
-        vals = [v.to(device="cuda", dtype=torch.float64).reshape(-1) for v in vals]
+        vals = [_lib.on_device(v, torch.float64).reshape(-1) for v in vals]
         L = max(v.numel() for v in vals)
         if any(v.numel() not in (1, L) for v in vals):
             raise ValueError("parameter arrays must share one length")
@@ -136,6 +136,6 @@ class AnnualParallaxTrajectory:
         P = torch.stack([v.expand(L) for v in vals], -1).contiguous()
         tt = t if torch.is_tensor(t) else torch.as_tensor(np.asarray(t, np.float64))
         shape = tuple(tt.shape)
-        tt = tt.to(device="cuda", dtype=torch.float64).reshape(-1).contiguous()
+        tt = _lib.on_device(tt, torch.float64).reshape(-1).contiguous()
         w = _Parallax.apply(P, tt, self._xp, self._tab, 1 if parametrization == "polar" else 0)
         return w.reshape((L,) + shape) if batched else w.reshape(shape)
