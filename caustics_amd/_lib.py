@@ -143,12 +143,20 @@ def stream_ptr(device=None):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def resolved(x):
+    """x as its memory has to hold it for a kernel: torch negates and conjugates views lazily
+    (z.conj().imag, w.conj()) by a flag on the tensor, which no pointer shows."""
+    if x.is_conj():
+        x = x.resolve_conj()
+    return x.resolve_neg() if x.is_neg() else x
+
+
 def on_device(x, dtype):
-    """Tensor x in dtype on the current device (x.to(device="cuda", dtype=dtype), without its
-    1 us where x is that already)."""
+    """Tensor x in dtype on the current device, resolved (x.to(device="cuda", dtype=dtype),
+    without its 1 us where x is that already)."""
     if x.dtype is dtype and x.is_cuda and x.get_device() == torch.cuda.current_device():
-        return x
-    return x.to(device="cuda", dtype=dtype)
+        return resolved(x)
+    return resolved(x.to(device="cuda", dtype=dtype))
 
 
 def ptr(t):

@@ -31,8 +31,7 @@ def _as_cuda_c128(x):
         t = torch.as_tensor(np.asarray(x))
     if not t.is_complex():
         t = t.to(torch.float64)
-    t = t.to(device="cuda", dtype=torch.complex128)
-    return t.contiguous()
+    return _lib.on_device(t, torch.complex128).contiguous()
 
 
 def _resolve_mode(compensated, mode):
@@ -69,7 +68,7 @@ class _RootsFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_roots, _g_status):
         coeffs_asc, roots = ctx.saved_tensors
-        g = g_roots.contiguous().to(torch.complex128)
+        g = _lib.resolved(g_roots.to(torch.complex128)).contiguous()
         gc = torch.empty_like(coeffs_asc)
         N, n1 = coeffs_asc.shape
         rc = _lib.lib().caus_roots_vjp(_lib.stream_ptr(), _lib.ptr(coeffs_asc), _lib.ptr(roots),

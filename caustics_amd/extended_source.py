@@ -33,7 +33,7 @@ def extended_workspace_bytes(nlenses, nsources, npts_max):
 
 def _col(x, n, dtype=torch.float64):
     t = x if isinstance(x, torch.Tensor) else torch.as_tensor(np.asarray(x))
-    t = t.to(device="cuda", dtype=dtype).reshape(-1)
+    t = _lib.on_device(t, dtype).reshape(-1)
     if t.numel() == 1:
         t = t.expand(n)
     if t.numel() != n:
@@ -223,7 +223,7 @@ def mag_extended_source(w0, rho, nlenses=2, npts_limb=150, limb_darkening=False,
     mode_id = _mode_id(roots_compensated, mode)
     w = w0 if isinstance(w0, torch.Tensor) else torch.as_tensor(np.asarray(w0))
     shape = tuple(w.shape)
-    w = w.to(device="cuda", dtype=torch.complex128).reshape(-1).contiguous()
+    w = _lib.on_device(w, torch.complex128).reshape(-1).contiguous()
     S = w.numel()
     names = PARAM_NAMES[nlenses]
     rho_t = _col(rho, S)
@@ -243,7 +243,7 @@ def extended_fwd_vjp(w0, rho, g_mag, nlenses=2, npts_limb=150, limb_darkening=Fa
     """Fused forward + VJP: (mag (S,), g_params (S, 4+P), status (S,)); g_params columns
     are Re w0, Im w0, rho, u1 and the lens parameters."""
     w = torch.as_tensor(np.asarray(w0)) if not isinstance(w0, torch.Tensor) else w0
-    w = w.to(device="cuda", dtype=torch.complex128).reshape(-1).contiguous()
+    w = _lib.on_device(w, torch.complex128).reshape(-1).contiguous()
     S = w.numel()
     names = PARAM_NAMES[nlenses]
     prm = torch.stack([_col(params[k], S) for k in names], -1).contiguous() if names else None

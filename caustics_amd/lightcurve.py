@@ -47,10 +47,9 @@ def lightcurve_fwd_vjp(t, lc_params, g_mag, nlenses=2, roots_itmax=2500, mode="f
                        return_status=False):
     """Fused forward + VJP.  t (T,), lc_params (L, 4+P) rows (t0, u0, tE, alpha, lens
     params...), g_mag (L, T) -> (mag (L, T), g_params (L, 4+P)[, status (L, T)])."""
-    t = torch.as_tensor(t, device="cuda", dtype=torch.float64).contiguous()
-    lcp = torch.as_tensor(lc_params, device="cuda", dtype=torch.float64).contiguous()
-    g = None if g_mag is None else torch.as_tensor(g_mag, device="cuda",
-                                                   dtype=torch.float64).contiguous()
+    f64 = lambda x: _lib.resolved(torch.as_tensor(x, device="cuda",  # noqa: E731
+                                                  dtype=torch.float64)).contiguous()
+    t, lcp, g = f64(t), f64(lc_params), None if g_mag is None else f64(g_mag)
     mag, gp, st = _call(t, lcp, g, nlenses, int(roots_itmax), _lib.MODES[mode], return_status)
     return (mag, gp, st) if return_status else (mag, gp)
 
@@ -83,7 +82,7 @@ class _LightCurve(torch.autograd.Function):
     def backward(ctx, g):
         t, jac, *lcp = ctx.saved_tensors
         nlenses, itmax, mode, L, shapes = ctx.meta
-        g = g.contiguous().to(torch.float64)
+        g = _lib.resolved(g.contiguous().to(torch.float64))
         if jac is not None:
             _, gp = jacobian_vjp(jac, 0, max(t.numel(), 1), g, False, True)
         else:
@@ -111,7 +110,8 @@ def mag_point_source_lightcurve(t, t0, u0, tE, alpha, nlenses=2, roots_itmax=250
     cols = [_lib.on_device(vals[n], torch.float64) if isinstance(vals[n], torch.Tensor)
             else torch.as_tensor(np.asarray(vals[n]), device="cuda").to(torch.float64)
             for n in names]
-    t = torch.as_tensor(t, device="cuda", dtype=torch.float64).contiguous().reshape(-1)
+    t = _lib.resolved(torch.as_tensor(t, device="cuda", dtype=torch.float64))
+    t = t.contiguous().reshape(-1)
     need = torch.is_grad_enabled() and any(c.requires_grad for c in cols)
     return _LightCurve.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode), need,
                              t, *cols)
@@ -125,7 +125,7 @@ def hexadecapole_gate(w_points, rho, nlenses=2, u1=0.0, roots_itmax=2500, **para
 
     w = w_points if isinstance(w_points, torch.Tensor) else torch.as_tensor(np.asarray(w_points))
     shape = tuple(w.shape)
-    w = w.to(device="cuda", dtype=torch.complex128).reshape(-1).contiguous()
+    w = _lib.on_device(w, torch.complex128).reshape(-1).contiguous()
     P = w.numel()
     rho_t = _col(rho, P)
     names = PARAM_NAMES[nlenses]
@@ -148,7 +148,7 @@ def hexadecapole_vjp(w_points, rho, g_mu, nlenses=2, u1=0.0, roots_itmax=2500, *
     from .extended_source import _col
 
     w = w_points if isinstance(w_points, torch.Tensor) else torch.as_tensor(np.asarray(w_points))
-    w = w.to(device="cuda", dtype=torch.complex128).reshape(-1).contiguous()
+    w = _lib.on_device(w, torch.complex128).reshape(-1).contiguous()
     P = w.numel()
     names = PARAM_NAMES[nlenses]
     prm = torch.stack([_col(params[k], P) for k in names], -1).contiguous() if names else None
@@ -234,7 +234,7 @@ def _mag_args(w_points, rho, nlenses, npts_limb, limb_darkening, u1, npts_ld, ro
         raise ValueError("`nlenses` has to be set to be <= 3.")
     w = w_points if isinstance(w_points, torch.Tensor) else torch.as_tensor(np.asarray(w_points))
     shape = tuple(w.shape)
-    w = w.to(device="cuda", dtype=torch.complex128).reshape(-1).contiguous()
+    w = _lib.on_device(w, torch.complex128).reshape(-1).contiguous()
     P = w.numel()
     names = PARAM_NAMES[nlenses]
     cfg = (nlenses, _host_npts(npts_limb, P), int(np.max(npts_limb)), bool(limb_darkening),

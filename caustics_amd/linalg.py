@@ -53,7 +53,8 @@ class _MargLL(torch.autograd.Function):
     def backward(ctx, g_ll, _g_beta):
         A, fobs, c_inv, off = ctx.saved_tensors
         _, _, gA = _call(A, fobs, c_inv, off, ctx.nseg,
-                         g_ll=g_ll.contiguous().to(torch.float64), want_grad=True)
+                         g_ll=_lib.resolved(g_ll.contiguous().to(torch.float64)),
+                         want_grad=True)
         return gA, None, None, None, None
 
 

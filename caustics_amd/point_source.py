@@ -141,7 +141,7 @@ class _MagPointSource(torch.autograd.Function):
         P = len(pshapes)
         N = wf.numel()
         want_w, want_p = ctx.needs_input_grad[4], any(ctx.needs_input_grad[5:])
-        gf = g.expand(shape).contiguous().reshape(-1).to(torch.float64)
+        gf = _lib.resolved(g.expand(shape).contiguous().reshape(-1).to(torch.float64))
         if jac is not None:
             g_w, g_p = jacobian_vjp(jac, 2, per, gf, want_w, want_p)
             pshape = shape if per == 1 else None   # summed over the rows already
@@ -234,7 +234,7 @@ def _images(w, nlenses, itmax, mode, z_init, sequential, params):
     status = torch.empty((B, N), dtype=torch.uint8, device="cuda")
     zi = None
     if z_init is not None:
-        zi = (z_init.to(device="cuda", dtype=torch.complex128) if torch.is_tensor(z_init)
+        zi = (_lib.on_device(z_init, torch.complex128) if torch.is_tensor(z_init)
               else torch.as_tensor(np.asarray(z_init, np.complex128), device="cuda"))
         zi = zi.reshape(n, B, N).permute(1, 2, 0).contiguous()
     # independent positions: one lens row per position, addressed as B*N sequences of 1
@@ -255,7 +255,7 @@ def images_point_source(w, nlenses=2, roots_itmax=2500, roots_compensated=False,
     (n, *w.shape) starts the solver from those roots (point_source.py:1652-1709)."""
     if nlenses not in (1, 2, 3):
         raise ValueError("`nlenses` has to be set to be <= 3.")
-    w = (w.to(device="cuda", dtype=torch.complex128) if torch.is_tensor(w)
+    w = (_lib.on_device(w, torch.complex128) if torch.is_tensor(w)
          else torch.as_tensor(np.asarray(w, np.complex128), device="cuda"))
     shape = w.shape
     wf = w.reshape(1, -1).contiguous()
@@ -275,7 +275,7 @@ def images_point_source_sequential(w, nlenses=2, roots_itmax=2500, roots_compens
     parameters of shape (B,) or scalars, and returns (B, n, N)."""
     if nlenses not in (1, 2, 3):
         raise ValueError("`nlenses` has to be set to be <= 3.")
-    w = (w.to(device="cuda", dtype=torch.complex128) if torch.is_tensor(w)
+    w = (_lib.on_device(w, torch.complex128) if torch.is_tensor(w)
          else torch.as_tensor(np.asarray(w, np.complex128), device="cuda"))
     one = w.dim() == 1
     w2 = (w.reshape(1, -1) if one else w).contiguous()
@@ -362,7 +362,8 @@ def critical_and_caustic_curves(npts=200, nlenses=2, **params):
             (params[k] for k in names)]
     batch = vals[0].ndim > 0
     cols = [None if isinstance(v, np.ndarray) and v.ndim == 0 else
-            torch.as_tensor(v, device="cuda").to(torch.float64).reshape(-1) for v in vals]
+            _lib.resolved(torch.as_tensor(v, device="cuda").to(torch.float64)).reshape(-1)
+            for v in vals]
     B = torch.broadcast_shapes(*[(1,) if c is None else c.shape for c in cols])[0]
     P = len(cols)
     n = _DEGREE_CRITICAL[nlenses]

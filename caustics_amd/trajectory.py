@@ -77,7 +77,7 @@ class _Parallax(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_w):
         P, t, xp, tab = ctx.saved_tensors
-        g = g_w.to(torch.complex128).contiguous()
+        g = _lib.resolved(g_w.to(torch.complex128)).contiguous()
         gP = torch.empty_like(P)
         rc = _lib.lib().caus_trajectory_annual_parallax(
             _lib.stream_ptr(), _lib.ptr(t), t.numel(), _lib.ptr(xp), _lib.ptr(tab), xp.numel(),

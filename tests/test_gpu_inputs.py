@@ -1,0 +1,131 @@
+"""Inputs as torch hands them over: views whose negation or conjugation is only a flag on the
+tensor."""
+import numpy as np
+import pytest
+import torch
+
+import caustics_amd as ca
+from caustics_amd.linalg import marginalized_log_likelihood
+
+pytestmark = pytest.mark.gpu
+
+B3 = dict(s=0.9, q=0.4, q3=0.3, r3=0.8, psi=0.7)
+
+
+def neg(x, dense=False):
+    """x as a view that torch negates on reading: its memory holds -x."""
+    x = torch.as_tensor(x, dtype=torch.float64, device="cuda")
+    v = torch._neg_view(-x) if dense else torch.complex(torch.zeros_like(x), -x).conj().imag
+    assert v.is_neg() and torch.equal(v.resolve_neg(), x)
+    return v
+
+
+def conj(z):
+    """z as a view that torch conjugates on reading."""
+    z = torch.as_tensor(z, dtype=torch.complex128, device="cuda")
+    v = z.conj().resolve_conj().conj()
+    assert v.is_conj() and torch.equal(v.resolve_conj(), z)
+    return v
+
+
+def plain(v):
+    return v.resolve_conj().resolve_neg() if torch.is_tensor(v) else v
+
+
+def _positions(n, seed=0):
+    r = np.random.default_rng(seed)
+    return r.uniform(-0.5, 0.5, n) + 1j * r.uniform(-0.5, 0.5, n)
+
+
+def _obs(n, seed=0):
+    r = np.random.default_rng(seed)
+    t = torch.as_tensor(r.uniform(1.0, 3.0, n), device="cuda")
+    return 2.0 * t + 0.3 + 0.01 * torch.as_tensor(r.normal(size=n), device="cuda"), \
+        torch.full((n,), 1e4, dtype=torch.float64, device="cuda"), t
+
+
+def _coeffs(n, seed=0):
+    r = np.random.default_rng(seed)
+    return r.normal(size=(n, 6)) + 1j * r.normal(size=(n, 6))
+
+
+W = _positions(7)
+T = np.linspace(-1.0, 1.0, 5)
+ORBIT = np.stack([np.cos(np.arange(101) / 58.0), np.sin(np.arange(101) / 58.0),
+                  0.1 * np.ones(101)], 1)
+
+# entry point on arguments, arguments with flagged views among them
+CALLS = {
+    "point_source_one": (lambda w, s, q: ca.mag_point_source(w, s=s, q=q),
+                         lambda: (conj(W), neg([0.9]), neg(0.4))),
+    "point_source_rows": (lambda w, s, q: ca.mag_point_source(w, s=s, q=q),
+                          lambda: (W, neg(np.linspace(0.8, 1.2, 7)), neg(np.linspace(0.1, 0.5, 7)))),
+    "point_source_triple": (lambda w, psi: ca.mag_point_source(w, nlenses=3, **{**B3, "psi": psi}),
+                            lambda: (W, neg([0.7]))),
+    "lightcurve": (lambda u0, al: ca.mag_point_source_lightcurve(T, 0.0, u0, 1.0, al, s=0.9, q=0.4),
+                   lambda: (neg([0.1, 0.2, 0.3]), neg([0.6]))),
+    "lightcurve_one": (lambda t, u0: ca.mag_point_source_lightcurve(t, 0.0, u0, 1.0, 0.6, s=0.9,
+                                                                    q=0.4),
+                       lambda: (neg([0.3]), neg([0.1]))),
+    "curves": (lambda s, q: torch.stack(ca.critical_and_caustic_curves(npts=20, s=s, q=q)),
+               lambda: (neg([0.9, 1.1]), neg([0.4]))),
+    "curves_triple": (lambda psi: torch.stack(
+        ca.critical_and_caustic_curves(npts=20, nlenses=3, **{**B3, "psi": psi})),
+        lambda: (neg(0.7),)),
+    "likelihood": (lambda a, f, c: marginalized_log_likelihood([a], [f], [c])[1],
+                   lambda: [neg(x.tolist(), dense=True) for x in
+                            (torch.stack([_obs(9, 1)[2], _obs(9)[2]]), *_obs(9)[:2])]),
+    "extended": (lambda w, rho, u1: ca.mag_extended_source(w, rho, s=0.9, q=0.4, u1=u1, npts_ld=10,
+                                                           npts_limb=60, limb_darkening=True),
+                 lambda: (conj(W), neg(np.full(7, 0.01)), neg([0.3]))),
+    "mag": (lambda w, rho: ca.mag(w, rho, s=0.9, q=0.4, npts_limb=60),
+            lambda: (conj(W), neg([0.01]))),
+    "roots": (lambda c, z: ca.ehrlich_aberth(c, z, custom_init=True),
+              lambda: (conj(_coeffs(3)), conj(_coeffs(3, 1)[:, :5]))),
+    "images": (lambda w: ca.images_point_source(w, a=0.45, e1=0.7)[0], lambda: (conj(W),)),
+    "images_sequential": (lambda w: ca.images_point_source_sequential(w, a=0.45, e1=0.7)[0],
+                          lambda: (conj(W),)),
+    "trajectory": (lambda t, u0: ca.AnnualParallaxTrajectory(
+        np.array([0.0, 100.0]), (1.0, 0.2), earth_pos=ORBIT, earth_vel=ORBIT[::-1]).compute(
+            t, t0=40.0, u0=u0, tE=20.0, piEE=0.1, piEN=0.2), lambda: (neg([30.0]), neg([0.1]))),
+}
+
+
+@pytest.mark.parametrize("name", list(CALLS))
+def test_flagged_views_are_read_as_their_values(gpu, name):
+    call, args = CALLS[name]
+    a = args()
+    assert torch.equal(plain(call(*a)), plain(call(*[plain(x) for x in a])))
+
+
+def test_gradients_through_flagged_views(gpu):
+    """Gradients of parameters that reach the entry points as flagged views."""
+    def run(flagged):
+        x = torch.tensor([0.9, 0.4, 0.1], dtype=torch.float64, device="cuda", requires_grad=True)
+        y = torch.complex(torch.zeros_like(x), -x).conj().imag if flagged else x
+        assert y.is_neg() == flagged
+        s, q, u0 = y[:1], y[1:2], y[2:]
+        m = ca.mag_point_source(W, s=s, q=q)
+        lc = ca.mag_point_source_lightcurve(T, 0.0, u0, 1.0, 0.6, s=s, q=q)
+        return torch.autograd.grad((m * m).sum() + (lc * lc).sum(), x)[0]
+
+    torch.testing.assert_close(run(True), run(False), rtol=1e-14, atol=0.0)
+
+
+def test_cotangents_as_flagged_views(gpu):
+    """A backward pass called with a flagged cotangent."""
+    w = torch.as_tensor(W[:1], device="cuda")
+    s = torch.tensor([0.9], dtype=torch.float64, device="cuda", requires_grad=True)
+    m = [ca.mag_point_source(w, s=s, q=0.4),
+         ca.mag_point_source_lightcurve(T[:1], 0.0, 0.1, 1.0, 0.6, s=s, q=0.4)]
+    for o in m:
+        g = neg(np.full(tuple(o.shape), 0.7))
+        a, = torch.autograd.grad(o, s, g, retain_graph=True)
+        b, = torch.autograd.grad(o, s, plain(g), retain_graph=True)
+        assert torch.equal(plain(a), plain(b))
+    c = torch.as_tensor(_coeffs(2), device="cuda").requires_grad_()
+    r = ca.ehrlich_aberth(c)
+    g = conj(_coeffs(2, 3)[:, :5].reshape(-1))
+    a, = torch.autograd.grad(r, c, g, retain_graph=True)
+    b, = torch.autograd.grad(r, c, plain(g))
+    assert torch.equal(plain(a), plain(b))
