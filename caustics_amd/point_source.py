@@ -354,8 +354,7 @@ def critical_and_caustic_curves(npts=200, nlenses=2, **params):
     if nlenses == 1:
         return torch.exp(-1j * phi), torch.zeros(npts, dtype=torch.complex128, device="cuda")
     names = PARAM_NAMES[nlenses]
-    if torch.is_grad_enabled() and any(isinstance(params[k], torch.Tensor)
-                                       and params[k].requires_grad for k in names):
+    if any(isinstance(params[k], torch.Tensor) and _differentiated(params[k]) for k in names):
         return _curves_tensor(phi, nlenses, [params[k] for k in names])
     # numbers go to the kernels by value
     vals = [v if isinstance(v, torch.Tensor) else np.asarray(v) for v in
@@ -385,9 +384,16 @@ def critical_and_caustic_curves(npts=200, nlenses=2, **params):
 _DEGREE_CRITICAL = {2: 4, 3: 6}
 
 
+def _differentiated(x):
+    """Whether a derivative with respect to x is recorded, or x carries a forward-mode tangent
+    (which the root solver refuses; a kernel would drop it)."""
+    return ((torch.is_grad_enabled() and x.requires_grad)
+            or torch.autograd.forward_ad.unpack_dual(x).tangent is not None)
+
+
 def _curves_tensor(phi, nlenses, params):
     """critical_and_caustic_curves as tensor expressions around the root solver and the
-    continuation, for parameters that require a gradient (it flows through the explicit
+    continuation, for differentiated parameters (a gradient flows through the explicit
     dependence of the map and the shift on them)."""
     from .ehrlich_aberth_primitive import poly_roots
 

@@ -1,5 +1,5 @@
 """Inputs as torch hands them over: views whose negation or conjugation is only a flag on the
-tensor."""
+tensor, forward-mode duals."""
 import numpy as np
 import pytest
 import torch
@@ -129,3 +129,24 @@ def test_cotangents_as_flagged_views(gpu):
     a, = torch.autograd.grad(r, c, g, retain_graph=True)
     b, = torch.autograd.grad(r, c, plain(g))
     assert torch.equal(plain(a), plain(b))
+
+
+# ---- forward-mode duals -----------------------------------------------------------------
+def _dual(x):
+    x = torch.as_tensor(x, dtype=torch.float64, device="cuda")
+    return torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+
+
+@pytest.mark.parametrize("call", [
+    lambda d: ca.critical_and_caustic_curves(npts=20, s=d, q=0.4),
+    lambda d: ca.critical_and_caustic_curves(npts=20, nlenses=3, **{**B3, "psi": d}),
+    lambda d: ca.mag_point_source(W, s=d, q=0.4),
+    lambda d: ca.mag_point_source_lightcurve(T, 0.0, d, 1.0, 0.6, s=0.9, q=0.4),
+    lambda d: marginalized_log_likelihood([_obs(9)[2] * d], [_obs(9)[0]], [_obs(9)[1]]),
+], ids=["curves", "curves_triple", "point_source", "lightcurve", "ll_A"])
+def test_forward_mode_is_refused(gpu, call):
+    """No entry point has a forward-mode derivative: a dual number is refused, never read as a
+    number without its tangent."""
+    with torch.autograd.forward_ad.dual_level():
+        with pytest.raises(Exception, match="forward mode|jvp"):
+            call(_dual(0.9))
