@@ -66,8 +66,9 @@ class _MargLLSegments(torch.autograd.Function):
     n), and the backward scales it."""
 
     @staticmethod
-    def forward(ctx, need, fs, cs, *As):
-        n = len(As)
+    def forward(ctx, need, n, *tensors):
+        # observations as tensor arguments too: autograd refuses those that carry a tangent
+        As, fs, cs = tensors[:n], tensors[n:2 * n], tensors[2 * n:]
         As = [a if a.shape[1] < 2 or a.stride(1) == 1 else a.contiguous() for a in As]
         B, lens = As[0].shape[0], [a.shape[1] for a in As]
         ll = torch.empty(B, dtype=torch.float64, device=As[0].device)
@@ -81,16 +82,19 @@ class _MargLLSegments(torch.autograd.Function):
         _lib.check(rc, "caus_marginalized_log_likelihood_segments")
         if need:
             ctx.save_for_backward(gA)
-        ctx.lens = lens
+        ctx.need, ctx.lens = need, lens
         ctx.mark_non_differentiable(beta)
         return ll, beta
 
     @staticmethod
     def backward(ctx, g_ll, _g_beta):
+        n = len(ctx.lens)
+        if not ctx.need:   # only observations require a gradient: they are data
+            return (None,) * (2 + 3 * n)
         (gA,) = ctx.saved_tensors
         with torch.no_grad():
             g = g_ll.to(torch.float64)[:, None] * gA
-        return (None, None, None, *g.split(ctx.lens, 1))
+        return (None, None, *g.split(ctx.lens, 1), *(None,) * (2 * n))
 
 
 def _f64(x, device):
@@ -124,7 +128,7 @@ def marginalized_log_likelihood(A_list, fobs_list, C_inv_list, dense_covariance=
         raise ValueError("each fobs / C_inv must have the length of its magnification array")
     if len(As) <= MAX_SEGMENTS:
         need = torch.is_grad_enabled() and any(a.requires_grad for a in As)
-        ll, beta = _MargLLSegments.apply(need, fs, cs, *As)
+        ll, beta = _MargLLSegments.apply(need, len(As), *As, *fs, *cs)
     else:
         A = torch.cat(As, 1).contiguous()
         fobs = torch.cat(fs)

@@ -1,5 +1,5 @@
 """Inputs as torch hands them over: views whose negation or conjugation is only a flag on the
-tensor, forward-mode duals."""
+tensor, forward-mode duals, observations that require gradients."""
 import numpy as np
 import pytest
 import torch
@@ -143,10 +143,20 @@ def _dual(x):
     lambda d: ca.mag_point_source(W, s=d, q=0.4),
     lambda d: ca.mag_point_source_lightcurve(T, 0.0, d, 1.0, 0.6, s=0.9, q=0.4),
     lambda d: marginalized_log_likelihood([_obs(9)[2] * d], [_obs(9)[0]], [_obs(9)[1]]),
-], ids=["curves", "curves_triple", "point_source", "lightcurve", "ll_A"])
+    lambda d: marginalized_log_likelihood([_obs(9)[2]], [_obs(9)[0] * d], [_obs(9)[1]]),
+    lambda d: marginalized_log_likelihood([_obs(9)[2]], [_obs(9)[0]], [_obs(9)[1] * d]),
+], ids=["curves", "curves_triple", "point_source", "lightcurve", "ll_A", "ll_fobs", "ll_c_inv"])
 def test_forward_mode_is_refused(gpu, call):
     """No entry point has a forward-mode derivative: a dual number is refused, never read as a
     number without its tangent."""
     with torch.autograd.forward_ad.dual_level():
         with pytest.raises(Exception, match="forward mode|jvp"):
             call(_dual(0.9))
+
+
+def test_likelihood_observations_get_no_gradient(gpu):
+    f, c, a = _obs(9)
+    f.requires_grad_()
+    _, ll = marginalized_log_likelihood([a], [f], [c])
+    ll.backward()   # accepted; the observations are data
+    assert f.grad is None
