@@ -197,8 +197,7 @@ extern "C" int caus_marginalized_log_likelihood_segments(
         return CAUS_ERR_ARG;
     LLSegments m{};
     for (int k = 0; k < nseg; ++k) {
-        if (n[k] < 0 || (B > 1 && lda[k] < 0) || (n[k] > 0 && (!A[k] || !fobs[k] || !c_inv[k])))
-            return CAUS_ERR_ARG;
+        if (n[k] < 0 || (B > 1 && lda[k] < 0)) return CAUS_ERR_ARG;
         m.A[k] = A[k];
         m.lda[k] = lda[k];
         m.n[k] = n[k];
@@ -208,7 +207,10 @@ extern "C" int caus_marginalized_log_likelihood_segments(
     }
     m.gA = g_A;
     if (B == 0) return CAUS_OK;
-    if (B > (int64_t(1) << 26) || !ll) return CAUS_ERR_ARG;
+    // as the matrix form: no epochs at all are refused, an empty segment among others is not
+    if (B > (int64_t(1) << 26) || !ll || m.ldg == 0) return CAUS_ERR_ARG;
+    for (int k = 0; k < nseg; ++k)
+        if (n[k] > 0 && (!A[k] || !fobs[k] || !c_inv[k])) return CAUS_ERR_ARG;
     const unsigned nb = (unsigned)((B + kLLCurves - 1) / kLLCurves);
     hipLaunchKernelGGL(k_marginalized_ll<LLSegments>, dim3(nb), dim3(kLLBlock), 0,
                        (hipStream_t)stream, m, B, (int)nseg, g_ll, ll, beta);

@@ -51,3 +51,19 @@ def test_argument_errors_enqueue_nothing():
     assert tr(None, None, 10, None, None, 5, None, 4, 2, None, None, None) == _lib.CAUS_ERR_ARG
     assert tr(None, None, 10, None, None, 5, None, 4, 0, None, 8, None) == _lib.CAUS_ERR_ARG
     assert tr(None, None, 10, None, None, 5, None, 0, 0, None, None, None) == _lib.CAUS_OK
+
+
+def test_likelihood_segments_of_no_curves_and_no_epochs():
+    """caus_marginalized_log_likelihood_segments: no curves are nothing to do (empty tensors
+    have null pointers), no epochs are refused; neither reaches a launch."""
+    L = _lib.load_library()
+    null, out = (ctypes.c_void_p * 1)(None), ctypes.c_double()
+    i64 = lambda v: (ctypes.c_int64 * 1)(v)  # noqa: E731
+
+    def call(n, B):
+        return L.caus_marginalized_log_likelihood_segments(
+            None, null, i64(n), null, null, i64(n), 1, B, ctypes.byref(out), None, None, None)
+
+    assert call(9, 0) == _lib.CAUS_OK and call(0, 0) == _lib.CAUS_OK
+    for n, B in ((0, 1), (9, 1), (-1, 0)):
+        assert call(n, B) == _lib.CAUS_ERR_ARG

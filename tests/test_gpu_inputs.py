@@ -160,3 +160,16 @@ def test_likelihood_observations_get_no_gradient(gpu):
     _, ll = marginalized_log_likelihood([a], [f], [c])
     ll.backward()   # accepted; the observations are data
     assert f.grad is None
+
+
+# ---- likelihood: no curves, no epochs ----------------------------------------------------
+def test_likelihood_of_no_curves(gpu):
+    f, c, _ = _obs(9)
+    beta, ll = marginalized_log_likelihood([torch.empty((0, 9), dtype=torch.float64)], [f], [c])
+    assert ll.shape == (0,) and beta[0].shape == (0, 2)
+
+
+def test_likelihood_of_no_epochs_is_refused(gpu):
+    e = torch.empty(0, dtype=torch.float64)
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        marginalized_log_likelihood([e], [e], [e])
