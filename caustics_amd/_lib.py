@@ -51,6 +51,10 @@ SIGNATURES = {
     "caus_mag_point_source_jac": (ctypes.c_int, [_vp, _i32, _vp, _i64, ctypes.POINTER(_vp),
                                                  ctypes.POINTER(_i64), _i64, _vp, _vp, _i32,
                                                  _i32]),
+    "caus_mag_point_source_jac_planes": (ctypes.c_int, [_vp, _i32, _vp, _i64,
+                                                        ctypes.POINTER(_vp),
+                                                        ctypes.POINTER(_i64), _i64, _vp, _vp,
+                                                        ctypes.c_uint32, _i32, _i32]),
     "caus_jacobian_workspace_bytes": (ctypes.c_int64, [_i32, _i64, _i64]),
     "caus_jacobian_vjp": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _i64, _vp, _vp, _vp, _vp,
                                          _i64]),
@@ -58,6 +62,9 @@ SIGNATURES = {
                                                         ctypes.POINTER(_vp),
                                                         ctypes.POINTER(_i64), _i64, _vp, _vp,
                                                         _i32, _i32]),
+    "caus_lightcurve_point_source_jac_planes": (ctypes.c_int, [
+        _vp, _i32, _vp, _i64, ctypes.POINTER(_vp), ctypes.POINTER(_i64), _i64, _vp, _vp,
+        ctypes.c_uint32, _i32, _i32]),
     "caus_lightcurve_workspace_bytes": (ctypes.c_int64, [_i32, _i64, _i64]),
     "caus_lightcurve_point_source": (ctypes.c_int, [_vp, _i32, _vp, _i64, _vp, _i64, _vp, _vp,
                                                     _vp, _vp, _i64, _vp, _i32, _i32]),

@@ -14,6 +14,8 @@ static __device__ __align__(256) double scratch[kLcScratchBytes / sizeof(double)
 
 namespace {
 
+constexpr uint32_t kAllDirs = ~0u;   // every direction's derivative
+
 int np_for(int nl) { return nl == 1 ? 0 : (nl == 2 ? 2 : 5); }
 
 int check_mode(int mode) {
@@ -23,17 +25,17 @@ int check_mode(int mode) {
 }
 
 int ps_dispatch(hipStream_t s, int nl, const cd* w, int64_t N, const PsCols& params,
-                int64_t per, const double* g_mag, double* mag, double* jac,
+                int64_t per, const double* g_mag, double* mag, double* jac, uint32_t dirs,
                 double* g_w, double* g_params, uint8_t* status, int itmax, int mode, bool vjp) {
     switch (nl) {
         case 1:
-            return mag_point_source_nl<1>(s, w, N, params, per, g_mag, mag, jac, g_w,
+            return mag_point_source_nl<1>(s, w, N, params, per, g_mag, mag, jac, dirs, g_w,
                                           g_params, status, itmax, mode, vjp);
         case 2:
-            return mag_point_source_nl<2>(s, w, N, params, per, g_mag, mag, jac, g_w,
+            return mag_point_source_nl<2>(s, w, N, params, per, g_mag, mag, jac, dirs, g_w,
                                           g_params, status, itmax, mode, vjp);
         case 3:
-            return mag_point_source_nl<3>(s, w, N, params, per, g_mag, mag, jac, g_w,
+            return mag_point_source_nl<3>(s, w, N, params, per, g_mag, mag, jac, dirs, g_w,
                                           g_params, status, itmax, mode, vjp);
         default:
             return CAUS_ERR_ARG;
@@ -41,18 +43,18 @@ int ps_dispatch(hipStream_t s, int nl, const cd* w, int64_t N, const PsCols& par
 }
 
 int lc_dispatch(hipStream_t s, int nl, const double* t, int64_t T, const PsCols& lcp, int64_t L,
-                const double* g_mag, double* mag, double* jac, double* ws, uint8_t* status,
-                int itmax, int mode, bool vjp) {
+                const double* g_mag, double* mag, double* jac, uint32_t dirs, double* ws,
+                uint8_t* status, int itmax, int mode, bool vjp) {
     switch (nl) {
         case 1:
-            return lightcurve_point_source_nl<1>(s, t, T, lcp, L, g_mag, mag, jac, ws, status,
-                                                 itmax, mode, vjp);
+            return lightcurve_point_source_nl<1>(s, t, T, lcp, L, g_mag, mag, jac, dirs, ws,
+                                                 status, itmax, mode, vjp);
         case 2:
-            return lightcurve_point_source_nl<2>(s, t, T, lcp, L, g_mag, mag, jac, ws, status,
-                                                 itmax, mode, vjp);
+            return lightcurve_point_source_nl<2>(s, t, T, lcp, L, g_mag, mag, jac, dirs, ws,
+                                                 status, itmax, mode, vjp);
         default:
-            return lightcurve_point_source_nl<3>(s, t, T, lcp, L, g_mag, mag, jac, ws, status,
-                                                 itmax, mode, vjp);
+            return lightcurve_point_source_nl<3>(s, t, T, lcp, L, g_mag, mag, jac, dirs, ws,
+                                                 status, itmax, mode, vjp);
     }
 }
 
@@ -235,10 +237,11 @@ static bool user_cols(const double* const* p, const int64_t* st, int n, PsCols& 
     return true;
 }
 
-extern "C" int caus_mag_point_source_jac(void* stream, int32_t nlenses, const double* w,
-                                         int64_t N, const double* const* params,
-                                         const int64_t* strides, int64_t per, double* mag,
-                                         double* jac, int32_t itmax, int32_t mode) {
+extern "C" int caus_mag_point_source_jac_planes(void* stream, int32_t nlenses, const double* w,
+                                                int64_t N, const double* const* params,
+                                                const int64_t* strides, int64_t per,
+                                                double* mag, double* jac, uint32_t planes,
+                                                int32_t itmax, int32_t mode) {
     if (N < 0 || itmax < 0 || nlenses < 1 || nlenses > 3 || check_mode(mode) != CAUS_OK ||
         per < 1)
         return CAUS_ERR_ARG;
@@ -246,21 +249,38 @@ extern "C" int caus_mag_point_source_jac(void* stream, int32_t nlenses, const do
     PsCols c{};
     if (!w || !mag || !user_cols(params, strides, np_for(nlenses), c)) return CAUS_ERR_ARG;
     return ps_dispatch((hipStream_t)stream, nlenses, reinterpret_cast<const cd*>(w), N, c, per,
-                       nullptr, mag, jac, nullptr, nullptr, nullptr, itmax, mode, jac != nullptr);
+                       nullptr, mag, jac, planes, nullptr, nullptr, nullptr, itmax, mode,
+                       jac != nullptr);
 }
 
-extern "C" int caus_lightcurve_point_source_jac(void* stream, int32_t nlenses, const double* t,
-                                                int64_t T, const double* const* params,
-                                                const int64_t* strides, int64_t L, double* mag,
-                                                double* jac, int32_t itmax, int32_t mode) {
+extern "C" int caus_mag_point_source_jac(void* stream, int32_t nlenses, const double* w,
+                                         int64_t N, const double* const* params,
+                                         const int64_t* strides, int64_t per, double* mag,
+                                         double* jac, int32_t itmax, int32_t mode) {
+    return caus_mag_point_source_jac_planes(stream, nlenses, w, N, params, strides, per, mag, jac,
+                                            kAllDirs, itmax, mode);
+}
+
+extern "C" int caus_lightcurve_point_source_jac_planes(
+    void* stream, int32_t nlenses, const double* t, int64_t T, const double* const* params,
+    const int64_t* strides, int64_t L, double* mag, double* jac, uint32_t planes, int32_t itmax,
+    int32_t mode) {
     if (T < 0 || L < 0 || itmax < 0 || nlenses < 1 || nlenses > 3 || check_mode(mode) != CAUS_OK)
         return CAUS_ERR_ARG;
     if (T == 0 || L == 0) return CAUS_OK;
     PsCols c{};
     if (L > 65535 || !t || !mag || !user_cols(params, strides, 4 + np_for(nlenses), c))
         return CAUS_ERR_ARG;
-    return lc_dispatch((hipStream_t)stream, nlenses, t, T, c, L, nullptr, mag, jac, nullptr,
-                       nullptr, itmax, mode, jac != nullptr);
+    return lc_dispatch((hipStream_t)stream, nlenses, t, T, c, L, nullptr, mag, jac, planes,
+                       nullptr, nullptr, itmax, mode, jac != nullptr);
+}
+
+extern "C" int caus_lightcurve_point_source_jac(void* stream, int32_t nlenses, const double* t,
+                                                int64_t T, const double* const* params,
+                                                const int64_t* strides, int64_t L, double* mag,
+                                                double* jac, int32_t itmax, int32_t mode) {
+    return caus_lightcurve_point_source_jac_planes(stream, nlenses, t, T, params, strides, L, mag,
+                                                   jac, kAllDirs, itmax, mode);
 }
 
 extern "C" int caus_mag_point_source(void* stream, int32_t nlenses, const double* w, int64_t N,
@@ -271,8 +291,8 @@ extern "C" int caus_mag_point_source(void* stream, int32_t nlenses, const double
     if (N == 0) return CAUS_OK;
     if (!w || !mag || (nlenses > 1 && !params) || params_stride < 0) return CAUS_ERR_ARG;
     return ps_dispatch((hipStream_t)stream, nlenses, reinterpret_cast<const cd*>(w), N,
-                       ps_rows(params, params_stride), 1, nullptr, mag, nullptr, nullptr, nullptr,
-                       status, itmax, mode, false);
+                       ps_rows(params, params_stride), 1, nullptr, mag, nullptr, kAllDirs,
+                       nullptr, nullptr, status, itmax, mode, false);
 }
 
 extern "C" int caus_mag_point_source_vjp(void* stream, int32_t nlenses, const double* w,
@@ -286,8 +306,8 @@ extern "C" int caus_mag_point_source_vjp(void* stream, int32_t nlenses, const do
     if (!w || !mag || !g_mag || (nlenses > 1 && !params) || params_stride < 0)
         return CAUS_ERR_ARG;
     return ps_dispatch((hipStream_t)stream, nlenses, reinterpret_cast<const cd*>(w), N,
-                       ps_rows(params, params_stride), 1, g_mag, mag, nullptr, g_w, g_params,
-                       status, itmax, mode, true);
+                       ps_rows(params, params_stride), 1, g_mag, mag, nullptr, kAllDirs, g_w,
+                       g_params, status, itmax, mode, true);
 }
 
 extern "C" int64_t caus_lightcurve_workspace_bytes(int32_t nlenses, int64_t T, int64_t L) {
@@ -311,8 +331,8 @@ extern "C" int caus_lightcurve_point_source(void* stream, int32_t nlenses, const
                 workspace_bytes < caus_lightcurve_workspace_bytes(nlenses, T, L)))
         return CAUS_ERR_ARG;
     hipStream_t s = (hipStream_t)stream;
-    const int rc = lc_dispatch(s, nlenses, t, T, ps_rows(lc_params, 4 + np_for(nlenses)), L, g_mag, mag, nullptr, workspace,
-                               status, itmax, mode, vjp);
+    const int rc = lc_dispatch(s, nlenses, t, T, ps_rows(lc_params, 4 + np_for(nlenses)), L, g_mag,
+                               mag, nullptr, kAllDirs, workspace, status, itmax, mode, vjp);
     if (rc != CAUS_OK || !vjp) return rc;
     const int nq = 4 + np_for(nlenses);
     const int64_t per_block = (int64_t)kPsBlock * lc_epochs_per_lane(T, L);

@@ -145,16 +145,17 @@ inline PsCols ps_rows(const double* rows, int64_t stride) {
 // ---------------------------------------------------------------------------
 // point-source magnification at arbitrary source positions
 //   VJP=false: mag only.  VJP=true: also the derivatives along Re w, Im w and every lens
-//   parameter: with jac they go there plane by plane (jac[d * N + i], the form a later
-//   backward pass scales), else g_w = g*(dm/dRe w + i dm/dIm w) and
+//   parameter: with jac those of the directions in dirs go there plane after plane (the form
+//   a later backward pass scales; forming only these, by a wave-uniform branch each, made the
+//   light curves' kernel 10% slower), else g_w = g*(dm/dRe w + i dm/dIm w) and
 //   g_params[i][k] = g * dm/dparam_k (per evaluation).
 // Item i uses parameter row i / per.
 template <int NL, int MODE, bool VJP>
 __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
     const cd* __restrict__ w, int64_t N, PsCols params, int64_t per,
     const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ jac,
-    double* __restrict__ g_w, double* __restrict__ g_params, uint8_t* __restrict__ status,
-    int itmax) {
+    uint32_t dirs, double* __restrict__ g_w, double* __restrict__ g_params,
+    uint8_t* __restrict__ status, int itmax) {
     constexpr int NP = NL == 1 ? 0 : n_user_params<NL>();
     constexpr int ND = VJP ? 2 + NP : 0;
     const int64_t i = (int64_t)blockIdx.x * kPsBlock + threadIdx.x;
@@ -200,8 +201,13 @@ __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
     if (status) status[i] = ok ? 1 : 0;
     if constexpr (VJP) {
         if (jac) {
+            double* plane = jac + i;
 #pragma unroll
-            for (int d = 0; d < ND; ++d) jac[d * N + i] = dm[d];
+            for (int d = 0; d < ND; ++d)
+                if ((dirs >> d) & 1u) {
+                    *plane = dm[d];
+                    plane += N;
+                }
             return;
         }
         const double g = g_mag[i];
@@ -222,7 +228,7 @@ __global__ __launch_bounds__(kPsBlock) void k_mag_point_source(
 // (trajectory.py:152-155 without parallax, psi -> alpha).  Grid (ceil(T/256), L):
 // each block is one light curve's chunk of epochs; with VJP the block reduces
 // g_mag * dm/dparam over its epochs in a fixed order into ws[l][chunk][param]; with jac the
-// derivatives themselves go there plane by plane (jac[param * L T + l * T + epoch]).
+// derivatives of the parameters in dirs go there plane after plane (L T epochs each).
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -240,7 +246,7 @@ template <int NL, int MODE, bool VJP>
 __global__ __launch_bounds__(kPsBlock) void k_lightcurve_point_source(
     const double* __restrict__ t, int64_t T, PsCols lcp,
     const double* __restrict__ g_mag, double* __restrict__ mag, double* __restrict__ jac,
-    double* __restrict__ ws, uint8_t* __restrict__ status, int itmax, int epl) {
+    uint32_t dirs, double* __restrict__ ws, uint8_t* __restrict__ status, int itmax, int epl) {
     constexpr int NP = NL == 1 ? 0 : n_user_params<NL>();
     constexpr int NQ = 4 + NP;
     constexpr int ND = VJP ? NQ : 0;
@@ -310,9 +316,13 @@ __global__ __launch_bounds__(kPsBlock) void k_lightcurve_point_source(
         if (status) status[l * T + ti] = ok ? 1 : 0;
         if constexpr (VJP) {
             if (jac) {
-                const int64_t LT = (int64_t)gridDim.y * T;
+                double* plane = jac + l * T + ti;
 #pragma unroll
-                for (int k = 0; k < NQ; ++k) jac[k * LT + l * T + ti] = dm[k];
+                for (int k = 0; k < NQ; ++k)
+                    if ((dirs >> k) & 1u) {
+                        *plane = dm[k];
+                        plane += (int64_t)gridDim.y * T;
+                    }
             } else {
                 const double g = g_mag[l * T + ti];
 #pragma unroll
@@ -353,51 +363,37 @@ static __global__ void k_lightcurve_finalize(const double* __restrict__ ws, doub
 template <int NL>
 int mag_point_source_nl(hipStream_t s, const cd* w, int64_t N, const PsCols& params,
                         int64_t per, const double* g_mag, double* mag,
-                        double* jac, double* g_w, double* g_params, uint8_t* status, int itmax,
-                        int mode, bool vjp);
+                        double* jac, uint32_t dirs, double* g_w, double* g_params,
+                        uint8_t* status, int itmax, int mode, bool vjp);
 template <int NL>
 int lightcurve_point_source_nl(hipStream_t s, const double* t, int64_t T, const PsCols& lcp,
                                int64_t L, const double* g_mag, double* mag, double* jac,
-                               double* ws, uint8_t* status, int itmax, int mode, bool vjp);
+                               uint32_t dirs, double* ws, uint8_t* status, int itmax, int mode,
+                               bool vjp);
+
+#define CAUS_PS_CASE(NL, MODE, VJP)                                                             \
+    hipLaunchKernelGGL((k_mag_point_source<NL, MODE, VJP>), grid, block, 0, s, w, N, params, per, \
+                       g_mag, mag, jac, dirs, g_w, g_params, status, itmax);                      \
+    break;
+#define CAUS_LC_CASE(NL, MODE, VJP)                                                             \
+    hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE, VJP>), grid, block, 0, s, t, T, lcp, \
+                       g_mag, mag, jac, dirs, ws, status, itmax, epl);                            \
+    break;
 
 #define CAUS_DEFINE_PS(NL)                                                                       \
     template <>                                                                                  \
     int mag_point_source_nl<NL>(hipStream_t s, const cd* w, int64_t N, const PsCols& params,     \
-                                int64_t per, const double* g_mag, double* mag,                   \
-                                double* jac, double* g_w, double* g_params, uint8_t* status,     \
+                                int64_t per, const double* g_mag, double* mag, double* jac,      \
+                                uint32_t dirs, double* g_w, double* g_params, uint8_t* status,   \
                                 int itmax, int mode, bool vjp) {                                 \
         const dim3 grid((unsigned)((N + kPsBlock - 1) / kPsBlock)), block(kPsBlock);             \
         switch (mode * 2 + (vjp ? 1 : 0)) {                                                      \
-            case 0:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, false>), grid, block, 0, s,\
-                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
-                                   status, itmax);                                               \
-                break;                                                                           \
-            case 1:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64, true>), grid, block, 0, s, \
-                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
-                                   status, itmax);                                               \
-                break;                                                                           \
-            case 2:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64_COMP, false>), grid, block, \
-                                   0, s, w, N, params, per, g_mag, mag, jac, g_w,                \
-                                   g_params, status, itmax);                                     \
-                break;                                                                           \
-            case 3:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_FP64_COMP, true>), grid, block,  \
-                                   0, s, w, N, params, per, g_mag, mag, jac, g_w,                \
-                                   g_params, status, itmax);                                     \
-                break;                                                                           \
-            case 4:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, false>), grid, block, 0, s,\
-                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
-                                   status, itmax);                                               \
-                break;                                                                           \
-            case 5:                                                                              \
-                hipLaunchKernelGGL((k_mag_point_source<NL, MODE_CF32, true>), grid, block, 0, s, \
-                                   w, N, params, per, g_mag, mag, jac, g_w, g_params,            \
-                                   status, itmax);                                               \
-                break;                                                                           \
+            case 0: CAUS_PS_CASE(NL, MODE_FP64, false)                                           \
+            case 1: CAUS_PS_CASE(NL, MODE_FP64, true)                                            \
+            case 2: CAUS_PS_CASE(NL, MODE_FP64_COMP, false)                                      \
+            case 3: CAUS_PS_CASE(NL, MODE_FP64_COMP, true)                                       \
+            case 4: CAUS_PS_CASE(NL, MODE_CF32, false)                                           \
+            case 5: CAUS_PS_CASE(NL, MODE_CF32, true)                                            \
             default:                                                                             \
                 return CAUS_ERR_ARG;                                                             \
         }                                                                                        \
@@ -406,42 +402,18 @@ int lightcurve_point_source_nl(hipStream_t s, const double* t, int64_t T, const 
     template <>                                                                                  \
     int lightcurve_point_source_nl<NL>(hipStream_t s, const double* t, int64_t T,                \
                                        const PsCols& lcp, int64_t L, const double* g_mag,        \
-                                       double* mag, double* jac, double* ws, uint8_t* status, int itmax,\
-                                       int mode, bool vjp) {                                     \
+                                       double* mag, double* jac, uint32_t dirs, double* ws,      \
+                                       uint8_t* status, int itmax, int mode, bool vjp) {         \
         const int epl = lc_epochs_per_lane(T, L);                                                \
         const int64_t per_block = (int64_t)kPsBlock * epl;                                       \
         const dim3 grid((unsigned)((T + per_block - 1) / per_block), (unsigned)L), block(kPsBlock);\
         switch (mode * 2 + (vjp ? 1 : 0)) {                                                      \
-            case 0:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64, false>), grid,      \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
-            case 1:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64, true>), grid,       \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
-            case 2:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64_COMP, false>), grid, \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
-            case 3:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_FP64_COMP, true>), grid,  \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
-            case 4:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_CF32, false>), grid,      \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
-            case 5:                                                                              \
-                hipLaunchKernelGGL((k_lightcurve_point_source<NL, MODE_CF32, true>), grid,       \
-                                   block, 0, s, t, T, lcp, g_mag, mag, jac, ws, status, itmax,   \
-                                   epl);                                                         \
-                break;                                                                           \
+            case 0: CAUS_LC_CASE(NL, MODE_FP64, false)                                           \
+            case 1: CAUS_LC_CASE(NL, MODE_FP64, true)                                            \
+            case 2: CAUS_LC_CASE(NL, MODE_FP64_COMP, false)                                      \
+            case 3: CAUS_LC_CASE(NL, MODE_FP64_COMP, true)                                       \
+            case 4: CAUS_LC_CASE(NL, MODE_CF32, false)                                           \
+            case 5: CAUS_LC_CASE(NL, MODE_CF32, true)                                            \
             default:                                                                             \
                 return CAUS_ERR_ARG;                                                             \
         }                                                                                        \

@@ -15,7 +15,8 @@ import numpy as np
 import torch
 
 from . import _lib
-from .point_source import JACOBIAN_MAX_BYTES, PARAM_NAMES, _mode_id, jacobian_vjp
+from .point_source import (JACOBIAN_MAX_BYTES, PARAM_NAMES, _mode_id, jacobian_vjp,
+                           kept_jacobian)
 
 __all__ = ["mag_point_source_lightcurve", "lightcurve_fwd_vjp", "hexadecapole_gate",
            "hexadecapole_vjp", "mag", "mag_fwd_vjp", "TRAJ_NAMES"]
@@ -65,38 +66,42 @@ class _LightCurve(torch.autograd.Function):
         T = t.numel()
         flat = [c.reshape(-1) if c.numel() == L else c.reshape(-1).expand(L) for c in cols]
         mag = torch.empty((L, T), dtype=torch.float64, device=t.device)
-        jac = None
-        if need and len(cols) * 8 * L * T <= JACOBIAN_MAX_BYTES:
-            jac = torch.empty((len(cols), L * T), dtype=torch.float64, device=t.device)
-        rc = _lib.lib().caus_lightcurve_point_source_jac(
-            _lib.stream_ptr(), nlenses, _lib.ptr(t), T, *_lib.columns(flat), L, _lib.ptr(mag),
-            _lib.ptr(jac), itmax, mode)
-        _lib.check(rc, "caus_lightcurve_point_source_jac")
+        jac, planes = None, 0
         if need:
-            ctx.save_for_backward(t, jac, *([] if jac is not None else
-                                            [torch.stack(flat, -1).contiguous()]))
-        ctx.meta = (nlenses, itmax, mode, L, [c.shape for c in cols])
+            grads = ctx.needs_input_grad[5:]
+            planes = sum(1 << k for k, g in enumerate(grads) if g)
+            jac = kept_jacobian(sum(grads), L * T, t.device, JACOBIAN_MAX_BYTES)
+        rc = _lib.lib().caus_lightcurve_point_source_jac_planes(
+            _lib.stream_ptr(), nlenses, _lib.ptr(t), T, *_lib.columns(flat), L, _lib.ptr(mag),
+            _lib.ptr(jac), planes, itmax, mode)
+        _lib.check(rc, "caus_lightcurve_point_source_jac_planes")
+        if jac is not None:
+            ctx.save_for_backward(jac)
+        elif need:
+            ctx.save_for_backward(None, t, torch.stack(flat, -1).contiguous())
+        ctx.meta = (nlenses, itmax, mode, L, T, [c.shape for c in cols], planes)
         return mag
 
     @staticmethod
     def backward(ctx, g):
-        t, jac, *lcp = ctx.saved_tensors
-        nlenses, itmax, mode, L, shapes = ctx.meta
+        jac, *again = ctx.saved_tensors
+        nlenses, itmax, mode, L, T, shapes, planes = ctx.meta
         g = _lib.resolved(g.contiguous().to(torch.float64))
         if jac is not None:
-            _, gp = jacobian_vjp(jac, 0, max(t.numel(), 1), g, False, True)
+            _, gp = jacobian_vjp(jac, 0, max(T, 1), g, False, True)
         else:
-            _, gp, _ = _call(t, lcp[0], g, nlenses, itmax, mode)
-            gp = gp.t()
-        if t.numel() == 0:
-            gp = torch.zeros((len(shapes), L), dtype=torch.float64, device=t.device)
+            _, gp, _ = _call(*again, g, nlenses, itmax, mode)
+            gp, planes = gp.t(), ~0
+        if T == 0:
+            gp, planes = torch.zeros((len(shapes), L), dtype=torch.float64, device=g.device), ~0
         gps = []
-        gp = gp.unbind(0)
+        gp = iter(gp.unbind(0))
         for k, shape in enumerate(shapes):
+            row = next(gp) if (planes >> k) & 1 else None
             if not ctx.needs_input_grad[5 + k]:
                 gps.append(None)
             else:
-                gps.append((gp[k] if shape.numel() == L else gp[k].sum()).reshape(shape))
+                gps.append((row if shape.numel() == L else row.sum()).reshape(shape))
         return (None, None, None, None, None, *gps)
 
 

@@ -62,16 +62,54 @@ def _prepare(w, nlenses, params):
     return w, ps
 
 
-# A backward pass scales and reduces the Jacobian that the forward pass kept, (2 + P) * 8
-# bytes a position (a light curve's epoch (4 + P) * 8).  Solving the roots again instead
-# costs 8 times as much (512,000 binary epochs: 93 against 11 us on one MI355X) and no
-# memory, so calls whose Jacobian would exceed this many bytes do that.
+# A backward pass scales and reduces the Jacobian that the forward pass kept, 8 bytes a position
+# for each parameter that requires a gradient (16 for the position itself).  Solving the roots
+# again instead costs 8 times as much (512,000 binary epochs: 93 against 11 us on one MI355X)
+# and no memory, so that is what a call does whose Jacobian would exceed this many bytes, or
+# would leave less than half of the card free (the Jacobians of one graph add up), or cannot be
+# allocated.
 JACOBIAN_MAX_BYTES = 4 << 30
+# Asking for the free memory takes 5 us, and up to 20 where the autograd engine's thread is slow
+# to wake, so it is asked once for this many bytes of Jacobians handed out.
+JACOBIAN_ASK_BYTES = 1 << 30
+# device index -> bytes that may be handed out before the next question (threads that race for it
+# hand out at most that much each)
+_jacobian_credit = {}
+
+
+def _half_free(need, device):
+    """need bytes out of the half of the card that Jacobians may take: what the driver has free,
+    and what torch's allocator holds unused."""
+    free, total = torch.cuda.mem_get_info(device)
+    if free - need >= total // 2:
+        return True
+    st = torch.cuda.memory_stats_as_nested_dict(device)
+    held = st["reserved_bytes"]["all"]["current"] - st["allocated_bytes"]["all"]["current"]
+    return free + held - need >= total // 2
+
+
+def kept_jacobian(planes, N, device, limit):
+    """Memory for the (planes, N) Jacobian of a forward pass, or None where the backward pass is
+    to solve again."""
+    need = 8 * planes * N
+    if need > limit:
+        return None
+    credit = _jacobian_credit.get(device.index, 0)
+    if need > credit:
+        credit = need + JACOBIAN_ASK_BYTES
+        if not _half_free(credit, device):
+            return None
+    _jacobian_credit[device.index] = credit - need
+    try:
+        return torch.empty((planes, N), dtype=torch.float64, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def jacobian_vjp(jac, nw, rows, g, want_w, want_p):
     """Backward pass of the kept Jacobian jac (nw + np, N) for cotangents g (N,): (g_w (N,)
-    complex or None, g_p (np, N / rows) sums over rows of consecutive items or None)."""
+    complex or None, g_p (np, N / rows) sums over rows of consecutive items or None).  The np
+    planes are those of the parameters that require a gradient, in their order."""
     npl, N = jac.shape
     n_p = npl - nw
     g_w = torch.empty(N, dtype=torch.complex128, device=jac.device) if want_w else None
@@ -119,34 +157,38 @@ class _MagPointSource(torch.autograd.Function):
         else:
             cols = [p.expand(shape).reshape(-1) for p in ps]
         mag = torch.empty(N, dtype=torch.float64, device=w.device)
-        jac = None
-        if need and (2 + P) * 8 * N <= JACOBIAN_MAX_BYTES:
-            jac = torch.empty((2 + P, N), dtype=torch.float64, device=w.device)
-        rc = _lib.lib().caus_mag_point_source_jac(_lib.stream_ptr(), nlenses, _lib.ptr(wf), N,
-                                                  *_lib.columns(cols), per, _lib.ptr(mag),
-                                                  _lib.ptr(jac), itmax, mode)
-        _lib.check(rc, "caus_mag_point_source_jac")
+        jac, nw, planes = None, 0, 0
+        if need:
+            grad_w, *grad_p = ctx.needs_input_grad[4:]
+            nw = 2 if grad_w else 0
+            planes = (3 if grad_w else 0) | sum(4 << k for k, g in enumerate(grad_p) if g)
+            jac = kept_jacobian(nw + sum(grad_p), N, w.device, JACOBIAN_MAX_BYTES)
+        rc = _lib.lib().caus_mag_point_source_jac_planes(
+            _lib.stream_ptr(), nlenses, _lib.ptr(wf), N, *_lib.columns(cols), per,
+            _lib.ptr(mag), _lib.ptr(jac), planes, itmax, mode)
+        _lib.check(rc, "caus_mag_point_source_jac_planes")
         if jac is not None:
-            ctx.save_for_backward(wf, jac)
+            ctx.save_for_backward(jac)
         elif need:
             prm = torch.stack([c.expand(N // per) for c in cols], -1).contiguous() if P else None
-            ctx.save_for_backward(wf, None, prm)
-        ctx.meta = (nlenses, itmax, mode, shape, per, w.shape, [p.shape for p in ps])
+            ctx.save_for_backward(None, wf, prm)
+        ctx.meta = (nlenses, itmax, mode, shape, per, w.shape, [p.shape for p in ps], nw, planes)
         return mag.reshape(shape)
 
     @staticmethod
     def backward(ctx, g):
-        nlenses, itmax, mode, shape, per, wshape, pshapes = ctx.meta
-        wf, jac, *prm = ctx.saved_tensors
+        nlenses, itmax, mode, shape, per, wshape, pshapes, nw, planes = ctx.meta
+        jac, *again = ctx.saved_tensors
         P = len(pshapes)
-        N = wf.numel()
         want_w, want_p = ctx.needs_input_grad[4], any(ctx.needs_input_grad[5:])
         gf = _lib.resolved(g.expand(shape).contiguous().reshape(-1).to(torch.float64))
         if jac is not None:
-            g_w, g_p = jacobian_vjp(jac, 2, per, gf, want_w, want_p)
+            g_w, g_p = jacobian_vjp(jac, nw, per, gf, want_w, want_p)
             pshape = shape if per == 1 else None   # summed over the rows already
         else:
-            prm = prm[0] if P else None
+            wf, prm = again
+            N = wf.numel()
+            planes = ~0
             pstride = P if P and prm.shape[0] > 1 else 0
             if pstride and per > 1:
                 prm = prm.repeat_interleave(per, 0)
@@ -161,14 +203,15 @@ class _MagPointSource(torch.autograd.Function):
             pshape = shape
         gw = g_w.reshape(shape).sum_to_size(wshape) if want_w else None
         gps = []
-        g_p = g_p.unbind(0) if g_p is not None else None
+        g_p = iter(g_p.unbind(0)) if g_p is not None else None
         for k, ps_shape in enumerate(pshapes):
+            row = next(g_p) if g_p is not None and (planes >> (2 + k)) & 1 else None
             if not ctx.needs_input_grad[5 + k]:
                 gps.append(None)
             elif pshape is None:
-                gps.append(g_p[k].reshape(ps_shape))
+                gps.append(row.reshape(ps_shape))
             else:
-                gps.append(g_p[k].reshape(shape).sum_to_size(ps_shape))
+                gps.append(row.reshape(shape).sum_to_size(ps_shape))
         return (None, None, None, None, gw, *gps)
 
 

@@ -131,6 +131,13 @@ int caus_mag_point_source_jac(void* stream, int32_t nlenses, const double* w, in
                               const double* const* params, const int64_t* strides,
                               int64_t per, double* mag, double* jac, int32_t itmax, int32_t mode);
 
+/* The same with the planes of the bits of `planes` only, plane after plane: bit 0 Re w, bit 1
+ * Im w, bit 2+k parameter k; jac (number of those bits, N). */
+int caus_mag_point_source_jac_planes(void* stream, int32_t nlenses, const double* w, int64_t N,
+                                     const double* const* params, const int64_t* strides,
+                                     int64_t per, double* mag, double* jac, uint32_t planes,
+                                     int32_t itmax, int32_t mode);
+
 /* The backward pass of a kept Jacobian of nw + np planes of N, nw (0 or 2) of them along
  * Re w and Im w, for cotangents g (N,):
  *   g_w      (N,) complex or NULL:  g * (plane 0 + i plane 1)
@@ -165,6 +172,13 @@ int caus_lightcurve_point_source_jac(void* stream, int32_t nlenses, const double
                                      const double* const* params, const int64_t* strides,
                                      int64_t L, double* mag, double* jac, int32_t itmax,
                                      int32_t mode);
+
+/* The same with the planes of the bits of `planes` only: bit k parameter k. */
+int caus_lightcurve_point_source_jac_planes(void* stream, int32_t nlenses, const double* t,
+                                            int64_t T, const double* const* params,
+                                            const int64_t* strides, int64_t L, double* mag,
+                                            double* jac, uint32_t planes, int32_t itmax,
+                                            int32_t mode);
 
 /* caus_lightcurve_point_source without a workspace argument: it allocates nothing and
  * takes no caller memory beyond inputs and outputs.  No counterpart in the reference; it
