@@ -2375,9 +2375,15 @@ int ext_flat_grid(int64_t max_lanes);
 // 2477 -> 2058, 3586 -> 5706.  Sources with sizes of their own count for less, since most are
 // far below the largest: 1,000 of 256-1024 points 624 -> 484 (two) and 1617 -> 1597 us (three),
 // 1,200 of 256-4096 1016 -> 1373 and 3666 -> 4860.
+// A limit on the sweeps that could stop a converging solve keeps the one-lane solver, whose
+// roots move one after the other: it counts, and needs, other sweeps than the group, whose roots
+// move together, and which sources of a call converge must not depend on how many there are.  Of
+// 4,800 sources at caustics (up to q3 = 1e-6) none needed more than 25 sweeps either way.
 template <int NL>
 bool ext_grouped(const ExtArgs& a) {
     constexpr int64_t tasks = 16000, sources = 1200;
+    constexpr int itmax = 250;
+    if (a.itmax < itmax) return false;
     const int64_t share = a.npts ? (NL == 3 ? 2 : 4) : 1;
     return a.S <= sources && a.S * a.nadd_max <= tasks * share;
 }

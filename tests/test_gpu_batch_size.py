@@ -1,0 +1,55 @@
+"""Contour results of a source by itself and of the same source in a large batch, which other
+kernels solve (small batches: groups of lanes)."""
+import numpy as np
+import pytest
+import torch
+
+import caustics_amd as ca
+from caustics_amd import _lib
+from caustics_amd.extended_source import _run
+
+pytestmark = pytest.mark.gpu
+
+LENSES = {
+    "binary": dict(s=0.9, q=0.4),
+    "planet": dict(s=0.7, q=1e-5),
+    "triple": dict(s=0.9, q=0.4, q3=0.3, r3=0.8, psi=0.7),
+    "triple_planet": dict(s=1.1, q=1e-3, q3=1e-6, r3=1.2, psi=2.1),
+}
+
+
+def at_caustics(lens, rho, S, seed=1):
+    """S source centres within two radii of the lens' caustics."""
+    r = np.random.default_rng(seed)
+    nl = 2 if len(LENSES[lens]) == 2 else 3
+    c = ca.critical_and_caustic_curves(npts=400, nlenses=nl, **LENSES[lens])[1]
+    return nl, r.choice(c.reshape(-1).cpu().numpy(), S) + \
+        rho * r.uniform(0, 2, S) * np.exp(2j * np.pi * r.uniform(size=S))
+
+
+def alone_and_among(lens, rho, S, itmax=2500, npts=200, ld=False):
+    """(mag, status, gradients) of S sources as a call of their own and among skipped ones,
+    which make the call large."""
+    nl, w = at_caustics(lens, rho, S)
+    f64 = lambda x: torch.as_tensor(x, dtype=torch.float64, device="cuda")  # noqa: E731
+    out = []
+    for pad in (0, 1300):
+        n = S + pad
+        prm = f64([list(LENSES[lens].values())]).expand(n, -1).contiguous()
+        wt = torch.as_tensor(np.resize(w, n), device="cuda")
+        res = _run(nl, wt, f64(np.full(n, rho)), prm, None, npts, ld,
+                   f64(np.full(n, 0.4)) if ld else None, 20, itmax, _lib.MODE_FP64,
+                   g=f64(np.ones(n)), skip=torch.arange(n, device="cuda") >= S)
+        out.append([x[:S].cpu().numpy() for x in res])
+    return out
+
+
+@pytest.mark.parametrize("lens", list(LENSES))
+@pytest.mark.parametrize("itmax", [1, 5, 8, 12, 16, 20, 249])
+def test_iteration_limit_means_the_same_in_every_batch(gpu, lens, itmax):
+    """A limit on the sweeps stops the same solves whatever else is in the call."""
+    alone, among = alone_and_among(lens, 1e-3, 60, itmax)
+    for a, b in zip(alone, among):
+        np.testing.assert_array_equal(a, b)
+    assert itmax < 249 or alone[1].all()
+    assert itmax > 8 or not alone[1].all()
