@@ -1579,7 +1579,9 @@ void k_ext_solve_add(ExtArgs A, int cur) {
 // sweep of the compensated polish take one root's instructions.  Roots are exchanged through
 // LDS within a wave.  All roots move together (Jacobi form), where the one-lane solver moves
 // them one after the other; both end in the compensated polish, which takes every root to the
-// double nearest the exact one whatever led there, so the results are the same.
+// double nearest the exact one whatever led there.  A nearly double pair can still move when
+// the polish's sweeps end, so the results are the same to rounding (of 19,200 sources at caustics
+// 1 magnification and 4 gradients differed, by up to 5e-12; all others were the same bits).
 template <int NL>
 constexpr int ext_group() {
     return NL == 3 ? 16 : 8;

@@ -101,12 +101,13 @@ def _run(nlenses, w, rho_t, prm, npts_host, npts_max, ld, u1_t, npts_ld, itmax, 
     continuation, stitching) overlap another chunk's solves and integrals; the caller's
     stream waits for all of them.  `skip`, a (S,) bool CUDA tensor, marks sources to
     leave out (npts_limb 0 for the kernels: no work, magnification and gradient 0); it
-    is applied on the device, so nothing waits for the host.  Per-source results do not
-    depend on the batch around them.  `work`, a (5,) int64 CUDA tensor, accumulates the
+    is applied on the device, so nothing waits for the host.  Per-source results depend on
+    the batch around them by rounding at most: small batches and chunks are solved by other
+    kernels than large ones (ext_grouped).  `work`, a (5,) int64 CUDA tensor, accumulates the
     kernels' work counters (FP64, FP32 and compensated root-iterations, limb-point
     solves, contour points).  The schedule (chunk workspace budget `chunk_bytes`,
     `streams`, the flat kernels' workgroups per CU) comes from the tuned table of
-    caustics_amd.autotune unless the caller fixes it; it changes no result."""
+    caustics_amd.autotune unless the caller fixes it; it changes no result otherwise."""
     L = _lib.lib()
     S = w.numel()
     if max_chunk is None and (chunk_bytes is None or streams is None):

@@ -53,3 +53,20 @@ def test_iteration_limit_means_the_same_in_every_batch(gpu, lens, itmax):
         np.testing.assert_array_equal(a, b)
     assert itmax < 249 or alone[1].all()
     assert itmax > 8 or not alone[1].all()
+
+
+@pytest.mark.parametrize("ld", [False, True])
+@pytest.mark.parametrize("rho", [1e-2, 1e-3, 1e-4])
+@pytest.mark.parametrize("lens", list(LENSES))
+def test_sources_at_caustics_by_themselves_and_in_a_large_call(gpu, lens, rho, ld):
+    """At caustics, with third lenses down to 1e-6, where an ulp in a coefficient moves roots by
+    1e-6 and magnifications by per cent: both ways have to round the coefficients alike and
+    polish the roots to the same doubles.  Only roots of a nearly double pair that has not come
+    to rest may differ: an ulp of such an image, 2e-16, is magnified by 1/|det J|, at most some
+    1e4 at these distances, once into the magnification's integrand and twice into a
+    derivative's."""
+    alone, among = alone_and_among(lens, rho, 300, ld=ld)
+    np.testing.assert_array_equal(alone[1], among[1])
+    np.testing.assert_allclose(alone[0], among[0], rtol=1e-11, atol=0.0)
+    largest = np.abs(among[2]).max(1, keepdims=True)
+    assert (np.abs(alone[2] - among[2]) <= 1e-8 * largest).all()
