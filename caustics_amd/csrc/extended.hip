@@ -138,31 +138,60 @@ namespace {
 // Greedy continuation of root sets along a sequence (match_points chained as in
 // critical_and_caustic_curves, point_source.py:1628-1640), one workgroup per chain
 // (chain.hpp): one wave up to 64 points, four above.  One lane per chain, point after point,
-// took 395 us for a chain of 200 points of 4 roots; this form 4.7 us.
+// takes 395 us for a chain of 200 points of 4 roots; this form 4.7 us.
 template <int DEG, int NT>
 __global__ __launch_bounds__(NT) void k_match_chain(const cd* __restrict__ pts, cd* out,
                                                     int64_t npts, int64_t nchains) {
     for (int64_t c = blockIdx.x; c < nchains; c += gridDim.x) {
+        const cd* p = pts + c * npts * DEG;
+        cd* o = out + c * npts * DEG;
+        // the permutation words wait in each output point's first component, which its own
+        // thread overwrites after reading the word
+        uint64_t* ow = reinterpret_cast<uint64_t*>(o);
+        auto get = [p](int64_t k, int r) { return p[k * DEG + r]; };
+        auto word = [ow](int64_t k) -> uint64_t& { return ow[2 * k * DEG]; };
+        chain_perms<DEG, NT>(get, word, npts);
+        for (int64_t k = threadIdx.x; k < npts; k += NT) {
+            const uint64_t w = word(k);
+#pragma unroll
+            for (int i = 0; i < DEG; ++i) o[k * DEG + i] = p[k * DEG + pget(w, i)];
+        }
+    }
+}
+
+// One lane per chain, point after point, for many short chains: up to 12 points leave most lanes
+// of a chain's wave idle.  One MI355X, a wave -> a lane per chain: 200,000 chains of 4 roots and 2
+// points 141 -> 16 us, 4 points 146 -> 31, 12 points 198 -> 152; of 10 roots and 12 points 604 ->
+// 381; 16,384 chains of 10 roots and 12 points 55 -> 46.  Of 16 points or of 8,192 chains some are
+// faster one way and some the other.
+// Bound: below a dozen points the launch, then the chain of dependent steps.
+template <int DEG>
+__global__ __launch_bounds__(64) void k_match_short_chains(const cd* __restrict__ pts,
+                                                           cd* __restrict__ out, int64_t npts,
+                                                           int64_t nchains) {
+    const int64_t c = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (c >= nchains) return;
     const cd* p = pts + c * npts * DEG;
     cd* o = out + c * npts * DEG;
-    // the permutation words wait in each output point's first component, which its own
-    // thread overwrites after reading the word
-    uint64_t* ow = reinterpret_cast<uint64_t*>(o);
-    auto get = [p](int64_t k, int r) { return p[k * DEG + r]; };
-    auto word = [ow](int64_t k) -> uint64_t& { return ow[2 * k * DEG]; };
-    chain_perms<DEG, NT>(get, word, npts);
-    for (int64_t k = threadIdx.x; k < npts; k += NT) {
-        const uint64_t w = word(k);
+    cd a[DEG], b[DEG];
+    load_pt<DEG>(p, 0, a);
+    store_pt<DEG>(o, 0, a);
+    for (int64_t k = 1; k < npts; ++k) {
+        load_pt<DEG>(p, k, b);
+        const uint64_t perm = greedy_match<DEG>(a, b);
 #pragma unroll
-        for (int i = 0; i < DEG; ++i) o[k * DEG + i] = p[k * DEG + pget(w, i)];
-    }
+        for (int i = 0; i < DEG; ++i) a[i] = p[k * DEG + pget(perm, i)];
+        store_pt<DEG>(o, k, a);
     }
 }
 
 template <int DEG>
 void match_chain(hipStream_t s, const cd* p, cd* o, int64_t npts, int64_t nchains) {
     const dim3 g((unsigned)(nchains < (1 << 20) ? nchains : (1 << 20)));   // strides over chains
-    if (npts <= 64)
+    if (npts <= 12 && nchains >= 16384)
+        hipLaunchKernelGGL((k_match_short_chains<DEG>), dim3((unsigned)((nchains + 63) / 64)),
+                           dim3(64), 0, s, p, o, npts, nchains);
+    else if (npts <= 64)
         hipLaunchKernelGGL((k_match_chain<DEG, 64>), g, dim3(64), 0, s, p, o, npts, nchains);
     else
         hipLaunchKernelGGL((k_match_chain<DEG, 256>), g, dim3(256), 0, s, p, o, npts, nchains);

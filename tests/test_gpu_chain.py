@@ -54,3 +54,25 @@ def test_match_chain_is_the_greedy_rule(gpu, n, npts):
         with np.errstate(invalid="ignore"):
             ref = greedy_chain(x[c])
         np.testing.assert_array_equal(o[c].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n", [2, 4, 5, 6, 10])
+@pytest.mark.parametrize("npts", [1, 2, 12, 13])
+def test_many_short_chains(gpu, n, npts):
+    """16,384 chains and one more, of up to 12 points (a lane each) and of 13, equal the same
+    chains a few at a time."""
+    g = np.random.default_rng(10 * n + npts)
+    few = g.normal(size=(511, npts, n)) + 1j * g.normal(size=(511, npts, n))
+    few[::7] = g.integers(-2, 3, few[::7].shape)          # ties and coincident rows
+    few[3, npts // 2, n // 2] = np.nan
+    few[5, npts // 3, 0] = complex(np.inf, 0.0)
+    many = np.resize(few, (16385, npts, n))
+
+    def chain(x):
+        p = torch.as_tensor(x, device="cuda")
+        o = torch.full_like(p, -7.0)
+        _lib.check(_lib.lib().caus_match_chain(_lib.stream_ptr(), _lib.ptr(p), _lib.ptr(o), npts,
+                                               n, len(x)), "caus_match_chain")
+        return o.cpu().numpy()
+
+    np.testing.assert_array_equal(chain(many), np.resize(chain(few), many.shape))
