@@ -70,3 +70,43 @@ def test_sources_at_caustics_by_themselves_and_in_a_large_call(gpu, lens, rho, l
     np.testing.assert_allclose(alone[0], among[0], rtol=1e-11, atol=0.0)
     largest = np.abs(among[2]).max(1, keepdims=True)
     assert (np.abs(alone[2] - among[2]) <= 1e-8 * largest).all()
+
+
+# few sources: groups of lanes, cut line integrals; many: the flat kernels; limb sizes of both
+# selection kernels (512 points are one wave's)
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("npts", [512, 1024])
+@pytest.mark.parametrize("S", [6, 1300])
+@pytest.mark.parametrize("lens", ["binary", "triple"])
+def test_workspace_contents_do_not_change_results(gpu, lens, S, npts, grad):
+    """Every workspace read is of memory that the same launch sequence wrote before, on every
+    route: a workspace holding the 64-bit value 1 in every word gives the bits of a zero-filled
+    one (a stale index would read 0 or 1 there, a stale double a tiny number)."""
+    from caustics_amd.extended_source import extended_workspace_bytes
+
+    rho = 1e-2
+    nl, w = at_caustics(lens, rho, S)
+    g = np.random.default_rng(S)
+    sizes = g.choice([4, 20, npts // 2, npts], S).astype(np.int32)
+    sizes[:2] = npts, 0   # one of the largest, one skipped
+    dev = lambda x: torch.as_tensor(x, device="cuda").contiguous()  # noqa: E731
+    wt, rho_t, u1 = dev(w), dev(np.full(S, rho)), dev(np.full(S, 0.4))
+    prm = dev(np.tile(list(LENSES[lens].values()), (S, 1)))
+    nt, gm = dev(sizes), dev(g.normal(size=S)) if grad else None
+    nb = extended_workspace_bytes(nl, S, npts)
+    out = []
+    for fill in (0, 1):
+        ws = torch.full(((nb + 7) // 8,), fill, dtype=torch.int64, device="cuda")
+        mag = torch.empty(S, dtype=torch.float64, device="cuda")
+        st = torch.empty(S, dtype=torch.uint8, device="cuda")
+        go = torch.zeros((S, 4 + prm.shape[1]), dtype=torch.float64, device="cuda")
+        _lib.check(_lib.lib().caus_mag_extended_source_work(
+            _lib.stream_ptr(), nl, _lib.ptr(wt), S, _lib.ptr(rho_t), _lib.ptr(prm), prm.shape[1],
+            _lib.ptr(nt), npts, 1, _lib.ptr(u1), 1, 20, _lib.ptr(gm), _lib.ptr(mag),
+            _lib.ptr(go) if grad else None, _lib.ptr(st), _lib.ptr(ws), ws.numel() * 8, 2500,
+            _lib.MODE_FP64, None), "caus_mag_extended_source_work")
+        torch.cuda.synchronize()
+        out.append((mag, go, st))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    assert out[0][0][1].item() == 0 and bool(torch.isfinite(out[0][0]).all())
