@@ -322,7 +322,7 @@ struct LDSource {
     double e[NL];
     cd r[NL];
     cd w0;
-    double rho, rho2x, irho, irho2, u1, c3;   // rho2x = 2 rho
+    double rho, rho2x, irho, irho2, u1, c3;   // rho2x = 2 rho (infinite: see ld_source)
 };
 template <int NL>
 __device__ __forceinline__ LDSource<NL> ld_source(const LensFrame<NL>& lf, cd w0, double rho,
@@ -336,7 +336,8 @@ __device__ __forceinline__ LDSource<NL> ld_source(const LensFrame<NL>& lf, cd w0
     q.w0 = cd{uniform(w0.re), uniform(w0.im)};
     q.rho = uniform(rho);
     q.irho = uniform(rcp(rho));
-    q.rho2x = uniform(2.0 * rho);
+    // r = |D| / rho of a negative radius is never above 1: the profile's outer branch is off
+    q.rho2x = uniform(rho < 0.0 ? INFINITY : 2.0 * rho);
     q.irho2 = uniform(q.irho * q.irho);
     q.u1 = uniform(u1);
     q.c3 = uniform(3.0 / (3.0 - u1));

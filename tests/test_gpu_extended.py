@@ -475,3 +475,25 @@ def test_small_batches_match_large_ones(gpu, nlenses, npts):
     # without gradients the line integrals of one source are cut over workgroups
     fwd = mag_extended_source(w, rho, **kw, **p)
     np.testing.assert_allclose(fwd.cpu().numpy(), few[0].cpu().numpy(), rtol=1e-13)
+
+
+@pytest.mark.parametrize("nlenses", [1, 2, 3])
+def test_negative_radius(gpu, nlenses):
+    """rho < 0 (a sampler's step out of range) is the formulas taken literally: r = |D|/rho is
+    negative, so the profile's inner branch holds everywhere; the oracle's value, and the
+    derivative along rho of the forward kernel."""
+    from caustics_amd.extended_source import extended_fwd_vjp
+
+    prm = {1: {}, 2: dict(s=0.9, q=0.4), 3: dict(s=0.9, q=0.4, q3=0.3, r3=0.8, psi=0.7)}[nlenses]
+    w, rho = np.array([0.1 + 0.05j, 0.6 + 0.2j, -0.4 + 0.5j]), -0.01
+    kw = dict(nlenses=nlenses, npts_limb=60, limb_darkening=True, npts_ld=11, u1=0.3)
+    mo = np.array([E.mag_extended_source(x, rho, **kw, **prm) for x in w])
+    m, g, _ = extended_fwd_vjp(w, rho, np.ones(3), **kw, **prm)
+    compare(m.cpu().numpy(), mo, f"rho < 0 nlenses={nlenses}")
+    f = lambda r: mag_extended_source(w, r, **kw, **prm).cpu().numpy()  # noqa: E731
+    assert np.array_equal(f(rho), m.cpu().numpy())
+    h = 1e-9
+    fd, fd2 = _fd(f, rho, h), _fd(f, rho, 2 * h)
+    stable = np.abs(fd - fd2) <= 1e-4 * np.maximum(np.abs(fd), 1e-3 * mo)
+    err = np.abs(g[:, 2].cpu().numpy() - fd) / np.maximum(np.abs(fd), 1e-3 * mo)
+    assert stable.any() and (err[stable] < 2e-4).all()
