@@ -2194,6 +2194,7 @@ __global__ __launch_bounds__(kExtBlock) void k_ext_contours(ExtArgs A, int buf) 
                     }
                     np += 1;
                     at_ += sq.len;
+                    wave_sync();   // every lane has read the segment
                     if (lane == q) {
                         // the reference zeroes a merged segment (rest[i] = 0): its ends
                         // then rank by their distance from the origin, not as the
