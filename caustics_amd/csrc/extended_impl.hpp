@@ -32,7 +32,7 @@ constexpr int kExtBlock = 256;    // block of the per-source integration kernel
 constexpr int kExtWaveBlock = 64; // block of the per-source bookkeeping kernels (one wave)
 constexpr int kExtMaxSeg = 32;     // >= 3 * (nlenses^2 + 1)
 constexpr int kExtMaxPieces = 48;  // pieces of one stitched contour
-constexpr int kExtSortMax = 4096;  // limb points per source (gaps sorted in LDS)
+constexpr int kExtSortMax = 4096;  // limb points per source (k_ext_select's register tiles)
 
 template <int NL>
 constexpr int ext_degree() {
@@ -231,12 +231,6 @@ struct Seg {
 };
 struct Piece {
     int row, start, len, rev;
-};
-struct Contour {
-    Piece pc[kExtMaxPieces];
-    int np;
-    int npts;  // points (without the closing point)
-    int par;   // parity of the first point
 };
 
 // Final limb points in limb order, row after row (image `row` of point k at row * ld + k):
@@ -837,68 +831,68 @@ __device__ double integrate_source_ld(ZRows zb, const double* theta, ExtCEntry* 
                                       int parts) {
     const int tid = threadIdx.x;
     if constexpr (!SUMS) {
-    // centroids (integrate.py:112); the closing point repeats c_0 in the sum
-    for (int c = 0; c < nc; ++c) {
-        const ExtCEntry& e = ct[c];
-        double sx = 0.0, sy = 0.0;
-        for (int k = tid; k < e.L; k += kExtBlock) {
-            const cd a = contour_point<DEG>(zb, e.pc, e.np, k);
-            sx += a.re;
-            sy += a.im;
-        }
-        const cd c0 = (e.L > 0) ? contour_point<DEG>(zb, e.pc, e.np, 0) : cd{0.0, 0.0};
-        const double zx = (block_sum(sx, shd) + c0.re) / e.cdiv;
-        const double zy = (block_sum(sy, shd) + c0.im) / e.cdiv;
-        if (tid == 0) {
-            ct[c].zx = zx;
-            ct[c].zy = zy;
-        }
-    }
-    __syncthreads();
-    // the P lines of every point, then the Q lines, flat over the contours
-    for (int u = tid + part * kExtBlock; u < 2 * T; u += parts * kExtBlock) {
-        const bool isP = u < T;
-        const int gi = isP ? u : u - T;
-        int c = 0;
-        while (c + 1 < nc && gi >= ct[c + 1].off) ++c;
-        const ExtCEntry& e = ct[c];
-        const int k = gi - e.off;
-        const cd zk = contour_point<DEG>(zb, e.pc, e.np, k);
-        if constexpr (!VJP) {
-            if (isP)
-                pq[2 * gi] = ld_line<NL, true>(zk.re, e.zy, zk.im, q, gl);
-            else
-                pq[2 * gi + 1] = ld_line<NL, false>(zk.im, e.zx, zk.re, q, gl);
-        } else {
-            const int L = e.L;
-            const int kn = (k + 1 == L) ? 0 : k + 1;
-            const int kp = (k == 0) ? L - 1 : k - 1;
-            const cd zn = contour_point<DEG>(zb, e.pc, e.np, kn);
-            const cd zp = contour_point<DEG>(zb, e.pc, e.np, kp);
-            // cotangent of P_k or Q_k from the two trapezoid terms it enters; P_k =
-            // P(x_k; y0 .. y_k), Q_k = Q(y_k; x0 .. x_k), (x0, y0) the centroid
-            double bar = 0.0, df, da, db;
-            if (isP) {
-                if (k < e.nterms) bar += 0.5 * (zn.re - zk.re);
-                if (kp < e.nterms) bar += 0.5 * (zk.re - zp.re);
-                pq[2 * gi] = ld_line_adj<NL, true>(zk.re, e.zy, zk.im, q, gl, e.par * bar, df, da,
-                                                   db, adj);
-                xy[2 * gi] = bar * df;
-                xy[2 * gi + 1] = bar * db;
-                yz[2 * gi] = bar * da;
-            } else {
-                if (k < e.nterms) bar += 0.5 * (zn.im - zk.im);
-                if (kp < e.nterms) bar += 0.5 * (zk.im - zp.im);
-                pq[2 * gi + 1] = ld_line_adj<NL, false>(zk.im, e.zx, zk.re, q, gl, e.par * bar,
-                                                        df, da, db, adj);
-                xq[2 * gi] = bar * db;
-                xq[2 * gi + 1] = bar * df;
-                yz[2 * gi + 1] = bar * da;
+        // centroids (integrate.py:112); the closing point repeats c_0 in the sum
+        for (int c = 0; c < nc; ++c) {
+            const ExtCEntry& e = ct[c];
+            double sx = 0.0, sy = 0.0;
+            for (int k = tid; k < e.L; k += kExtBlock) {
+                const cd a = contour_point<DEG>(zb, e.pc, e.np, k);
+                sx += a.re;
+                sy += a.im;
+            }
+            const cd c0 = (e.L > 0) ? contour_point<DEG>(zb, e.pc, e.np, 0) : cd{0.0, 0.0};
+            const double zx = (block_sum(sx, shd) + c0.re) / e.cdiv;
+            const double zy = (block_sum(sy, shd) + c0.im) / e.cdiv;
+            if (tid == 0) {
+                ct[c].zx = zx;
+                ct[c].zy = zy;
             }
         }
-    }
-    if (!VJP && parts > 1) return 0.0;
-    __syncthreads();
+        __syncthreads();
+        // the P lines of every point, then the Q lines, flat over the contours
+        for (int u = tid + part * kExtBlock; u < 2 * T; u += parts * kExtBlock) {
+            const bool isP = u < T;
+            const int gi = isP ? u : u - T;
+            int c = 0;
+            while (c + 1 < nc && gi >= ct[c + 1].off) ++c;
+            const ExtCEntry& e = ct[c];
+            const int k = gi - e.off;
+            const cd zk = contour_point<DEG>(zb, e.pc, e.np, k);
+            if constexpr (!VJP) {
+                if (isP)
+                    pq[2 * gi] = ld_line<NL, true>(zk.re, e.zy, zk.im, q, gl);
+                else
+                    pq[2 * gi + 1] = ld_line<NL, false>(zk.im, e.zx, zk.re, q, gl);
+            } else {
+                const int L = e.L;
+                const int kn = (k + 1 == L) ? 0 : k + 1;
+                const int kp = (k == 0) ? L - 1 : k - 1;
+                const cd zn = contour_point<DEG>(zb, e.pc, e.np, kn);
+                const cd zp = contour_point<DEG>(zb, e.pc, e.np, kp);
+                // cotangent of P_k or Q_k from the two trapezoid terms it enters; P_k =
+                // P(x_k; y0 .. y_k), Q_k = Q(y_k; x0 .. x_k), (x0, y0) the centroid
+                double bar = 0.0, df, da, db;
+                if (isP) {
+                    if (k < e.nterms) bar += 0.5 * (zn.re - zk.re);
+                    if (kp < e.nterms) bar += 0.5 * (zk.re - zp.re);
+                    pq[2 * gi] = ld_line_adj<NL, true>(zk.re, e.zy, zk.im, q, gl, e.par * bar, df,
+                                                       da, db, adj);
+                    xy[2 * gi] = bar * df;
+                    xy[2 * gi + 1] = bar * db;
+                    yz[2 * gi] = bar * da;
+                } else {
+                    if (k < e.nterms) bar += 0.5 * (zn.im - zk.im);
+                    if (kp < e.nterms) bar += 0.5 * (zk.im - zp.im);
+                    pq[2 * gi + 1] = ld_line_adj<NL, false>(zk.im, e.zx, zk.re, q, gl, e.par * bar,
+                                                            df, da, db, adj);
+                    xq[2 * gi] = bar * db;
+                    xq[2 * gi + 1] = bar * df;
+                    yz[2 * gi + 1] = bar * da;
+                }
+            }
+        }
+        if (!VJP && parts > 1) return 0.0;
+        __syncthreads();
     }
     double total = 0.0;
     for (int c = 0; c < nc; ++c) {
@@ -2113,7 +2107,8 @@ __global__ __launch_bounds__(kExtBlock) void k_ext_contours(ExtArgs A, int buf) 
                     // lane each
                     cd e = cd{0.0, 0.0};
                     if (lane < 8 && !aempty) {
-                        const int k = lane < 3 ? lane : lane < 6 ? at_ - (lane - 3) : 4 * M - 8 + lane;
+                        const int k =
+                            lane < 3 ? lane : lane < 6 ? at_ - (lane - 3) : 4 * M - 8 + lane;
                         if (k >= 0 && k <= at_) e = contour_point<DEG>(zb, act.pc, np, k);
                     }
                     cd hx[3], tx[3];
@@ -2447,20 +2442,21 @@ int ext_run(hipStream_t s, const ExtArgs& a) {
             hipLaunchKernelGGL((k_ext_refine<NL, kExtBlock, kExtSortMax / kExtBlock>), dim3(nb),
                                dim3(kExtBlock), 0, s, a);
     } else {
-    static_assert(kExtSelWave % 64 == 0 && kExtSortMax % kExtBlock == 0, "select register tiles");
-    for (int round = 0; round < 10; ++round) {
-        // one wave while its 8 registers of keys hold the contour (no barrier in the
-        // bisection); four waves of 16 above
-        if (a.mmax <= kExtSelWave)
-            hipLaunchKernelGGL((k_ext_select<NL, kExtWaveBlock, kExtSelWave / 64>), dim3(nb),
-                               dim3(kExtWaveBlock), 0, s, a, cur, round);
-        else
-            hipLaunchKernelGGL((k_ext_select<NL, kExtBlock, kExtSortMax / kExtBlock>), dim3(nb),
-                               dim3(kExtBlock), 0, s, a, cur, round);
-        hipLaunchKernelGGL((k_ext_solve_add<NL, MODE>), dim3(add_grid), dim3(kExtFlatBlock), 0, s,
-                           a, cur);
-        cur ^= 1;
-    }
+        static_assert(kExtSelWave % 64 == 0 && kExtSortMax % kExtBlock == 0,
+                      "select register tiles");
+        for (int round = 0; round < 10; ++round) {
+            // one wave while its 8 registers of keys hold the contour (no barrier in the
+            // bisection); four waves of 16 above
+            if (a.mmax <= kExtSelWave)
+                hipLaunchKernelGGL((k_ext_select<NL, kExtWaveBlock, kExtSelWave / 64>), dim3(nb),
+                                   dim3(kExtWaveBlock), 0, s, a, cur, round);
+            else
+                hipLaunchKernelGGL((k_ext_select<NL, kExtBlock, kExtSortMax / kExtBlock>), dim3(nb),
+                                   dim3(kExtBlock), 0, s, a, cur, round);
+            hipLaunchKernelGGL((k_ext_solve_add<NL, MODE>), dim3(add_grid), dim3(kExtFlatBlock), 0,
+                               s, a, cur);
+            cur ^= 1;
+        }
     }
     hipLaunchKernelGGL((k_ext_chain<NL, true>), dim3(nb), dim3(kExtBlock), 0, s, a, cur);  // final
     if constexpr (NL > 1)

@@ -7,8 +7,9 @@ refinement, chains the image rows along the limb, splits and stitches the image
 segments into closed contours and integrates them (uniform: Green's theorem with the
 trapezoid rule; linear limb darkening: Dominik's P/Q line integrals with Gauss-Legendre
 quadrature).  The work runs as one fixed sequence of HIP launches over the whole batch:
-flat launches for the limb solves (one limb point per lane), one wave or workgroup per
-source for continuation, gap selection, stitching and integration.  Gradients with
+flat launches for the limb solves (one limb point per lane; small batches: per group of
+lanes), a workgroup per source for continuation, gap selection, stitching and integration
+(small batches: several for the line integrals without gradients).  Gradients with
 respect to the source centre, rho, u1 and the lens parameters come from the fused
 forward+VJP pass.  ``roots_compensated=True`` runs the limb solves with the
 compensated stage (ehrlich_aberth.h:153-292).
