@@ -51,7 +51,7 @@ __host__ __device__ inline size_t ext_ws_bytes(int deg, int mmax) {
     b += ext_align(2 * (size_t)mmax * sizeof(double));            // theta x2
     b += ext_align(2 * (size_t)mmax * deg * sizeof(cd));          // z x2
     b += ext_align(2 * (size_t)mmax * sizeof(uint32_t));          // flags x2
-    b += ext_align((size_t)(mmax + 1) * sizeof(uint64_t));        // permutations / changepoints
+    b += ext_align((size_t)(mmax + 1) * sizeof(uint64_t));        // permutations
     b += ext_align(2 * ((size_t)mmax * deg + 2) * sizeof(double)); // P, Q
     b += ext_align(2 * ((size_t)mmax * deg + 2) * sizeof(double)); // point cotangents
     b += ext_align(2 * ((size_t)mmax * deg + 2) * sizeof(double)); // centroid cotangent parts
@@ -636,7 +636,7 @@ struct LDAdj {
 // only these sums; the profile's constants and the line's scale are applied once a part.
 // Bound: FP64 issue.  Per node of two lenses 87 FP64 operations and 3 quarter-rate seeds;
 // with every derivative formed node by node it was 124 and 3.  Integration of 4,096 binary
-// sources of 256-4096 limb points (3.2e9 nodes): 17.0 -> 11.8 ms, of 12,000 triple-lens
+// sources of 256-4096 limb points (3.2e9 nodes): 17.0 -> 11.8-12.2 ms, of 12,000 triple-lens
 // sources (2.0e9 nodes): 17.8 -> 10.8 ms (of which 0.5 ms the Gauss-Legendre nodes).
 template <int NL, bool ISP>
 __device__ __forceinline__ double ld_line_adj(double fixed, double a, double b,
