@@ -392,7 +392,7 @@ def critical_and_caustic_curves(npts=200, nlenses=2, **params):
     reference API (point_source.py:1582-1649): roots of the critical-curve polynomial
     on a grid of phi (GPU solver), continued along phi with match_points, mapped through
     the lens equation and shifted by x_cm (HIP kernels).  Parameters may also be
-    arrays of length B, giving (B, n_curves, npts)."""
+    arrays of length B (s, and any of the others), giving (B, n_curves, npts)."""
     phi = torch.linspace(-np.pi, np.pi, npts, dtype=torch.float64, device="cuda")
     if nlenses == 1:
         return torch.exp(-1j * phi), torch.zeros(npts, dtype=torch.complex128, device="cuda")
@@ -407,6 +407,8 @@ def critical_and_caustic_curves(npts=200, nlenses=2, **params):
             _lib.resolved(torch.as_tensor(v, device="cuda").to(torch.float64)).reshape(-1)
             for v in vals]
     B = torch.broadcast_shapes(*[(1,) if c is None else c.shape for c in cols])[0]
+    if B != (1 if cols[0] is None else cols[0].numel()):
+        raise RuntimeError(f"{names[0]} has to have the length of the batch, {B}")
     P = len(cols)
     n = _DEGREE_CRITICAL[nlenses]
     crit = torch.empty((B, n, npts), dtype=torch.complex128, device="cuda")

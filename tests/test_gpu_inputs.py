@@ -173,3 +173,15 @@ def test_likelihood_of_no_epochs_is_refused(gpu):
     e = torch.empty(0, dtype=torch.float64)
     with pytest.raises(RuntimeError, match="invalid argument"):
         marginalized_log_likelihood([e], [e], [e])
+
+
+# ---- critical curves: the batch is that of s ----------------------------------------------
+@pytest.mark.parametrize("s", [0.9, [0.9]])
+@pytest.mark.parametrize("name", ["q", "psi"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_curves_of_one_s_and_several_lenses_are_refused(gpu, s, name, grad):
+    p = {**(dict(q=0.4) if name == "q" else B3), "s": s, name: np.linspace(0.2, 0.6, 5)}
+    if grad:   # the tensor form
+        p[name] = torch.as_tensor(p[name], device="cuda").requires_grad_()
+    with pytest.raises(RuntimeError):
+        ca.critical_and_caustic_curves(npts=20, nlenses=2 if name == "q" else 3, **p)
