@@ -95,11 +95,16 @@ def kept_jacobian(planes, N, device, limit):
     if need > limit:
         return None
     credit = _jacobian_credit.get(device.index, 0)
-    if need > credit:
+    # Where hooks take what is saved, the sizes decide alone: activation checkpointing runs the
+    # forward pass again, when other memory is free, and requires that the same is saved (and
+    # holds one segment's Jacobians at a time); save_on_cpu takes them off the card.
+    hooked = torch._C._autograd._top_saved_tensors_default_hooks(True) is not None
+    if need > credit and not hooked:
         credit = need + JACOBIAN_ASK_BYTES
         if not _half_free(credit, device):
             return None
-    _jacobian_credit[device.index] = credit - need
+    if not hooked:
+        _jacobian_credit[device.index] = credit - need
     try:
         return torch.empty((planes, N), dtype=torch.float64, device=device)
     except torch.OutOfMemoryError:

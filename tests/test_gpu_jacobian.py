@@ -25,14 +25,12 @@ def _run(nlenses, lightcurve, wrt):
     x = {k: torch.as_tensor(v, device="cuda") for k, v in _inputs(nlenses, lightcurve).items()}
     for k in wrt:
         x[k].requires_grad_()
-    held = []
-    with torch.autograd.graph.saved_tensors_hooks(lambda t: held.append(tuple(t.shape)) or t,
-                                                  lambda t: t):
-        if lightcurve:
-            m = ca.mag_point_source_lightcurve(np.linspace(-1, 1, N), nlenses=nlenses, **x)
-        else:
-            m = ca.mag_point_source(x.pop("w") if "w" not in wrt else x["w"], nlenses=nlenses,
-                                    **{k: v for k, v in x.items() if k != "w"})
+    if lightcurve:
+        m = ca.mag_point_source_lightcurve(np.linspace(-1, 1, N), nlenses=nlenses, **x)
+    else:
+        m = ca.mag_point_source(x["w"], nlenses=nlenses,
+                                **{k: v for k, v in x.items() if k != "w"})
+    held = [None if t is None else tuple(t.shape) for t in m.grad_fn.saved_tensors]
     g = torch.autograd.grad(m, [x[k] for k in wrt], torch.linspace(0.5, 2, N, device="cuda",
                                                                    dtype=torch.float64).reshape(
                                                                        m.shape))
@@ -95,3 +93,31 @@ def test_free_memory_is_asked_once_a_gibibyte(gpu, monkeypatch):
     for k in range(10):
         assert point_source.kept_jacobian(1, quarter, dev, 1 << 40) is not None
         assert len(asked) == 1 + k // 5   # each question covers its own call and four more
+
+
+@pytest.mark.parametrize("lightcurve", [False, True])
+def test_checkpoint_saves_the_same_in_both_forward_passes(gpu, lightcurve, monkeypatch):
+    """Activation checkpointing runs the forward pass a second time, with other memory free, and
+    compares what the two saved."""
+    from torch.utils.checkpoint import checkpoint
+
+    total = torch.cuda.mem_get_info()[1]
+    asked = []
+
+    def scarce(*a):   # free in the first forward pass, not in the second
+        asked.append(1)
+        return (total if len(asked) == 1 else 0, total)
+
+    monkeypatch.setattr(point_source, "_jacobian_credit", {})
+    monkeypatch.setattr(point_source, "JACOBIAN_ASK_BYTES", 0)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", scarce)
+    w = torch.as_tensor(_inputs(2, False)["w"], device="cuda")
+
+    def f(s):
+        if lightcurve:
+            return ca.mag_point_source_lightcurve(np.linspace(-1, 1, N), s=s, q=0.4, **TRAJ).sum()
+        return ca.mag_point_source(w, s=s, q=0.4).sum()
+
+    s = torch.tensor(0.9, dtype=torch.float64, device="cuda", requires_grad=True)
+    g, = torch.autograd.grad(checkpoint(f, s, use_reentrant=False), s)
+    torch.testing.assert_close(g, torch.autograd.grad(f(s), s)[0], rtol=1e-10, atol=0.0)
