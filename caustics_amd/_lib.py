@@ -161,9 +161,9 @@ def resolved(x):
 def on_device(x, dtype):
     """Tensor x in dtype on the current device, resolved (x.to(device="cuda", dtype=dtype),
     without its 1 us where x is that already)."""
-    if x.dtype is dtype and x.is_cuda and x.get_device() == torch.cuda.current_device():
-        return resolved(x)
-    return resolved(x.to(device="cuda", dtype=dtype))
+    if not (x.dtype is dtype and x.is_cuda and x.get_device() == torch.cuda.current_device()):
+        x = x.to(device="cuda", dtype=dtype)
+    return resolved(x) if x.is_neg() or x.is_conj() else x
 
 
 def ptr(t):

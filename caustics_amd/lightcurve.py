@@ -69,7 +69,7 @@ class _LightCurve(torch.autograd.Function):
         jac, planes = None, 0
         if need:
             grads = ctx.needs_input_grad[5:]
-            planes = sum(1 << k for k, g in enumerate(grads) if g)
+            planes = sum([1 << k for k, g in enumerate(grads) if g])
             jac = kept_jacobian(sum(grads), L * T, t.device, JACOBIAN_MAX_BYTES)
         rc = _lib.lib().caus_lightcurve_point_source_jac_planes(
             _lib.stream_ptr(), nlenses, _lib.ptr(t), T, *_lib.columns(flat), L, _lib.ptr(mag),
@@ -86,7 +86,9 @@ class _LightCurve(torch.autograd.Function):
     def backward(ctx, g):
         jac, *again = ctx.saved_tensors
         nlenses, itmax, mode, L, T, shapes, planes = ctx.meta
-        g = _lib.resolved(g.contiguous().to(torch.float64))
+        g = g.contiguous().to(torch.float64)
+        if g.is_neg():
+            g = g.resolve_neg()
         if jac is not None:
             _, gp = jacobian_vjp(jac, 0, max(T, 1), g, False, True)
         else:

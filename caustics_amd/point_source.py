@@ -75,6 +75,7 @@ JACOBIAN_ASK_BYTES = 1 << 30
 # device index -> bytes that may be handed out before the next question (threads that race for it
 # hand out at most that much each)
 _jacobian_credit = {}
+_saved_tensor_hooks = torch._C._autograd._top_saved_tensors_default_hooks
 
 
 def _half_free(need, device):
@@ -94,17 +95,16 @@ def kept_jacobian(planes, N, device, limit):
     need = 8 * planes * N
     if need > limit:
         return None
-    credit = _jacobian_credit.get(device.index, 0)
+    dev = device.index
+    credit = _jacobian_credit.get(dev, 0)
     # Where hooks take what is saved, the sizes decide alone: activation checkpointing runs the
     # forward pass again, when other memory is free, and requires that the same is saved (and
     # holds one segment's Jacobians at a time); save_on_cpu takes them off the card.
-    hooked = torch._C._autograd._top_saved_tensors_default_hooks(True) is not None
-    if need > credit and not hooked:
+    if need > credit and _saved_tensor_hooks(True) is None:
         credit = need + JACOBIAN_ASK_BYTES
         if not _half_free(credit, device):
             return None
-    if not hooked:
-        _jacobian_credit[device.index] = credit - need
+    _jacobian_credit[dev] = max(credit - need, 0)
     try:
         return torch.empty((planes, N), dtype=torch.float64, device=device)
     except torch.OutOfMemoryError:
@@ -166,7 +166,7 @@ class _MagPointSource(torch.autograd.Function):
         if need:
             grad_w, *grad_p = ctx.needs_input_grad[4:]
             nw = 2 if grad_w else 0
-            planes = (3 if grad_w else 0) | sum(4 << k for k, g in enumerate(grad_p) if g)
+            planes = (3 if grad_w else 0) | sum([4 << k for k, g in enumerate(grad_p) if g])
             jac = kept_jacobian(nw + sum(grad_p), N, w.device, JACOBIAN_MAX_BYTES)
         rc = _lib.lib().caus_mag_point_source_jac_planes(
             _lib.stream_ptr(), nlenses, _lib.ptr(wf), N, *_lib.columns(cols), per,
