@@ -64,13 +64,15 @@ class _LightCurve(torch.autograd.Function):
     def forward(ctx, nlenses, itmax, mode, need, t, *cols):
         L = max([c.numel() for c in cols])
         T = t.numel()
-        flat = [c.reshape(-1) if c.numel() == L else c.reshape(-1).expand(L) for c in cols]
+        flat = [c if c.shape == (L,) else
+                c.reshape(-1) if c.numel() == L else c.reshape(-1).expand(L) for c in cols]
         mag = torch.empty((L, T), dtype=torch.float64, device=t.device)
         jac, planes = None, 0
+        wrt = []
         if need:
-            grads = ctx.needs_input_grad[5:]
-            planes = sum([1 << k for k, g in enumerate(grads) if g])
-            jac = kept_jacobian(sum(grads), L * T, t.device, JACOBIAN_MAX_BYTES)
+            wrt = [k for k, g in enumerate(ctx.needs_input_grad[5:]) if g]
+            planes = sum([1 << k for k in wrt])
+            jac = kept_jacobian(len(wrt), L * T, t.device, JACOBIAN_MAX_BYTES)
         rc = _lib.lib().caus_lightcurve_point_source_jac_planes(
             _lib.stream_ptr(), nlenses, _lib.ptr(t), T, *_lib.columns(flat), L, _lib.ptr(mag),
             _lib.ptr(jac), planes, itmax, mode)
@@ -79,13 +81,13 @@ class _LightCurve(torch.autograd.Function):
             ctx.save_for_backward(jac)
         elif need:
             ctx.save_for_backward(None, t, torch.stack(flat, -1).contiguous())
-        ctx.meta = (nlenses, itmax, mode, L, T, [c.shape for c in cols], planes)
+        ctx.meta = (nlenses, itmax, mode, L, T, [c.shape for c in cols], wrt)
         return mag
 
     @staticmethod
     def backward(ctx, g):
         jac, *again = ctx.saved_tensors
-        nlenses, itmax, mode, L, T, shapes, planes = ctx.meta
+        nlenses, itmax, mode, L, T, shapes, wrt = ctx.meta
         g = g.contiguous().to(torch.float64)
         if g.is_neg():
             g = g.resolve_neg()
@@ -93,17 +95,15 @@ class _LightCurve(torch.autograd.Function):
             _, gp = jacobian_vjp(jac, 0, max(T, 1), g, False, True)
         else:
             _, gp, _ = _call(*again, g, nlenses, itmax, mode)
-            gp, planes = gp.t(), ~0
+            gp, wrt = gp.t(), range(len(shapes))
         if T == 0:
-            gp, planes = torch.zeros((len(shapes), L), dtype=torch.float64, device=g.device), ~0
-        gps = []
-        gp = iter(gp.unbind(0))
-        for k, shape in enumerate(shapes):
-            row = next(gp) if (planes >> k) & 1 else None
-            if not ctx.needs_input_grad[5 + k]:
-                gps.append(None)
-            else:
-                gps.append((row if shape.numel() == L else row.sum()).reshape(shape))
+            gp = torch.zeros((len(wrt), L), dtype=torch.float64, device=g.device)
+        gps = [None] * len(shapes)
+        for k, row in zip(wrt, gp.unbind(0)):
+            shape = shapes[k]
+            if ctx.needs_input_grad[5 + k]:
+                gps[k] = (row if row.shape == shape else
+                          (row if shape.numel() == L else row.sum()).reshape(shape))
         return (None, None, None, None, None, *gps)
 
 
@@ -117,8 +117,8 @@ def mag_point_source_lightcurve(t, t0, u0, tE, alpha, nlenses=2, roots_itmax=250
     cols = [_lib.on_device(vals[n], torch.float64) if isinstance(vals[n], torch.Tensor)
             else torch.as_tensor(np.asarray(vals[n]), device="cuda").to(torch.float64)
             for n in names]
-    t = _lib.resolved(torch.as_tensor(t, device="cuda", dtype=torch.float64))
-    t = t.contiguous().reshape(-1)
+    t = torch.as_tensor(t, device="cuda", dtype=torch.float64)
+    t = (_lib.resolved(t) if t.is_neg() else t).contiguous().reshape(-1)
     need = torch.is_grad_enabled() and any(c.requires_grad for c in cols)
     return _LightCurve.apply(nlenses, int(roots_itmax), _mode_id(roots_compensated, mode), need,
                              t, *cols)

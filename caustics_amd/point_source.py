@@ -162,12 +162,12 @@ class _MagPointSource(torch.autograd.Function):
         else:
             cols = [p.expand(shape).reshape(-1) for p in ps]
         mag = torch.empty(N, dtype=torch.float64, device=w.device)
-        jac, nw, planes = None, 0, 0
+        jac, nw, planes, wrt = None, 0, 0, []
         if need:
-            grad_w, *grad_p = ctx.needs_input_grad[4:]
-            nw = 2 if grad_w else 0
-            planes = (3 if grad_w else 0) | sum([4 << k for k, g in enumerate(grad_p) if g])
-            jac = kept_jacobian(nw + sum(grad_p), N, w.device, JACOBIAN_MAX_BYTES)
+            nw = 2 if ctx.needs_input_grad[4] else 0
+            wrt = [k for k, g in enumerate(ctx.needs_input_grad[5:]) if g]
+            planes = (3 if nw else 0) + sum([4 << k for k in wrt])
+            jac = kept_jacobian(nw + len(wrt), N, w.device, JACOBIAN_MAX_BYTES)
         rc = _lib.lib().caus_mag_point_source_jac_planes(
             _lib.stream_ptr(), nlenses, _lib.ptr(wf), N, *_lib.columns(cols), per,
             _lib.ptr(mag), _lib.ptr(jac), planes, itmax, mode)
@@ -177,12 +177,12 @@ class _MagPointSource(torch.autograd.Function):
         elif need:
             prm = torch.stack([c.expand(N // per) for c in cols], -1).contiguous() if P else None
             ctx.save_for_backward(None, wf, prm)
-        ctx.meta = (nlenses, itmax, mode, shape, per, w.shape, [p.shape for p in ps], nw, planes)
+        ctx.meta = (nlenses, itmax, mode, shape, per, w.shape, [p.shape for p in ps], nw, wrt)
         return mag.reshape(shape)
 
     @staticmethod
     def backward(ctx, g):
-        nlenses, itmax, mode, shape, per, wshape, pshapes, nw, planes = ctx.meta
+        nlenses, itmax, mode, shape, per, wshape, pshapes, nw, wrt = ctx.meta
         jac, *again = ctx.saved_tensors
         P = len(pshapes)
         want_w, want_p = ctx.needs_input_grad[4], any(ctx.needs_input_grad[5:])
@@ -193,7 +193,7 @@ class _MagPointSource(torch.autograd.Function):
         else:
             wf, prm = again
             N = wf.numel()
-            planes = ~0
+            wrt = range(P)
             pstride = P if P and prm.shape[0] > 1 else 0
             if pstride and per > 1:
                 prm = prm.repeat_interleave(per, 0)
@@ -207,16 +207,11 @@ class _MagPointSource(torch.autograd.Function):
             g_p = g_p.t()
             pshape = shape
         gw = g_w.reshape(shape).sum_to_size(wshape) if want_w else None
-        gps = []
-        g_p = iter(g_p.unbind(0)) if g_p is not None else None
-        for k, ps_shape in enumerate(pshapes):
-            row = next(g_p) if g_p is not None and (planes >> (2 + k)) & 1 else None
-            if not ctx.needs_input_grad[5 + k]:
-                gps.append(None)
-            elif pshape is None:
-                gps.append(row.reshape(ps_shape))
-            else:
-                gps.append(row.reshape(shape).sum_to_size(ps_shape))
+        gps = [None] * P
+        for k, row in zip(wrt, g_p.unbind(0) if g_p is not None else ()):
+            if ctx.needs_input_grad[5 + k]:
+                gps[k] = (row.reshape(pshapes[k]) if pshape is None else
+                          row.reshape(shape).sum_to_size(pshapes[k]))
         return (None, None, None, None, gw, *gps)
 
 
